@@ -2,12 +2,13 @@
 //
 // CDNA4 executes 64-lane wavefronts. Kernels here map a vertex to a "group" of
 // G lanes (G in {4, 8, 16, 32, 64}) or to a whole workgroup; group reductions use
-// width-limited shuffles, which lower to DPP / ds_swizzle row operations.
+// DPP moves where the pattern has one, else width-limited shuffles.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace gpart_hip {
 
@@ -31,6 +32,63 @@ __device__ __forceinline__ std::uint64_t lanemask_lt() {
     return lane == 0 ? 0ULL : (~0ULL >> (64 - lane));
 }
 
+// Lane exchanges. __shfl_* go through the LDS crossbar (ds_bpermute, two per 64-bit
+// value and step); DPP operands move data between neighbouring lanes inside a
+// vector instruction. Patterns with a DPP form use it: xor 1 and 2 (quad_perm),
+// xor 8 (rotation by half a row of 16) and the prefix steps of wave_scan below.
+// Every lane that a pattern reads must be active, as with __shfl_*.
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppRowRor8 = 0x128;
+constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
+constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;
+
+// Lanes without a source (and rows outside RowMask) receive 0.
+template <int Control, int RowMask = 0xf>
+__device__ __forceinline__ unsigned dpp_or_zero(unsigned v) {
+    return static_cast<unsigned>(
+        __builtin_amdgcn_update_dpp(0, static_cast<int>(v), Control, RowMask, 0xf, false));
+}
+template <int Control, int RowMask = 0xf>
+__device__ __forceinline__ unsigned long long dpp_or_zero(unsigned long long v) {
+    const unsigned lo = dpp_or_zero<Control, RowMask>(static_cast<unsigned>(v));
+    const unsigned hi = dpp_or_zero<Control, RowMask>(static_cast<unsigned>(v >> 32));
+    return (static_cast<unsigned long long>(hi) << 32) | lo;
+}
+
+// Inclusive prefix sums over the wave: four steps inside each row of 16 lanes, then
+// the last lane of rows 0 and 2 into rows 1 and 3, then lane 31 into rows 2 and 3.
+// Every lane of the wave must be active.
+template <typename T>
+__device__ __forceinline__ T wave_scan(T v) {
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "4- or 8-byte integers");
+    using U = std::conditional_t<sizeof(T) == 4, unsigned, unsigned long long>;
+    U x = static_cast<U>(v);
+    x += dpp_or_zero<kDppRowShr1>(x);
+    x += dpp_or_zero<kDppRowShr2>(x);
+    x += dpp_or_zero<kDppRowShr4>(x);
+    x += dpp_or_zero<kDppRowShr8>(x);
+    x += dpp_or_zero<kDppBcast15, 0xa>(x);
+    x += dpp_or_zero<kDppBcast31, 0xc>(x);
+    return static_cast<T>(x);
+}
+
+// Lane `src`'s value, the same src on every lane.
+__device__ __forceinline__ unsigned read_lane(unsigned v, int src) {
+    return static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(v), src));
+}
+__device__ __forceinline__ unsigned long long read_lane(unsigned long long v, int src) {
+    const unsigned lo = read_lane(static_cast<unsigned>(v), src);
+    const unsigned hi = read_lane(static_cast<unsigned>(v >> 32), src);
+    return (static_cast<unsigned long long>(hi) << 32) | lo;
+}
+
+// __shfl_xor(v, mask, width) for mask < width; mask is a constant after inlining.
+__device__ __forceinline__ unsigned lane_xor(unsigned v, int mask, int width) {
+    if (mask == 1) return dpp_or_zero<kDppXor1>(v);
+    if (mask == 2) return dpp_or_zero<kDppXor2>(v);
+    if (mask == 8) return dpp_or_zero<kDppRowRor8>(v);
+    return __shfl_xor(v, mask, width);
+}
+
 template <typename T>
 __device__ __forceinline__ T shfl(T v, int src, int width) {
     return __shfl(v, src, width);
@@ -43,8 +101,8 @@ __device__ __forceinline__ unsigned long long shfl_u64(unsigned long long v, int
 }
 
 __device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v, int mask, int width) {
-    const unsigned lo = __shfl_xor(static_cast<unsigned>(v), mask, width);
-    const unsigned hi = __shfl_xor(static_cast<unsigned>(v >> 32), mask, width);
+    const unsigned lo = lane_xor(static_cast<unsigned>(v), mask, width);
+    const unsigned hi = lane_xor(static_cast<unsigned>(v >> 32), mask, width);
     return (static_cast<unsigned long long>(hi) << 32) | lo;
 }
 
@@ -66,6 +124,7 @@ __device__ __forceinline__ long long shfl_xor_i64(long long v, int mask, int wid
 
 template <int G>
 __device__ __forceinline__ unsigned long long group_sum_u64(unsigned long long v) {
+    if constexpr (G == kWave) return read_lane(wave_scan(v), kWave - 1);
 #pragma unroll
     for (int m = G / 2; m > 0; m /= 2) v += shfl_xor_u64(v, m, G);
     return v;
@@ -73,9 +132,7 @@ __device__ __forceinline__ unsigned long long group_sum_u64(unsigned long long v
 
 template <int G>
 __device__ __forceinline__ long long group_sum_i64(long long v) {
-#pragma unroll
-    for (int m = G / 2; m > 0; m /= 2) v += shfl_xor_i64(v, m, G);
-    return v;
+    return static_cast<long long>(group_sum_u64<G>(static_cast<unsigned long long>(v)));
 }
 
 template <int G>

@@ -155,17 +155,12 @@ __device__ unsigned long long block_key_prefix(bool pending, int key, unsigned l
     unsigned long long open = __ballot(pending);
     while (open) {
         const int leader = __ffsll(static_cast<unsigned long long>(open)) - 1;
-        const int current = __shfl(key, leader, kWave);
+        const int current = static_cast<int>(read_lane(static_cast<unsigned>(key), leader));
         const bool member = pending && key == current;
         const unsigned long long members = __ballot(member);
-        unsigned long long x = member ? w : 0;
-#pragma unroll
-        for (int d = 1; d < kWave; d <<= 1) {
-            const auto other = shfl_up_u64(x, d, kWave);
-            if (lane >= d) x += other;
-        }
+        const unsigned long long x = wave_scan(member ? w : 0ULL);
         if (member) mine = x - w;
-        const auto total = shfl_u64(x, kWave - 1, kWave);
+        const auto total = read_lane(x, kWave - 1);
         if (lane == 0) wave_total[wave][current] = total;
         open &= ~members;
     }

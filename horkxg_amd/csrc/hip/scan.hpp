@@ -55,28 +55,27 @@ __device__ T block_exclusive_scan(T value, Op op, T* total, T* shared_waves) {
     const int wave = threadIdx.x / kWave;
     const int waves = blockDim.x / kWave;
     T inclusive = value;
+    if constexpr (std::is_integral_v<T> && std::is_same_v<Op, SumOp<T>>) {
+        inclusive = wave_scan(value);
+    } else {
 #pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const T other = shfl_up_any(inclusive, d);
-        if (lane >= d) inclusive = op(other, inclusive);
+        for (int d = 1; d < kWave; d <<= 1) {
+            const T other = shfl_up_any(inclusive, d);
+            if (lane >= d) inclusive = op(other, inclusive);
+        }
     }
     if (lane == kWave - 1) shared_waves[wave] = inclusive;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        T running = op.identity();
-        for (int w = 0; w < waves; ++w) {
-            const T t = shared_waves[w];
-            shared_waves[w] = running;
-            running = op(running, t);
-        }
-        shared_waves[waves] = running;
+    // every thread combines the wave totals itself: one barrier and no serial thread
+    T wave_prefix = op.identity(), all = op.identity();
+    for (int w = 0; w < waves; ++w) {
+        if (w == wave) wave_prefix = all;
+        all = op(all, shared_waves[w]);
     }
-    __syncthreads();
-    const T wave_prefix = shared_waves[wave];
+    *total = all;
     T exclusive = shfl_up_any(inclusive, 1);
     if (lane == 0) exclusive = op.identity();
     exclusive = op(wave_prefix, exclusive);
-    *total = shared_waves[waves];
     __syncthreads();
     return exclusive;
 }
