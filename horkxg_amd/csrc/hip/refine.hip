@@ -46,7 +46,7 @@ struct RoundState {
     unsigned long long max_weight;
     long long edges;       // CSR entries of all movers (light + heavy)
     unsigned long long cut_directed;  // rebuild rounds: directed cut weight after the round
-    unsigned long long pad[1];
+    unsigned long long arrivals;  // workgroups of the round's last launch that have finished
     unsigned long long pw[32];
 };
 
@@ -274,7 +274,7 @@ __global__ void __launch_bounds__(kBlock) lp_proposals_kernel(std::int64_t n, co
 #pragma unroll
     for (int m = G / 2; m > 0; m /= 2) {
         const auto ob = shfl_xor_u64(best, m, G);
-        const int op = __shfl_xor(best_p, m, G);
+        const int op = static_cast<int>(lane_xor(static_cast<unsigned>(best_p), m, G));
         const auto oc = shfl_xor_u64(current, m, G);
         if (ob > best || (ob == best && op < best_p)) {
             best = ob;
@@ -301,22 +301,64 @@ __global__ void __launch_bounds__(kBlock) lp_proposals_kernel(std::int64_t n, co
     gains[v] = gain;
 }
 
+// Appends the taking threads' vertices to the light/heavy mover lists (one
+// global atomic per list per workgroup pass). Called by every thread of the
+// workgroup.
+template <typename O>
+__device__ void append_movers(bool take, std::int32_t v, const O* offsets, std::int32_t* light,
+                              std::int32_t* heavy, RoundState* st, unsigned* counts, unsigned long long* base) {
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    const long long degree = take ? static_cast<long long>(offsets[v + 1] - offsets[v]) : 0;
+    const bool is_heavy = degree > kHeavyDegree;
+    const long long edges = group_sum_i64<kWave>(degree);
+    if (lane == 0 && edges) atomicAdd(reinterpret_cast<unsigned long long*>(&st->edges),
+                                      static_cast<unsigned long long>(edges));
+    const bool is_light = take && !is_heavy;
+    const unsigned long long bl = __ballot(is_light), bh = __ballot(is_heavy);
+    if (lane == 0) {
+        counts[wave] = static_cast<unsigned>(__popcll(bl));
+        counts[kBlock / kWave + wave] = static_cast<unsigned>(__popcll(bh));
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned tl = 0, th = 0;
+        for (int q = 0; q < kBlock / kWave; ++q) {
+            tl += counts[q];
+            th += counts[kBlock / kWave + q];
+        }
+        base[0] = tl ? atomicAdd(reinterpret_cast<unsigned long long*>(&st->light), tl) : 0;
+        base[1] = th ? atomicAdd(reinterpret_cast<unsigned long long*>(&st->heavy), th) : 0;
+    }
+    __syncthreads();
+    if (take) {
+        unsigned before = 0;
+        const unsigned* row = is_heavy ? counts + kBlock / kWave : counts;
+        for (int q = 0; q < wave; ++q) before += row[q];
+        const unsigned long long mask = is_heavy ? bh : bl;
+        before += static_cast<unsigned>(__popcll(mask & lanemask_lt()));
+        (is_heavy ? heavy : light)[(is_heavy ? base[1] : base[0]) + before] = v;
+    }
+    __syncthreads();
+}
+
 // incremental_priority_filter (:48-67) over one class list with G lanes per row,
 // by the workgroups numbered `block` of the list's range. Called by every thread
-// of the workgroup.
+// of the workgroup; true on the one lane of a row whose vertex (*vertex) moves.
 template <typename O, typename W, int G>
-__device__ __forceinline__ void priority_filter_rows(std::int64_t count, const std::int32_t* list, long long block,
+__device__ __forceinline__ bool priority_filter_rows(std::int64_t count, const std::int32_t* list, long long block,
                                                      const O* offsets, const std::int32_t* neighbors,
                                                      const W* weights, const std::int32_t* labels,
                                                      const std::int32_t* targets, const long long* gains,
-                                                     std::int32_t* flags, long long* block_sum) {
+                                                     std::int32_t* flags, long long* block_sum,
+                                                     std::int32_t* vertex) {
     const std::int64_t group = (block * blockDim.x + threadIdx.x) / G;
     const int sub = threadIdx.x & (G - 1);
     const bool active = group < count;
     const std::int32_t v = active ? (list ? list[group] : static_cast<std::int32_t>(group)) : 0;
     const std::int32_t target = active ? targets[v] : -1;
     // rows above kHubChunk entries are hubs, done in chunks by priority_filter_hub_kernel
-    if (G == kBlock && active && offsets[v + 1] - offsets[v] > kHubChunk) return;  // uniform per block
+    bool take = false;
+    if (G == kBlock && active && offsets[v + 1] - offsets[v] > kHubChunk) return false;  // uniform per block
     long long correction = 0;
     if (active && target >= 0)
         correction = filter_correction(v, target, labels[v], gains[v], static_cast<std::int64_t>(offsets[v]) + sub,
@@ -324,7 +366,10 @@ __device__ __forceinline__ void priority_filter_rows(std::int64_t count, const s
                                        targets, gains);
     if constexpr (G <= kWave) {
         correction = group_sum_i64<G>(correction);
-        if (active && sub == 0) flags[v] = target >= 0 && gains[v] + correction >= 0;
+        if (active && sub == 0) {
+            take = target >= 0 && gains[v] + correction >= 0;
+            flags[v] = take ? labels[v] + 1 : 0;
+        }
     } else {
         correction = group_sum_i64<kWave>(correction);
         if (lane_id() == 0) block_sum[threadIdx.x / kWave] = correction;
@@ -332,31 +377,44 @@ __device__ __forceinline__ void priority_filter_rows(std::int64_t count, const s
         if (threadIdx.x == 0 && active) {
             long long total = 0;
             for (int w = 0; w < kBlock / kWave; ++w) total += block_sum[w];
-            flags[v] = target >= 0 && gains[v] + total >= 0;
+            take = target >= 0 && gains[v] + total >= 0;
+            flags[v] = take ? labels[v] + 1 : 0;
         }
     }
+    *vertex = v;
+    return take;
 }
 
 // The three degree classes in one launch: workgroups [0, low_blocks) take the low
 // rows (8 lanes each), the next medium_blocks the medium rows (a wave each), the
-// rest the high rows (a workgroup each).
-template <typename O, typename W>
+// rest the high rows (a workgroup each). Append: the workgroups also append their
+// movers to the round's lists (three counter atomics per workgroup that has any,
+// so only for small levels; the lists' order does not matter).
+template <typename O, typename W, bool Append>
 __global__ void __launch_bounds__(kBlock) priority_filter_kernel(
     std::int64_t low_count, const std::int32_t* low, unsigned low_blocks, std::int64_t medium_count,
     const std::int32_t* medium, unsigned medium_blocks, std::int64_t high_count, const std::int32_t* high,
     const O* offsets, const std::int32_t* neighbors, const W* weights, const std::int32_t* labels,
-    const std::int32_t* targets, const long long* gains, std::int32_t* flags) {
+    const std::int32_t* targets, const long long* gains, std::int32_t* flags, std::int32_t* light,
+    std::int32_t* heavy, RoundState* st) {
     __shared__ long long block_sum[kBlock / kWave];
     const long long b = blockIdx.x;
+    bool take;
+    std::int32_t v = 0;
     if (b < low_blocks)
-        priority_filter_rows<O, W, 8>(low_count, low, b, offsets, neighbors, weights, labels, targets, gains, flags,
-                                      block_sum);
+        take = priority_filter_rows<O, W, 8>(low_count, low, b, offsets, neighbors, weights, labels, targets, gains,
+                                             flags, block_sum, &v);
     else if (b < low_blocks + medium_blocks)
-        priority_filter_rows<O, W, 64>(medium_count, medium, b - low_blocks, offsets, neighbors, weights, labels,
-                                       targets, gains, flags, block_sum);
+        take = priority_filter_rows<O, W, 64>(medium_count, medium, b - low_blocks, offsets, neighbors, weights,
+                                              labels, targets, gains, flags, block_sum, &v);
     else
-        priority_filter_rows<O, W, kBlock>(high_count, high, b - low_blocks - medium_blocks, offsets, neighbors,
-                                           weights, labels, targets, gains, flags, block_sum);
+        take = priority_filter_rows<O, W, kBlock>(high_count, high, b - low_blocks - medium_blocks, offsets,
+                                                  neighbors, weights, labels, targets, gains, flags, block_sum, &v);
+    if constexpr (Append) {
+        __shared__ unsigned counts[2 * (kBlock / kWave)];
+        __shared__ unsigned long long base[2];
+        if (__syncthreads_or(take)) append_movers(take, v, offsets, light, heavy, st, counts, base);
+    }
 }
 
 // Hub rows (degree > kHubChunk): each chunk adds its share of the correction to
@@ -394,31 +452,104 @@ __global__ void __launch_bounds__(kBlock) priority_filter_hub_kernel(const std::
 }
 
 __global__ void priority_filter_hub_finish_kernel(std::int64_t count, const std::int64_t* chunk_start,
-                                                  const std::int32_t* list, const std::int32_t* targets,
-                                                  const long long* gains, long long* sums, std::int32_t* flags) {
+                                                  const std::int32_t* list, const std::int32_t* labels,
+                                                  const std::int32_t* targets, const long long* gains,
+                                                  long long* sums, std::int32_t* flags) {
     const std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= count || chunk_start[i] == chunk_start[i + 1]) return;
     const std::int32_t v = list[i];
-    flags[v] = targets[v] >= 0 && gains[v] + sums[i] >= 0;
+    flags[v] = targets[v] >= 0 && gains[v] + sums[i] >= 0 ? labels[v] + 1 : 0;
     sums[i] = 0;
 }
 
-// incremental_update_cache_and_cut (:69-95) over a mover list whose length is on
-// the device, G lanes per mover, by the workgroups [0, blocks) numbered `block`;
-// the block's gain sum goes to *delta. Called by every thread of the workgroup.
+// The round's status into the host-visible words (word 0: seq, stored last, after
+// a system-scope fence). Called by one wave; weight(p) and delta are the part
+// weights and the cut decrease as the round left them. Lane p < k holds part p's
+// weight; every lane writes one status word.
+template <typename Weight>
+__device__ void publish_status(const RoundState* st, Weight weight, long long delta, int k,
+                               unsigned long long* status, unsigned long long* counter) {
+    constexpr int kHead = static_cast<int>(offsetof(RoundState, pw) / 8);  // words before pw
+    constexpr int kDelta = static_cast<int>(offsetof(RoundState, delta) / 8);
+    constexpr int kMax = static_cast<int>(offsetof(RoundState, max_weight) / 8);
+    const int lane = lane_id();
+    const unsigned long long w = lane < k ? weight(lane) : 0;
+    unsigned long long maximum = w;
+    for (int m = kWave / 2; m > 0; m /= 2) {
+        const unsigned long long o = shfl_xor_u64(maximum, m, kWave);
+        maximum = o > maximum ? o : maximum;
+    }
+    if (lane < kHead) {
+        const auto* words = reinterpret_cast<const unsigned long long*>(st);
+        status[1 + lane] = lane == kMax ? maximum : lane == kDelta ? static_cast<unsigned long long>(delta) : words[lane];
+    }
+    if (lane < k) status[1 + kHead + lane] = w;
+    __threadfence_system();
+    if (lane == 0) {
+        const unsigned long long seq = *counter + 1;
+        *counter = seq;
+        __hip_atomic_store(status, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+static_assert(sizeof(RoundState) % 8 == 0 && sizeof(RoundState) / 8 + 1 <= kStatusWords, "status words");
+
+__global__ void __launch_bounds__(kWave) round_status_kernel(const RoundState* st,
+                                                             const unsigned long long* part_weights, int k,
+                                                             unsigned long long* status,
+                                                             unsigned long long* counter) {
+    publish_status(st, [&](int p) { return part_weights[p]; }, st->delta, k, status, counter);
+}
+
+// The part weight moves of a workgroup's committed movers, in LDS.
+struct PartMoves {
+    unsigned long long gained[32], lost[32];
+    __device__ __forceinline__ void clear() {
+        if (threadIdx.x < 32) gained[threadIdx.x] = lost[threadIdx.x] = 0;
+        __syncthreads();
+    }
+    __device__ __forceinline__ void flush(int k, unsigned long long* part_weights) const {
+        if (threadIdx.x < static_cast<unsigned>(k)) {
+            const unsigned long long change = gained[threadIdx.x] - lost[threadIdx.x];
+            if (change) atomicAdd(part_weights + threadIdx.x, change);
+        }
+    }
+};
+
+// incremental_commit (:97-109) of one mover: its label, its lock after an LP round,
+// its weight. Its old part is in flags, so nobody reads a mover's label any more.
+template <typename W>
+__device__ __forceinline__ void commit_mover(std::int32_t v, std::int32_t source, std::int32_t target,
+                                             const W* vertex_weights, std::int32_t* labels, std::int32_t* locks,
+                                             PartMoves& moves) {
+    const auto w = static_cast<unsigned long long>(vertex_weights[v]);
+    atomicAdd(&moves.lost[source], w);
+    atomicAdd(&moves.gained[target], w);
+    labels[v] = target;
+    if (locks) locks[v] = 1;
+}
+
+// incremental_update_cache_and_cut (:69-95) and incremental_commit (:97-109) over a
+// mover list whose length is on the device, G lanes per mover, by the workgroups
+// [0, blocks) numbered `block`; returns the lane's gain. update: false in rebuild
+// rounds, which only commit. flags holds a mover's old part + 1, so labels may
+// change meanwhile: a neighbour's label is read only when it does not move.
 template <typename O, typename W, int G, typename C>
-__device__ __forceinline__ void update_cache_movers(long long count, const std::int32_t* movers, const O* offsets,
-                                                    const std::int32_t* neighbors, const W* weights,
-                                                    const std::int32_t* labels, const std::int32_t* targets,
-                                                    const std::int32_t* flags, int k, C* cache, long long* delta,
-                                                    long long block, long long blocks, long long* block_sum) {
+__device__ __forceinline__ long long update_cache_movers(long long count, const std::int32_t* movers,
+                                                         const O* offsets, const std::int32_t* neighbors,
+                                                         const W* weights, const W* vertex_weights,
+                                                         std::int32_t* labels, const std::int32_t* targets,
+                                                         const std::int32_t* flags, std::int32_t* locks, int k,
+                                                         C* cache, bool update, long long block, long long blocks,
+                                                         PartMoves& moves) {
     const int sub = threadIdx.x & (G - 1);
     const long long groups = blocks * (kBlock / G);
     long long gain = 0;
     for (long long group = (block * blockDim.x + threadIdx.x) / G; group < count; group += groups) {
         const std::int32_t v = movers[group];
-        const std::int32_t source = labels[v];
+        const std::int32_t source = flags[v] - 1;
         const std::int32_t target = targets[v];
+        if (sub == 0) commit_mover(v, source, target, vertex_weights, labels, locks, moves);
+        if (!update) continue;
         for (std::int64_t e = static_cast<std::int64_t>(offsets[v]) + sub; e < offsets[v + 1]; e += G) {
             const std::int32_t u = neighbors[e];
             if (u == v) continue;
@@ -426,44 +557,103 @@ __device__ __forceinline__ void update_cache_movers(long long count, const std::
             // modular arithmetic: entries fit C at every point of the round
             atomicAdd(cache + static_cast<std::int64_t>(u) * k + source, static_cast<C>(0ULL - w));
             atomicAdd(cache + static_cast<std::int64_t>(u) * k + target, static_cast<C>(w));
-            const bool fu = flags[u] != 0;
+            const std::int32_t fu = flags[u];
             if (!fu || u > v) {
-                const std::int32_t lu = labels[u];
+                const std::int32_t lu = fu ? fu - 1 : labels[u];
                 const std::int32_t nu = fu ? targets[u] : lu;
                 gain += static_cast<long long>(w) * ((source != lu) - (target != nu));
             }
         }
     }
-    gain = group_sum_i64<kWave>(gain);
-    if (lane_id() == 0) block_sum[threadIdx.x / kWave] = gain;
+    return gain;
+}
+
+// Adds the workgroup's sum of v to *out with one atomic. Called by every thread
+// of a kBlock-thread workgroup; block_sum holds kBlock / kWave entries.
+__device__ __forceinline__ void block_add_i64(long long v, long long* block_sum, long long* out) {
+    v = group_sum_i64<kWave>(v);
+    if (lane_id() == 0) block_sum[threadIdx.x / kWave] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
         long long total = 0;
         for (int w = 0; w < kBlock / kWave; ++w) total += block_sum[w];
-        if (total) atomicAdd(reinterpret_cast<unsigned long long*>(delta), static_cast<unsigned long long>(total));
+        if (total) atomicAdd(reinterpret_cast<unsigned long long*>(out), static_cast<unsigned long long>(total));
     }
 }
 
-// The light movers (8 lanes each) on workgroups [0, light_blocks), and, when
-// heavy is given, the heavy movers (a wave each) on the rest of the grid.
+// Cache updates and commits of a round. Workgroups [0, light_blocks) take the light
+// movers (8 lanes each); the rest of the grid the heavy movers (a wave each). With
+// no such rest (wave_heavy_blocks == 0) the light workgroups commit the heavy movers,
+// whose entries update_cache_tiles_kernel walks next.
+//
+// status (optional): the last workgroup to finish publishes the round's status, so
+// that the round ends with this launch (commit and status as launches of their own
+// cost 3.8 and 3.6 us per round on the 128^3 mesh). Only workgroups with movers of
+// their own take part (the others return at once), so the arrival counter sees as
+// many atomics as there is work. What the last workgroup reads of the others --
+// part weights and the cut decrease -- was written by device-scope atomics, which
+// have left the workgroup when it arrives (s_waitcnt before its barrier) and are
+// performed past the XCDs' caches; it reads them with device-scope atomic loads. No
+// cache write-back is needed: the labels are read by later launches only.
 template <typename O, typename W, typename C>
-__global__ void __launch_bounds__(kBlock) update_cache_kernel(const RoundState* st, const std::int32_t* light,
-                                                              const std::int32_t* heavy, unsigned light_blocks,
-                                                              const O* offsets, const std::int32_t* neighbors,
-                                                              const W* weights, const std::int32_t* labels,
-                                                              const std::int32_t* targets,
-                                                              const std::int32_t* flags, int k,
-                                                              C* cache, long long* delta, long long rebuild_above) {
+__global__ void __launch_bounds__(kBlock) update_cache_kernel(
+    RoundState* st, const std::int32_t* light, const std::int32_t* heavy, unsigned light_blocks,
+    unsigned wave_heavy_blocks, const O* offsets, const std::int32_t* neighbors, const W* weights,
+    const W* vertex_weights, std::int32_t* labels, const std::int32_t* targets, const std::int32_t* flags,
+    std::int32_t* locks, int k, C* cache, unsigned long long* part_weights, long long rebuild_above,
+    unsigned long long* status, unsigned long long* counter) {
     __shared__ long long block_sum[kBlock / kWave];
+    __shared__ PartMoves moves;
+    __shared__ int last;
     // a rebuild round recomputes cache and cut from the CSR after the commit
-    if (rebuild_above >= 0 && st->edges > rebuild_above) return;
-    if (blockIdx.x < light_blocks)
-        update_cache_movers<O, W, 8, C>(st->light, light, offsets, neighbors, weights, labels, targets, flags, k,
-                                        cache, delta, blockIdx.x, light_blocks, block_sum);
-    else
-        update_cache_movers<O, W, kWave, C>(st->heavy, heavy, offsets, neighbors, weights, labels, targets, flags,
-                                            k, cache, delta, blockIdx.x - light_blocks, gridDim.x - light_blocks,
-                                            block_sum);
+    const bool update = rebuild_above < 0 || st->edges <= rebuild_above;
+    const long long lights = st->light, heavies = st->heavy;
+    // the workgroups with movers: the first `pl` light ones, the first `ph` heavy ones
+    auto blocks_of = [](long long count, long long per, unsigned blocks) {
+        const long long want = (count + per - 1) / per;
+        return static_cast<unsigned>(want < blocks ? want : blocks);
+    };
+    const unsigned pl = blocks_of(wave_heavy_blocks || heavies < lights ? lights : max(lights, heavies),
+                                  kBlock / 8, light_blocks);
+    const unsigned ph = blocks_of(heavies, kBlock / kWave, wave_heavy_blocks);
+    const bool is_light = blockIdx.x < light_blocks;
+    const bool none = pl + ph == 0;
+    if (is_light ? blockIdx.x >= pl && !(none && blockIdx.x == 0) : blockIdx.x - light_blocks >= ph) return;
+    moves.clear();
+    long long gain;
+    if (is_light) {
+        gain = update_cache_movers<O, W, 8, C>(lights, light, offsets, neighbors, weights, vertex_weights, labels,
+                                               targets, flags, locks, k, cache, update, blockIdx.x, max(pl, 1U),
+                                               moves);
+        if (!wave_heavy_blocks)
+            for (long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x; i < heavies;
+                 i += static_cast<long long>(max(pl, 1U)) * kBlock) {
+                const std::int32_t v = heavy[i];
+                commit_mover(v, flags[v] - 1, targets[v], vertex_weights, labels, locks, moves);
+            }
+    } else {
+        gain = update_cache_movers<O, W, kWave, C>(heavies, heavy, offsets, neighbors, weights, vertex_weights,
+                                                   labels, targets, flags, locks, k, cache, update,
+                                                   blockIdx.x - light_blocks, ph, moves);
+    }
+    block_add_i64(gain, block_sum, &st->delta);  // its barrier also completes the LDS sums
+    moves.flush(k, part_weights);
+    if (!status) return;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned long long before = __hip_atomic_fetch_add(&st->arrivals, 1ULL, __ATOMIC_RELAXED,
+                                                                 __HIP_MEMORY_SCOPE_AGENT);
+        last = before + 1 == (none ? 1 : pl + ph);
+    }
+    __syncthreads();
+    if (last && threadIdx.x < kWave) {
+        auto load = [](const unsigned long long* p) {
+            return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        const auto delta = static_cast<long long>(load(reinterpret_cast<const unsigned long long*>(&st->delta)));
+        publish_status(st, [&](int p) { return load(part_weights + p); }, delta, k, status, counter);
+    }
 }
 
 // Heavy movers (degree > kHeavyDegree) as one flattened entry range: heavy_start
@@ -491,7 +681,8 @@ __global__ void heavy_tiles_kernel(const RoundState* st, const long long* heavy_
     }
 }
 
-// incremental_update_cache_and_cut over the heavy movers' entries, kTileRun per lane.
+// incremental_update_cache_and_cut over the heavy movers' entries, kTileRun per lane
+// (update_cache_kernel has committed them; flags holds their old parts).
 template <typename O, typename W, typename C>
 __global__ void __launch_bounds__(kTileLanes) update_cache_tiles_kernel(
     const RoundState* st, const long long* heavy_start, const std::int32_t* tile_mover, const std::int32_t* movers,
@@ -509,14 +700,14 @@ __global__ void __launch_bounds__(kTileLanes) update_cache_tiles_kernel(
         std::int32_t i;
         if (!tile_run(heavy_start, tile_mover, tiles, count, total, t, &x, &stop, &i)) continue;
         std::int32_t v = movers[i];
-        std::int32_t source = labels[v], target = targets[v];
+        std::int32_t source = flags[v] - 1, target = targets[v];
         long long next = heavy_start[i + 1];
         std::int64_t base = static_cast<std::int64_t>(offsets[v]) - heavy_start[i];
         for (; x < stop; ++x) {
             while (x >= next) {
                 ++i;
                 v = movers[i];
-                source = labels[v];
+                source = flags[v] - 1;
                 target = targets[v];
                 base = static_cast<std::int64_t>(offsets[v]) - heavy_start[i];
                 next = heavy_start[i + 1];
@@ -527,84 +718,17 @@ __global__ void __launch_bounds__(kTileLanes) update_cache_tiles_kernel(
             const auto w = static_cast<unsigned long long>(weights[e]);
             atomicAdd(cache + static_cast<std::int64_t>(u) * k + source, static_cast<C>(0ULL - w));
             atomicAdd(cache + static_cast<std::int64_t>(u) * k + target, static_cast<C>(w));
-            const bool fu = flags[u] != 0;
+            const std::int32_t fu = flags[u];
             if (!fu || u > v) {
-                const std::int32_t lu = labels[u];
+                const std::int32_t lu = fu ? fu - 1 : labels[u];
                 const std::int32_t nu = fu ? targets[u] : lu;
                 gain += static_cast<long long>(w) * ((source != lu) - (target != nu));
             }
         }
     }
-    gain = group_sum_i64<kWave>(gain);
-    if (lane_id() == 0) block_sum[threadIdx.x / kWave] = gain;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        long long sum = 0;
-        for (int w = 0; w < kTileLanes / kWave; ++w) sum += block_sum[w];
-        if (sum) atomicAdd(reinterpret_cast<unsigned long long*>(delta), static_cast<unsigned long long>(sum));
-    }
+    static_assert(kTileLanes == kBlock, "block_add_i64 sums a kBlock-thread workgroup");
+    block_add_i64(gain, block_sum, delta);
 }
-
-// incremental_commit (:97-109) over light then heavy movers; part weight changes
-// are summed per workgroup before they reach the k global counters.
-template <typename W>
-__global__ void __launch_bounds__(kBlock) commit_kernel(const RoundState* st, const std::int32_t* light,
-                                                        const std::int32_t* heavy, std::int32_t* labels,
-                                                        const std::int32_t* targets, const W* vertex_weights,
-                                                        unsigned long long* part_weights, std::int32_t* locks,
-                                                        bool lp, int k) {
-    __shared__ unsigned long long gained[32], lost[32];
-    if (threadIdx.x < 32) gained[threadIdx.x] = lost[threadIdx.x] = 0;
-    __syncthreads();
-    const long long nl = st->light, total = nl + st->heavy;
-    for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
-         i += static_cast<long long>(gridDim.x) * blockDim.x) {
-        const std::int32_t v = i < nl ? light[i] : heavy[i - nl];
-        const std::int32_t source = labels[v];
-        const std::int32_t target = targets[v];
-        const auto w = static_cast<unsigned long long>(vertex_weights[v]);
-        atomicAdd(&lost[source], w);
-        atomicAdd(&gained[target], w);
-        labels[v] = target;
-        if (lp) locks[v] = 1;
-    }
-    __syncthreads();
-    if (threadIdx.x < k) {
-        const unsigned long long change = gained[threadIdx.x] - lost[threadIdx.x];
-        if (change) atomicAdd(part_weights + threadIdx.x, change);
-    }
-}
-
-// The round's status, also copied to the host-visible status words (word 0: seq,
-// stored last, after a system-scope fence).
-// One wave: lane p < k holds part p's weight; every lane writes one status word.
-__global__ void __launch_bounds__(kWave) round_status_kernel(RoundState* st, const unsigned long long* part_weights,
-                                                             int k, unsigned long long* status,
-                                                             unsigned long long* counter) {
-    constexpr int kHead = static_cast<int>(offsetof(RoundState, pw) / 8);  // words before pw
-    const int lane = threadIdx.x;
-    const unsigned long long w = lane < k ? part_weights[lane] : 0;
-    unsigned long long maximum = w;
-    for (int m = kWave / 2; m > 0; m /= 2) {
-        const unsigned long long o = shfl_xor_u64(maximum, m, kWave);
-        maximum = o > maximum ? o : maximum;
-    }
-    if (lane < 32) st->pw[lane] = w;
-    if (lane == 0) st->max_weight = maximum;
-    __syncthreads();
-    // words of the head (with max_weight) and pw[0, k): a store per lane, in parallel
-    const auto* words = reinterpret_cast<const unsigned long long*>(st);
-    if (lane < kHead + k) status[1 + lane] = words[lane];
-    __threadfence_system();
-    __syncthreads();
-    if (lane == 0) {
-        const unsigned long long seq = *counter + 1;
-        *counter = seq;
-        __hip_atomic_store(status, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-}
-static_assert(sizeof(RoundState) % 8 == 0 && sizeof(RoundState) / 8 + 1 <= kStatusWords, "status words");
-static_assert(offsetof(RoundState, pw) / 8 + 32 <= static_cast<std::size_t>(kWave), "one wave writes the status");
 
 // Movers are split by degree so the cache update can give heavy rows a workgroup.
 struct MoverPair {
@@ -658,48 +782,6 @@ struct MoverStore {
 // the weight of the lower-id members of their bucket (a blocked multisplit),
 // one legal outcome of the reference's atomicAdd ranking.
 
-// Appends the taking threads' vertices to the light/heavy mover lists (one
-// global atomic per list per workgroup pass) and flags them. Called by every
-// thread of the workgroup.
-template <typename O>
-__device__ void append_movers(bool take, std::int32_t v, const O* offsets, std::int32_t* light,
-                              std::int32_t* heavy, std::int32_t* flags, RoundState* st, unsigned* counts,
-                              unsigned long long* base) {
-    const int lane = lane_id(), wave = threadIdx.x / kWave;
-    const long long degree = take ? static_cast<long long>(offsets[v + 1] - offsets[v]) : 0;
-    const bool is_heavy = degree > kHeavyDegree;
-    const long long edges = group_sum_i64<kWave>(degree);
-    if (lane == 0 && edges) atomicAdd(reinterpret_cast<unsigned long long*>(&st->edges),
-                                      static_cast<unsigned long long>(edges));
-    const bool is_light = take && !is_heavy;
-    const unsigned long long bl = __ballot(is_light), bh = __ballot(is_heavy);
-    if (lane == 0) {
-        counts[wave] = static_cast<unsigned>(__popcll(bl));
-        counts[kBlock / kWave + wave] = static_cast<unsigned>(__popcll(bh));
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned tl = 0, th = 0;
-        for (int q = 0; q < kBlock / kWave; ++q) {
-            tl += counts[q];
-            th += counts[kBlock / kWave + q];
-        }
-        base[0] = tl ? atomicAdd(reinterpret_cast<unsigned long long*>(&st->light), tl) : 0;
-        base[1] = th ? atomicAdd(reinterpret_cast<unsigned long long*>(&st->heavy), th) : 0;
-    }
-    __syncthreads();
-    if (take) {
-        unsigned before = 0;
-        const unsigned* row = is_heavy ? counts + kBlock / kWave : counts;
-        for (int q = 0; q < wave; ++q) before += row[q];
-        const unsigned long long mask = is_heavy ? bh : bl;
-        before += static_cast<unsigned>(__popcll(mask & lanemask_lt()));
-        (is_heavy ? heavy : light)[(is_heavy ? base[1] : base[0]) + before] = v;
-        flags[v] = 1;
-    }
-    __syncthreads();
-}
-
 // Candidates: vertices of overloaded parts, in id order. Every flag is cleared
 // on the way (movers are flagged later in the iteration).
 struct OverloadedLoad {
@@ -722,6 +804,103 @@ struct CandidateStore {
         if (v == n - 1) st->candidates = prefix + item;
     }
 };
+
+// The choice of incremental_rebalance_proposals (:111-157) for one vertex of an
+// overloaded part, by a group of G lanes, lane j owning parts [8j, 8j + 8) of its
+// cache row: the destination (-1: none) and the source bucket (-1: none). pw: the
+// part weights (LDS). Every lane returns both.
+struct BalanceChoice {
+    int target;
+    int bucket;
+};
+template <int G, typename C>
+__device__ __forceinline__ BalanceChoice balance_choice(std::int64_t v, std::int32_t source, std::uint64_t weight,
+                                                        const C* cache, int j, int k, const unsigned long long* pw,
+                                                        std::uint64_t capacity, const PowerTable& powers) {
+    const C* row = cache + v * k;
+    unsigned long long slack[kRowSpan];
+    unsigned long long conn = 0, best_slack = 0, current = 0;
+    int bp = 0x7fffffff;
+    unsigned long long span[kRowSpan];
+    load_span(row, j, k, span);
+    // lane-local best by (conn, slack), lowest index on ties (ascending p)
+#pragma unroll
+    for (int e = 0; e < kRowSpan; ++e) {
+        const int p = j * kRowSpan + e;
+        const unsigned long long value = span[e];
+        if (p == source) current = value;
+        const bool ok = p < k && p != source && pw[p] < capacity && weight <= capacity - pw[p];
+        slack[e] = ok ? capacity - pw[p] : 0;
+        if (ok && (bp == 0x7fffffff || value > conn || (value == conn && slack[e] > best_slack))) {
+            conn = value;
+            best_slack = slack[e];
+            bp = p;
+        }
+    }
+#pragma unroll
+    for (int m = G / 2; m > 0; m /= 2) {
+        const auto oc = shfl_xor_u64(conn, m, G);
+        const auto os = shfl_xor_u64(best_slack, m, G);
+        const int op = static_cast<int>(lane_xor(static_cast<unsigned>(bp), m, G));
+        const auto ocur = shfl_xor_u64(current, m, G);
+        const bool ob = op != 0x7fffffff;
+        const bool mine = bp != 0x7fffffff;
+        if (ob && (!mine || oc > conn || (oc == conn && (os > best_slack || (os == best_slack && op < bp))))) {
+            conn = oc;
+            best_slack = os;
+            bp = op;
+        }
+        current = ocur > current ? ocur : current;  // only the source's lane holds it
+    }
+    int best = bp == 0x7fffffff ? -1 : bp;
+    if (best >= 0 && conn == 0) {
+        // No affinity anywhere: a ticket mix32(v) mod total slack walks the
+        // eligible parts in index order. Saturating sums of non-negative terms do
+        // not depend on the order of addition, so the running total before part p
+        // is the lane's running prefix plus the saturated total of lower lanes;
+        // the walk stops at the first part whose running total exceeds the ticket.
+        unsigned long long running[kRowSpan];
+        unsigned long long lane_total = 0;
+#pragma unroll
+        for (int e = 0; e < kRowSpan; ++e) {
+            lane_total = ~0ULL - lane_total < slack[e] ? ~0ULL : lane_total + slack[e];
+            running[e] = lane_total;
+        }
+        unsigned long long inclusive = lane_total;
+#pragma unroll
+        for (int d = 1; d < G; d <<= 1) {
+            const auto other = shfl_up_u64(inclusive, d, G);
+            if (j >= d) inclusive = ~0ULL - inclusive < other ? ~0ULL : inclusive + other;
+        }
+        const unsigned long long before = G > 1 ? shfl_up_u64(inclusive, 1, G) : 0;
+        const unsigned long long lower = j > 0 ? before : 0;
+        const unsigned long long total = shfl_u64(inclusive, G - 1, G);  // > 0: some part is eligible
+        const std::uint32_t hash = mix32(static_cast<std::uint32_t>(v));
+        const unsigned long long ticket =
+            total > 0xffffffffULL ? hash : hash % static_cast<std::uint32_t>(total);
+        int hit = 0x7fffffff;
+#pragma unroll
+        for (int e = kRowSpan - 1; e >= 0; --e) {
+            const unsigned long long upto = ~0ULL - lower < running[e] ? ~0ULL : lower + running[e];
+            if (upto > ticket) hit = j * kRowSpan + e;
+        }
+#pragma unroll
+        for (int m = G / 2; m > 0; m /= 2) {
+            const int other = static_cast<int>(lane_xor(static_cast<unsigned>(hit), m, G));
+            hit = other < hit ? other : hit;
+        }
+        best = hit;
+    }
+    int bucket = -1;
+    if (best >= 0) {
+        const double gain =
+            conn >= current ? static_cast<double>(conn - current) : -static_cast<double>(current - conn);
+        const double per_weight = gain / static_cast<double>(weight);
+        bucket = source * kBalanceWidth + gain_bucket(per_weight, powers) * kBalanceSections +
+                 static_cast<int>(mix32(static_cast<std::uint32_t>(v)) % kBalanceSections);
+    }
+    return BalanceChoice{best, bucket};
+}
 
 // incremental_rebalance_proposals (:111-157) + balance_source_histogram (:174-186).
 // One group of G lanes per candidate, lane j owning parts [8j, 8j + 8).
@@ -751,96 +930,284 @@ __global__ void __launch_bounds__(kBlock) balance_proposals_kernel(RoundState* s
         const std::int64_t v = cand[index];
         const std::int32_t source = labels[v];
         const std::uint64_t weight = static_cast<std::uint64_t>(vertex_weights[v]);
-        const C* row = cache + v * k;
-        unsigned long long slack[kRowSpan];
-        unsigned long long conn = 0, best_slack = 0, current = 0;
-        int bp = 0x7fffffff;
-        unsigned long long span[kRowSpan];
-        load_span(row, j, k, span);
-        // lane-local best by (conn, slack), lowest index on ties (ascending p)
-#pragma unroll
-        for (int e = 0; e < kRowSpan; ++e) {
-            const int p = j * kRowSpan + e;
-            const unsigned long long value = span[e];
-            if (p == source) current = value;
-            const bool ok = p < k && p != source && pw[p] < capacity && weight <= capacity - pw[p];
-            slack[e] = ok ? capacity - pw[p] : 0;
-            if (ok && (bp == 0x7fffffff || value > conn || (value == conn && slack[e] > best_slack))) {
-                conn = value;
-                best_slack = slack[e];
-                bp = p;
-            }
-        }
-#pragma unroll
-        for (int m = G / 2; m > 0; m /= 2) {
-            const auto oc = shfl_xor_u64(conn, m, G);
-            const auto os = shfl_xor_u64(best_slack, m, G);
-            const int op = __shfl_xor(bp, m, G);
-            const auto ocur = shfl_xor_u64(current, m, G);
-            const bool ob = op != 0x7fffffff;
-            const bool mine = bp != 0x7fffffff;
-            if (ob && (!mine || oc > conn || (oc == conn && (os > best_slack || (os == best_slack && op < bp))))) {
-                conn = oc;
-                best_slack = os;
-                bp = op;
-            }
-            current = ocur > current ? ocur : current;  // only the source's lane holds it
-        }
-        int best = bp == 0x7fffffff ? -1 : bp;
-        if (best >= 0 && conn == 0) {
-            // No affinity anywhere: a ticket mix32(v) mod total slack walks the
-            // eligible parts in index order. Saturating sums of non-negative terms do
-            // not depend on the order of addition, so the running total before part p
-            // is the lane's running prefix plus the saturated total of lower lanes;
-            // the walk stops at the first part whose running total exceeds the ticket.
-            unsigned long long running[kRowSpan];
-            unsigned long long lane_total = 0;
-#pragma unroll
-            for (int e = 0; e < kRowSpan; ++e) {
-                lane_total = ~0ULL - lane_total < slack[e] ? ~0ULL : lane_total + slack[e];
-                running[e] = lane_total;
-            }
-            unsigned long long inclusive = lane_total;
-#pragma unroll
-            for (int d = 1; d < G; d <<= 1) {
-                const auto other = shfl_up_u64(inclusive, d, G);
-                if (j >= d) inclusive = ~0ULL - inclusive < other ? ~0ULL : inclusive + other;
-            }
-            const unsigned long long before = G > 1 ? shfl_up_u64(inclusive, 1, G) : 0;
-            const unsigned long long lower = j > 0 ? before : 0;
-            const unsigned long long total = shfl_u64(inclusive, G - 1, G);  // > 0: some part is eligible
-            const std::uint32_t hash = mix32(static_cast<std::uint32_t>(v));
-            const unsigned long long ticket =
-                total > 0xffffffffULL ? hash : hash % static_cast<std::uint32_t>(total);
-            int hit = 0x7fffffff;
-#pragma unroll
-            for (int e = kRowSpan - 1; e >= 0; --e) {
-                const unsigned long long upto = ~0ULL - lower < running[e] ? ~0ULL : lower + running[e];
-                if (upto > ticket) hit = j * kRowSpan + e;
-            }
-#pragma unroll
-            for (int m = G / 2; m > 0; m /= 2) {
-                const int other = __shfl_xor(hit, m, G);
-                hit = other < hit ? other : hit;
-            }
-            best = hit;
-        }
+        const BalanceChoice choice = balance_choice<G, C>(v, source, weight, cache, j, k, pw, capacity, powers);
         if (j == 0) {
-            int bucket = -1;
-            if (best >= 0) {
-                const double gain =
-                    conn >= current ? static_cast<double>(conn - current) : -static_cast<double>(current - conn);
-                const double per_weight = gain / static_cast<double>(weight);
-                bucket = source * kBalanceWidth + gain_bucket(per_weight, powers) * kBalanceSections +
-                         static_cast<int>(mix32(static_cast<std::uint32_t>(v)) % kBalanceSections);
-                table_add(table, static_cast<unsigned>(bucket), weight, counts);
-            }
-            targets[v] = best;
-            cbucket[index] = bucket;
+            if (choice.bucket >= 0) table_add(table, static_cast<unsigned>(choice.bucket), weight, counts);
+            targets[v] = choice.target;
+            cbucket[index] = choice.bucket;
         }
     }
     __syncthreads();
     table_flush(table, counts);
+}
+
+// ---------------------------------------------------------------- small levels
+//
+// A rebalance iteration of a level of at most kSelectVertices vertices takes three
+// launches: the proposals of every vertex (no candidate list: a vertex of a part
+// within capacity is skipped), both selections in one workgroup, and the update.
+// Such a level is bound by its chain of launches, each 3-5 us whatever it does: the
+// ten launches these two replace (candidate scan, proposals, two bucket scans, two
+// times two selections, commit, status) took 46-65 us per iteration with the host's
+// wait, on levels of 669 to 12,220 vertices.
+
+// balance_choice for every vertex of an overloaded part. choices[v]: the bucket
+// within a part in bits 0-9, the source part in bits 10-14, the destination in bits
+// 15-19; -1 for a vertex without a destination, -2 for one of no overloaded part.
+// Flags and the round state are cleared on the way.
+constexpr int kNoCandidate = -2;
+constexpr int kBucketBits = 10, kSourceShift = 10, kTargetShift = 15;
+static_assert(kBalanceWidth <= 1 << kBucketBits, "a part's buckets fit their field");
+template <typename W, int G, typename C>
+__global__ void __launch_bounds__(kBlock) balance_vertices_kernel(RoundState* st, std::int64_t n, const C* cache,
+                                                                  const std::int32_t* labels, const W* vertex_weights,
+                                                                  int k, const unsigned long long* part_weights,
+                                                                  std::uint64_t capacity, PowerTable powers,
+                                                                  std::int32_t* targets, std::int32_t* choices,
+                                                                  std::int32_t* flags) {
+    __shared__ unsigned long long pw[32];
+    if (blockIdx.x == 0 && threadIdx.x < sizeof(RoundState) / 8)
+        reinterpret_cast<unsigned long long*>(st)[threadIdx.x] = 0;
+    if (threadIdx.x < 32) pw[threadIdx.x] = threadIdx.x < static_cast<unsigned>(k) ? part_weights[threadIdx.x] : 0;
+    __syncthreads();
+    const std::int64_t v = (static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / G;
+    if (v >= n) return;  // uniform per group
+    const int j = threadIdx.x & (G - 1);
+    const std::int32_t source = labels[v];
+    BalanceChoice choice{-1, kNoCandidate};
+    if (pw[source] > capacity)  // uniform per group
+        choice = balance_choice<G, C>(v, source, static_cast<std::uint64_t>(vertex_weights[v]), cache, j, k, pw,
+                                      capacity, powers);
+    if (j == 0) {
+        targets[v] = choice.target;
+        choices[v] = choice.bucket < 0 ? choice.bucket
+                                       : choice.bucket - source * kBalanceWidth + (source << kSourceShift) +
+                                             (choice.target << kTargetShift);
+        flags[v] = 0;
+    }
+}
+
+// Both selections of an iteration in one workgroup. A wave owns 64 * Items
+// consecutive vertices, lane l's item i the one at 64 * i + l (every load of a wave
+// is one run; Items consecutive vertices per lane took 41 instead of 27 us at 12,220
+// vertices); the choices stay in registers. The bucket histogram of the
+// sources, then of the destinations, is summed in LDS: 32 parts x 800 buckets of 32
+// bits when the part weights' total fits, else 16 parts x 800 of 64 bits per window.
+// Within a part the members before the first bucket that reaches its threshold are
+// taken, those behind it refused (source_side and destination_side state the same
+// tests). That bucket's own members of all parts are gathered in id order into the
+// histogram's space and ranked together, kSelectThreads at a time.
+constexpr int kSelectThreads = 1024;
+constexpr int kSelectMaxItems = 16;
+constexpr std::int64_t kSelectVertices = kSelectThreads * kSelectMaxItems;
+constexpr int kSelectWaves = kSelectThreads / kWave;
+struct SelectShared {
+    union {
+        unsigned narrow[32 * kBalanceWidth];
+        unsigned long long wide[16 * kBalanceWidth];
+        struct {
+            std::int32_t vertex[kSelectVertices];
+            unsigned char part[kSelectVertices];   // its part
+            unsigned char taken[kSelectVertices];  // the outcome
+        } pending;
+    } u;
+    unsigned long long pw[32];
+    unsigned long long running[32];  // weight before the boundary bucket, then before the next member
+    int boundary[32];                // the boundary bucket, kBalanceWidth: every bucket is taken
+    unsigned long long waves[2][kSelectWaves];
+    unsigned long long wave_total[kSelectWaves][32];
+};
+
+// Exclusive prefix of one value per thread over the kSelectThreads threads, and
+// their total: one barrier (the wave totals are scanned by every wave itself);
+// successive calls alternate `slot`, so that a call's totals are not overwritten
+// before every wave has read them.
+__device__ __forceinline__ unsigned long long select_scan(unsigned long long value, unsigned long long* total,
+                                                          SelectShared& sh, int slot) {
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    const unsigned long long inclusive = wave_scan(value);
+    if (lane == kWave - 1) sh.waves[slot][wave] = inclusive;
+    __syncthreads();
+    const unsigned long long sums = wave_scan(lane < kSelectWaves ? sh.waves[slot][lane] : 0ULL);
+    *total = read_lane(sums, kSelectWaves - 1);
+    const auto below = read_lane(sums, __builtin_amdgcn_readfirstlane(wave > 0 ? wave - 1 : 0));
+    return (wave > 0 ? below : 0) + inclusive - value;
+}
+
+template <typename O, typename W, int Items>
+__global__ void __launch_bounds__(kSelectThreads) balance_select_kernel(
+    RoundState* st, std::int64_t n, const std::int32_t* choices, const W* vertex_weights, const O* offsets, int k,
+    const unsigned long long* part_weights, std::uint64_t capacity, std::int32_t* light, std::int32_t* heavy,
+    std::int32_t* flags) {
+    __shared__ SelectShared sh;
+    const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
+    const int first = wave * kWave * Items + lane;
+    const int count_n = static_cast<int>(n);
+    int item[Items];
+    W weight[Items];
+#pragma unroll
+    for (int i = 0; i < Items; ++i) item[i] = first + i * kWave < count_n ? choices[first + i * kWave] : kNoCandidate;
+#pragma unroll
+    for (int i = 0; i < Items; ++i) weight[i] = first + i * kWave < count_n ? vertex_weights[first + i * kWave] : W{0};
+    if (t < 32) sh.pw[t] = t < k ? part_weights[t] : 0;
+    __syncthreads();
+    unsigned long long total = 0;
+    for (int p = 0; p < k; ++p) total += sh.pw[p];
+    const bool narrow = total <= 0xffffffffULL;
+    const int window = narrow ? 32 : 16;
+    unsigned long long candidates = 0;
+    unsigned in = 0;  // the items that take part in the selection
+#pragma unroll
+    for (int i = 0; i < Items; ++i) {
+        candidates += item[i] != kNoCandidate;
+        in |= static_cast<unsigned>(item[i] >= 0) << i;
+    }
+
+    auto threshold = [&](int p, bool destinations) -> unsigned long long {
+        const unsigned long long w = sh.pw[p];
+        return destinations ? (w < capacity ? capacity - w : 0) : (w > capacity ? w - capacity : 0);
+    };
+    // Selects among the items in `in`, by the part at `shift`: the mask of the taken.
+    auto select = [&](int shift, bool destinations) -> unsigned {
+        for (int base = 0; base < k; base += window) {
+            const int parts = min(window, k - base);
+            if (narrow) {
+                for (int b = t; b < parts * kBalanceWidth; b += kSelectThreads) sh.u.narrow[b] = 0;
+            } else {
+                for (int b = t; b < parts * kBalanceWidth; b += kSelectThreads) sh.u.wide[b] = 0;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < Items; ++i) {
+                const int q = (item[i] >> shift & 31) - base;
+                if (!(in >> i & 1U) || q < 0 || q >= parts) continue;
+                const int b = q * kBalanceWidth + (item[i] & ((1 << kBucketBits) - 1));
+                if (narrow) atomicAdd(&sh.u.narrow[b], static_cast<unsigned>(weight[i]));
+                else atomicAdd(&sh.u.wide[b], static_cast<unsigned long long>(weight[i]));
+            }
+            __syncthreads();
+            // a wave per part, 13 buckets per lane
+            constexpr int kPer = (kBalanceWidth + kWave - 1) / kWave;
+            for (int q = wave; q < parts; q += kSelectWaves) {
+                const unsigned long long limit = threshold(base + q, destinations);
+                if (!destinations && limit == 0) continue;  // not overloaded: no members
+                unsigned long long count[kPer], sum = 0;
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) {
+                    const int b = lane * kPer + i;
+                    count[i] = b >= kBalanceWidth ? 0
+                               : narrow           ? sh.u.narrow[q * kBalanceWidth + b]
+                                                  : sh.u.wide[q * kBalanceWidth + b];
+                    sum += count[i];
+                }
+                unsigned long long running = wave_scan(sum) - sum, at = 0;
+                int found = kBalanceWidth;
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) {
+                    const bool reached = destinations ? running + count[i] > limit : running + count[i] >= limit;
+                    if (reached && found == kBalanceWidth && lane * kPer + i < kBalanceWidth) {
+                        found = lane * kPer + i;
+                        at = running;
+                    }
+                    running += count[i];
+                }
+                const unsigned long long lanes = __ballot(found < kBalanceWidth);
+                const int owner = lanes ? __ffsll(static_cast<unsigned long long>(lanes)) - 1 : 0;
+                if (lane == owner) {
+                    sh.boundary[base + q] = found;
+                    sh.running[base + q] = at;
+                }
+            }
+            __syncthreads();
+        }
+        unsigned taken = 0, pending = 0;
+#pragma unroll
+        for (int i = 0; i < Items; ++i) {
+            if (!(in >> i & 1U)) continue;
+            const int b = item[i] & ((1 << kBucketBits) - 1), boundary = sh.boundary[item[i] >> shift & 31];
+            if (b < boundary) taken |= 1U << i;
+            else if (b == boundary) pending |= 1U << i;
+        }
+        // the wave's pending items in id order, from the waves' totals
+        int in_wave = 0;
+#pragma unroll
+        for (int i = 0; i < Items; ++i) in_wave += __popcll(__ballot(pending >> i & 1U));
+        unsigned long long members;
+        const auto at = static_cast<int>(
+            select_scan(lane == 0 ? static_cast<unsigned long long>(in_wave) : 0ULL, &members, sh, destinations ? 1 : 0));
+        const int wave_at = static_cast<int>(read_lane(static_cast<unsigned>(at), 0));
+        int slot = wave_at;
+#pragma unroll
+        for (int i = 0; i < Items; ++i) {
+            const unsigned long long lanes = __ballot(pending >> i & 1U);
+            if (pending >> i & 1U) {
+                const int x = slot + __popcll(lanes & lanemask_lt());
+                sh.u.pending.vertex[x] = first + i * kWave;
+                sh.u.pending.part[x] = static_cast<unsigned char>(item[i] >> shift & 31);
+            }
+            slot += __popcll(lanes);
+        }
+        __syncthreads();
+        for (int base = 0; base < static_cast<int>(members); base += kSelectThreads) {
+            const int x = base + t;
+            const bool member = x < static_cast<int>(members);
+            const int p = member ? sh.u.pending.part[x] : 0;
+            const unsigned long long w =
+                member ? static_cast<unsigned long long>(vertex_weights[sh.u.pending.vertex[x]]) : 0;
+            const unsigned long long rank = block_key_prefix<kSelectThreads>(member, p, w, sh.wave_total, sh.running);
+            const unsigned long long limit = threshold(p, destinations);
+            if (member) sh.u.pending.taken[x] = destinations ? rank + w <= limit : rank < limit;
+        }
+        __syncthreads();
+        slot = wave_at;
+#pragma unroll
+        for (int i = 0; i < Items; ++i) {
+            const unsigned long long lanes = __ballot(pending >> i & 1U);
+            if (pending >> i & 1U && sh.u.pending.taken[slot + __popcll(lanes & lanemask_lt())]) taken |= 1U << i;
+            slot += __popcll(lanes);
+        }
+        __syncthreads();
+        return taken;
+    };
+
+    in = select(kSourceShift, false);
+    const unsigned moving = select(kTargetShift, true);
+
+    // the mover lists (their order does not matter)
+    unsigned long long counts = 0, edges = 0;
+    unsigned is_heavy = 0;
+#pragma unroll
+    for (int i = 0; i < Items; ++i) {
+        if (!(moving >> i & 1U)) continue;
+        const int v = first + i * kWave;
+        const auto degree = static_cast<unsigned long long>(offsets[v + 1] - offsets[v]);
+        edges += degree;
+        if (degree > kHeavyDegree) is_heavy |= 1U << i;
+        counts += degree > kHeavyDegree ? 1ULL << 20 : 1ULL;
+    }
+    // light movers, heavy movers and candidates in 20 bits each (at most 2^14)
+    unsigned long long listed, all_edges;
+    unsigned long long at = select_scan(counts | candidates << 40, &listed, sh, 0) & 0xffffffffffULL;
+    (void)select_scan(edges, &all_edges, sh, 1);
+#pragma unroll
+    for (int i = 0; i < Items; ++i) {
+        if (!(moving >> i & 1U)) continue;
+        const int v = first + i * kWave;
+        if (is_heavy >> i & 1U) {
+            heavy[at >> 20] = v;
+            at += 1ULL << 20;
+        } else {
+            light[at & 0xfffffU] = v;
+            at += 1;
+        }
+        flags[v] = (item[i] >> kSourceShift & 31) + 1;
+    }
+    if (t == 0) {
+        st->light = static_cast<long long>(listed & 0xfffffU);
+        st->heavy = static_cast<long long>(listed >> 20 & 0xfffffU);
+        st->edges = static_cast<long long>(all_edges);
+        st->candidates = static_cast<long long>(listed >> 40);
+    }
 }
 
 // balance_scan_buckets (:188-202): bucket totals (the kReplicas copies summed),
@@ -1045,7 +1412,8 @@ template <typename O, typename W>
 __global__ void __launch_bounds__(kBlock) balance_destinations_kernel(
     RoundState* st, const std::int32_t* cand, std::int32_t* dbucket, const W* vertex_weights, const O* offsets_csr,
     const unsigned long long* counts, const unsigned long long* offsets, const unsigned long long* thresholds,
-    unsigned long long* block_sums, std::int32_t* light, std::int32_t* heavy, std::int32_t* flags) {
+    unsigned long long* block_sums, const std::int32_t* labels, std::int32_t* light, std::int32_t* heavy,
+    std::int32_t* flags) {
     __shared__ unsigned long long sums[32];
     __shared__ unsigned counts_lds[2 * (kBlock / kWave)];
     __shared__ unsigned long long base_lds[2];
@@ -1065,13 +1433,14 @@ __global__ void __launch_bounds__(kBlock) balance_destinations_kernel(
                 const BucketSide side = destination_side(offsets[d], counts[d], thresholds[part]);
                 if (side == kTaken) {
                     take = true;
+                    flags[v] = labels[v] + 1;
                 } else if (side == kBoundary) {
                     dbucket[i] = -3 - d;
                     atomicAdd(&sums[part], static_cast<unsigned long long>(vertex_weights[v]));
                 }
             }
         }
-        append_movers(take, v, offsets_csr, light, heavy, flags, st, counts_lds, base_lds);
+        append_movers(take, v, offsets_csr, light, heavy, st, counts_lds, base_lds);
     }
     if (threadIdx.x < 32) block_sums[static_cast<long long>(blockIdx.x) * 32 + threadIdx.x] = sums[threadIdx.x];
 }
@@ -1081,8 +1450,8 @@ template <typename O, typename W>
 __global__ void __launch_bounds__(kBlock) balance_destination_ranks_kernel(
     RoundState* st, const std::int32_t* cand, const std::int32_t* dbucket, const W* vertex_weights,
     const O* offsets_csr, const unsigned long long* offsets, const unsigned long long* thresholds,
-    const unsigned long long* column_prefix, const unsigned long long* block_sums, std::int32_t* light,
-    std::int32_t* heavy, std::int32_t* flags) {
+    const unsigned long long* column_prefix, const unsigned long long* block_sums, const std::int32_t* labels,
+    std::int32_t* light, std::int32_t* heavy, std::int32_t* flags) {
     __shared__ unsigned long long wave_total[kBlock / kWave][32];
     __shared__ unsigned long long running[32];
     __shared__ unsigned long long groups[kBlock / 32][32];
@@ -1108,7 +1477,8 @@ __global__ void __launch_bounds__(kBlock) balance_destination_ranks_kernel(
         }
         const unsigned long long rank = block_key_prefix<kBlock>(pending, part, w, wave_total, running);
         const bool take = pending && offsets[d] + rank + w <= thresholds[part];
-        append_movers(take, v, offsets_csr, light, heavy, flags, st, counts_lds, base_lds);
+        if (take) flags[v] = labels[v] + 1;
+        append_movers(take, v, offsets_csr, light, heavy, st, counts_lds, base_lds);
     }
 }
 
@@ -1414,19 +1784,27 @@ struct Ops {
                     (n + 1) * sizeof(O) + m * (4 + sizeof(W)) + 4 * m + static_cast<double>(sizeof(C)) * n * k);
     }
 
+    // append: the movers also go to the round's lists (levels without hub rows only).
     static void filter_movers(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
                               const std::int32_t* labels, const std::int32_t* targets, const long long* gains,
-                              std::int32_t* flags) {
+                              std::int32_t* flags, bool append, std::int32_t* light, std::int32_t* heavy,
+                              RoundState* st) {
         const auto* off = static_cast<const O*>(g->offsets);
         const auto* w = static_cast<const W*>(g->edge_weights);
         profile_begin(ctx, GPART_PROFILE_REFINE_FILTER);
         const unsigned low_blocks = grid_for(c->low_count * 8), medium_blocks = grid_for(c->medium_count * 64);
         const auto high_blocks = static_cast<unsigned>(c->high_count);
-        if (low_blocks + medium_blocks + high_blocks > 0)
-            hipLaunchKernelGGL((priority_filter_kernel<O, W>), dim3(low_blocks + medium_blocks + high_blocks),
-                               dim3(kBlock), 0, ctx->stream, c->low_count, c->low, low_blocks, c->medium_count,
-                               c->medium, medium_blocks, c->high_count, c->high, off, g->neighbors, w, labels,
-                               targets, gains, flags);
+        const unsigned blocks = low_blocks + medium_blocks + high_blocks;
+        if (blocks > 0 && append)
+            hipLaunchKernelGGL((priority_filter_kernel<O, W, true>), dim3(blocks), dim3(kBlock), 0, ctx->stream,
+                               c->low_count, c->low, low_blocks, c->medium_count, c->medium, medium_blocks,
+                               c->high_count, c->high, off, g->neighbors, w, labels, targets, gains, flags, light,
+                               heavy, st);
+        else if (blocks > 0)
+            hipLaunchKernelGGL((priority_filter_kernel<O, W, false>), dim3(blocks), dim3(kBlock), 0, ctx->stream,
+                               c->low_count, c->low, low_blocks, c->medium_count, c->medium, medium_blocks,
+                               c->high_count, c->high, off, g->neighbors, w, labels, targets, gains, flags, light,
+                               heavy, st);
         if (c->max_degree > kHubChunk) {
             HubChunks chunks;
             build_hub_chunks(ctx, off, c->high, c->high_count, c->high_edges, kHubChunk, chunks);
@@ -1436,8 +1814,8 @@ struct Ops {
                                chunks.total(), chunks.start.get(), chunks.hub.get(), c->high, off, g->neighbors, w,
                                labels, targets, gains, sums.get());
             hipLaunchKernelGGL(priority_filter_hub_finish_kernel, dim3(grid_for(c->high_count)), dim3(kBlock), 0,
-                               ctx->stream, c->high_count, chunks.start.get(), c->high, targets, gains, sums.get(),
-                               flags);
+                               ctx->stream, c->high_count, chunks.start.get(), c->high, labels, targets, gains,
+                               sums.get(), flags);
         }
         GPART_LAUNCH_CHECK();
         const double nd = static_cast<double>(g->n), m = static_cast<double>(g->m);
@@ -1449,30 +1827,38 @@ struct Ops {
     // from the round's mover entries, between atomic updates (two per mover entry)
     // and a full rebuild of the cache after the commit (one gather per entry, no
     // atomics, same cache); the cut delta is summed from the movers' entries
-    // either way.
+    // either way. Ends with the round's status: published by the update launch where
+    // that is the round's last, else by a launch of its own.
     static void apply(gpart_ctx* ctx, RoundRun& run, const gpart_csr_view* g, const gpart_degree_classes* c,
                       RoundState* st, const std::int32_t* light, const std::int32_t* heavy, std::int32_t* labels,
                       const std::int32_t* targets, const std::int32_t* flags, int k, C* cache,
-                      unsigned long long* part_weights, std::int32_t* locks, bool lp) {
+                      unsigned long long* part_weights, std::int32_t* locks) {
         const std::int64_t n = g->n;
         const auto* off = static_cast<const O*>(g->offsets);
         const auto* w = static_cast<const W*>(g->edge_weights);
+        const auto* vw = static_cast<const W*>(g->vertex_weights);
         const long long rebuild_above = rebuild_threshold(ctx, g);
-        const auto light_blocks = static_cast<unsigned>(std::min<std::int64_t>(grid_for(n * 8), 4 * kRoundBlocks));
-        run.phase(GPART_PROFILE_CACHE_UPDATE, [&] {
-        profile_begin(ctx, GPART_PROFILE_CACHE_UPDATE);
         // levels whose degrees stay at most kWaveHeavyMaxDegree update their heavy
         // movers a wave each, in the same launch
         const bool wave_heavy = c->max_degree > kHeavyDegree && c->max_degree <= kWaveHeavyMaxDegree;
+        const bool tiles = c->max_degree > kWaveHeavyMaxDegree;
+        const bool ends_round = !tiles && rebuild_above < 0;
+        auto* status = reinterpret_cast<unsigned long long*>(ctx->status_device);
         const std::int64_t heavy_bound = c->medium_count + c->high_count;
+        // a launch that ends the round keeps the arrivals at its counter few
+        const std::int64_t cap = ends_round ? kRoundBlocks : 4 * kRoundBlocks;
+        const auto light_blocks = static_cast<unsigned>(std::min<std::int64_t>(grid_for(n * 8), cap));
         const unsigned heavy_blocks =
-            wave_heavy ? static_cast<unsigned>(std::max<std::int64_t>(
-                             1, std::min<std::int64_t>(grid_for(heavy_bound * kWave), 4 * kRoundBlocks)))
+            wave_heavy ? static_cast<unsigned>(
+                             std::max<std::int64_t>(1, std::min<std::int64_t>(grid_for(heavy_bound * kWave), cap)))
                        : 0;
+        run.phase(GPART_PROFILE_CACHE_UPDATE, [&] {
+        profile_begin(ctx, GPART_PROFILE_CACHE_UPDATE);
         hipLaunchKernelGGL((update_cache_kernel<O, W, C>), dim3(light_blocks + heavy_blocks), dim3(kBlock), 0,
-                           ctx->stream, st, light, wave_heavy ? heavy : nullptr, light_blocks, off, g->neighbors, w,
-                           labels, targets, flags, k, cache, &st->delta, rebuild_above);
-        if (!wave_heavy && c->max_degree > kHeavyDegree) {
+                           ctx->stream, st, light, heavy, light_blocks, heavy_blocks, off, g->neighbors, w, vw,
+                           labels, targets, flags, locks, k, cache, part_weights, rebuild_above,
+                           ends_round ? status : nullptr, ctx->status_counter);
+        if (tiles) {
             Scratch<long long> heavy_start(ctx, heavy_bound + 1);
             Scratch<std::int32_t> tile_mover(ctx, tile_count(g->m) + 1);
             device_scan<long long, SumOp<long long>>(ctx, HeavyDegreeLoad<O>{st, heavy, off},
@@ -1481,22 +1867,22 @@ struct Ops {
             hipLaunchKernelGGL(heavy_tiles_kernel,
                                dim3(static_cast<unsigned>(std::min<std::int64_t>(grid_for(heavy_bound), kRoundBlocks))),
                                dim3(kBlock), 0, ctx->stream, st, heavy_start.get(), tile_mover.get());
-            const auto tiles = static_cast<unsigned>(std::max<std::int64_t>(
+            const auto blocks = static_cast<unsigned>(std::max<std::int64_t>(
                 1, std::min<std::int64_t>(tile_count(g->m), 2 * kRoundBlocks)));
-            hipLaunchKernelGGL((update_cache_tiles_kernel<O, W, C>), dim3(tiles), dim3(kTileLanes), 0, ctx->stream,
+            hipLaunchKernelGGL((update_cache_tiles_kernel<O, W, C>), dim3(blocks), dim3(kTileLanes), 0, ctx->stream,
                                st, heavy_start.get(), tile_mover.get(), heavy, off, g->neighbors, w, labels, targets,
                                flags, k, cache, &st->delta, rebuild_above);
         }
+        GPART_LAUNCH_CHECK();
         profile_end(ctx, GPART_PROFILE_CACHE_UPDATE, 0.0);
         });
+        if (ends_round) return;
         run.phase(-1, [&] {
-            hipLaunchKernelGGL(commit_kernel<W>,
-                               dim3(static_cast<unsigned>(std::min<std::int64_t>(grid_for(n), kRoundBlocks))),
-                               dim3(kBlock), 0, ctx->stream, st, light, heavy, labels, targets,
-                               static_cast<const W*>(g->vertex_weights), part_weights, locks, lp, k);
-            GPART_LAUNCH_CHECK();
             if (rebuild_above >= 0)
                 build_cache(ctx, g, c, labels, k, cache, &st->edges, rebuild_above, &st->cut_directed);
+            hipLaunchKernelGGL(round_status_kernel, dim3(1), dim3(kWave), 0, ctx->stream, st, part_weights, k, status,
+                               ctx->status_counter);
+            GPART_LAUNCH_CHECK();
         });
     }
 
@@ -1505,15 +1891,9 @@ struct Ops {
         return ctx->rebuild_share > 0 && g->m >= ctx->rebuild_min_entries ? g->m / ctx->rebuild_share : -1;
     }
 
-    // The round's status into the fine-grained status words (the last phase), then
-    // the host's wait and reading of it.
-    static void finish(gpart_ctx* ctx, RoundRun& run, const gpart_csr_view* g, RoundState* st,
-                       const unsigned long long* part_weights, int k, gpart_refine_status* out) {
-        run.phase(-1, [&] {
-            hipLaunchKernelGGL(round_status_kernel, dim3(1), dim3(kWave), 0, ctx->stream, st, part_weights, k,
-                               reinterpret_cast<unsigned long long*>(ctx->status_device), ctx->status_counter);
-            GPART_LAUNCH_CHECK();
-        });
+    // The host's wait for the status that apply's last launch publishes, and its
+    // reading.
+    static void finish(gpart_ctx* ctx, RoundRun& run, const gpart_csr_view* g, int k, gpart_refine_status* out) {
         run.end();
         const std::uint64_t seq = ++ctx->status_seq;
         wait_status(ctx, seq);
@@ -1567,14 +1947,22 @@ struct Ops {
             GPART_LAUNCH_CHECK();
             profile_end(ctx, GPART_PROFILE_REFINE_PROPOSALS, static_cast<double>(n) * (20.0 + sizeof(C) * k));
         });
-        run.phase(GPART_PROFILE_REFINE_FILTER, [&] { filter_movers(ctx, g, c, labels, targets, gains, flags); });
-        run.phase(-1, [&] {
-            device_scan<MoverPair, MoverPairOp>(ctx, MoverLoad<O>{flags, off},
-                                                MoverStore{light.get(), heavy.get(), n, st.get()}, n, MoverPairOp{});
+        // Small levels list their movers in the filter launch; on large ones its
+        // thousands of workgroups would contend for the list counters (128^3 mesh
+        // uncoarsening 43 -> 49 ms), so their movers come from a scan of the flags.
+        const bool append = n <= kSelectVertices && c->max_degree <= kHubChunk;
+        run.phase(GPART_PROFILE_REFINE_FILTER, [&] {
+            filter_movers(ctx, g, c, labels, targets, gains, flags, append, light.get(), heavy.get(), st.get());
         });
+        if (!append)
+            run.phase(-1, [&] {
+                device_scan<MoverPair, MoverPairOp>(ctx, MoverLoad<O>{flags, off},
+                                                    MoverStore{light.get(), heavy.get(), n, st.get()}, n,
+                                                    MoverPairOp{});
+            });
         apply(ctx, run, g, c, st.get(), light.get(), heavy.get(), labels, targets, flags, k, cache, part_weights,
-              locks, true);
-        finish(ctx, run, g, st.get(), part_weights, k, out);
+              locks);
+        finish(ctx, run, g, k, out);
     }
 
     // Everything a round's launches depend on besides its own scratch.
@@ -1598,16 +1986,75 @@ struct Ops {
         return key;
     }
 
+    // A rebalance iteration of a small level (balance_vertices_kernel,
+    // balance_select_kernel, update).
+    static void rebalance_round_small(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
+                                      C* cache, std::int32_t* labels, int k, unsigned long long* part_weights,
+                                      std::uint64_t capacity, std::int32_t* targets, std::int32_t* flags,
+                                      const PowerTable& powers, gpart_refine_status* out) {
+        const std::int64_t n = g->n;
+        const auto* off = static_cast<const O*>(g->offsets);
+        const auto* vw = static_cast<const W*>(g->vertex_weights);
+        RoundRun run(ctx, round_plan(ctx, n, round_key(ctx, g, c, cache, labels, k, targets, flags, part_weights,
+                                                       {2, capacity})));
+        Scratch<RoundState> st(ctx, 1);
+        Scratch<std::int32_t> choices(ctx, n), light(ctx, n), heavy(ctx, n);
+        const int G = group_for_k(k);
+        run.phase(GPART_PROFILE_REBALANCE, [&] {
+            profile_begin(ctx, GPART_PROFILE_REBALANCE);
+#define GPART_BALANCE_VERTICES(GG)                                                                                 \
+    hipLaunchKernelGGL((balance_vertices_kernel<W, GG, C>), dim3(grid_for(n * GG)), dim3(kBlock), 0, ctx->stream, \
+                       st.get(), n, cache, labels, vw, k, part_weights, capacity, powers, targets, choices.get(), flags)
+            switch (G) {
+                case 1: GPART_BALANCE_VERTICES(1); break;
+                case 2: GPART_BALANCE_VERTICES(2); break;
+                default: GPART_BALANCE_VERTICES(4); break;
+            }
+#undef GPART_BALANCE_VERTICES
+            GPART_LAUNCH_CHECK();
+            profile_end(ctx, GPART_PROFILE_REBALANCE, 0.0);
+        });
+        run.phase(-1, [&] {
+#define GPART_BALANCE_SELECT(ITEMS)                                                                              \
+    hipLaunchKernelGGL((balance_select_kernel<O, W, ITEMS>), dim3(1), dim3(kSelectThreads), 0, ctx->stream,      \
+                       st.get(), n, choices.get(), vw, off, k, part_weights, capacity, light.get(), heavy.get(), \
+                       flags)
+            if (n <= kSelectThreads) GPART_BALANCE_SELECT(1);
+            else if (n <= 4 * kSelectThreads) GPART_BALANCE_SELECT(4);
+            else GPART_BALANCE_SELECT(kSelectMaxItems);
+#undef GPART_BALANCE_SELECT
+            GPART_LAUNCH_CHECK();
+        });
+        apply(ctx, run, g, c, st.get(), light.get(), heavy.get(), labels, targets, flags, k, cache, part_weights,
+              nullptr);
+        finish(ctx, run, g, k, out);
+    }
+
     // One rebalance iteration: proposals, source and destination bucket quotas,
     // apply; one synchronisation.
     static void rebalance_round(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
                                 C* cache, std::int32_t* labels, int k,
                                 unsigned long long* part_weights, std::uint64_t capacity, std::int32_t* targets,
                                 std::int32_t* flags, gpart_refine_status* out) {
+        static const PowerTable powers = make_power_table();
+        if (g->n <= kSelectVertices)
+            rebalance_round_small(ctx, g, c, cache, labels, k, part_weights, capacity, targets, flags, powers, out);
+        else
+            rebalance_round_large(ctx, g, c, cache, labels, k, part_weights, capacity, targets, flags, powers, out);
+        // per candidate: id, label, weight, cache row, target and bucket writes
+        profile_add_bytes(ctx, GPART_PROFILE_REBALANCE,
+                          static_cast<double>(out->candidates) * (16.0 + sizeof(W) + sizeof(C) * k));
+        // one bucket-histogram add per candidate (balance_source_histogram, :173-186)
+        profile_add_units(ctx, GPART_PROFILE_REBALANCE, static_cast<double>(out->candidates));
+    }
+
+    static void rebalance_round_large(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
+                                      C* cache, std::int32_t* labels, int k, unsigned long long* part_weights,
+                                      std::uint64_t capacity, std::int32_t* targets, std::int32_t* flags,
+                                      const PowerTable& powers, gpart_refine_status* out) {
         const std::int64_t n = g->n;
         const auto* off = static_cast<const O*>(g->offsets);
         const auto* vw = static_cast<const W*>(g->vertex_weights);
-        static const PowerTable powers = make_power_table();
         const std::int64_t width = static_cast<std::int64_t>(k) * kBalanceWidth;
         // Both replica arrays live in the context between rounds and are zero at rest
         // (the bucket scans clear what they read); the proposals kernel zeroes the
@@ -1681,24 +2128,19 @@ struct Ops {
                            dst_counts, dst_offsets, part_weights, capacity, true, dst_thresholds);
         hipLaunchKernelGGL((balance_destinations_kernel<O, W>), dim3(slices), dim3(kBlock), 0, ctx->stream,
                            st_ptr, cand.get(), dbucket.get(), vw, off, dst_counts, dst_offsets, dst_thresholds,
-                           sums.get(), light.get(), heavy.get(), flags);
+                           sums.get(), labels, light.get(), heavy.get(), flags);
         if (!inline_columns)
             hipLaunchKernelGGL(column_scan_kernel, dim3(k), dim3(kBucketScanThreads), 0, ctx->stream, sums.get(),
                                slices, prefix.get());
         hipLaunchKernelGGL((balance_destination_ranks_kernel<O, W>), dim3(slices), dim3(kBlock), 0, ctx->stream,
                            st_ptr, cand.get(), dbucket.get(), vw, off, dst_offsets, dst_thresholds, column_prefix,
-                           sums.get(), light.get(), heavy.get(), flags);
+                           sums.get(), labels, light.get(), heavy.get(), flags);
         GPART_LAUNCH_CHECK();
         });
         apply(ctx, run, g, c, st_ptr, light.get(), heavy.get(), labels, targets, flags, k, cache, part_weights,
-              nullptr, false);
-        finish(ctx, run, g, st_ptr, part_weights, k, out);
+              nullptr);
+        finish(ctx, run, g, k, out);
         ctx->rebalance_counters_zero = true;
-        // per candidate: id, label, weight, cache row, target and bucket writes
-        profile_add_bytes(ctx, GPART_PROFILE_REBALANCE,
-                          static_cast<double>(out->candidates) * (16.0 + sizeof(W) + sizeof(C) * k));
-        // one bucket-histogram add per candidate (balance_source_histogram, :173-186)
-        profile_add_units(ctx, GPART_PROFILE_REBALANCE, static_cast<double>(out->candidates));
     }
 };
 
