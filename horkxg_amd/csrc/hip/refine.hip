@@ -20,6 +20,7 @@
 #include "tiles.hpp"
 #include "hubs.hpp"
 #include "refine_device.hpp"
+#include "refine_rows.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -248,7 +249,8 @@ template <int G, typename C>
 __global__ void __launch_bounds__(kBlock) lp_proposals_kernel(std::int64_t n, const C* cache,
                                                               const std::int32_t* labels, int k, double filter,
                                                               std::int32_t* locks, std::int32_t* targets,
-                                                              long long* gains, RoundState* st) {
+                                                              long long* gains, unsigned char* state,
+                                                              RoundState* st) {
     // the round's state starts at zero (the filter appends the movers to it)
     if (blockIdx.x == 0 && threadIdx.x < sizeof(RoundState) / 8)
         reinterpret_cast<unsigned long long*>(st)[threadIdx.x] = 0;
@@ -283,6 +285,7 @@ __global__ void __launch_bounds__(kBlock) lp_proposals_kernel(std::int64_t n, co
         current = oc > current ? oc : current;  // only the source's lane holds it
     }
     if (j != 0) return;
+    if (state) state[v] = static_cast<unsigned char>(source);  // refine_rows.hpp
     if (locks[v] != 0) {
         locks[v] = 0;
         targets[v] = -1;
@@ -349,8 +352,8 @@ __device__ __forceinline__ bool priority_filter_rows(std::int64_t count, const s
                                                      const O* offsets, const std::int32_t* neighbors,
                                                      const W* weights, const std::int32_t* labels,
                                                      const std::int32_t* targets, const long long* gains,
-                                                     std::int32_t* flags, long long* block_sum,
-                                                     std::int32_t* vertex) {
+                                                     std::int32_t* flags, unsigned char* state,
+                                                     long long* block_sum, std::int32_t* vertex) {
     const std::int64_t group = (block * blockDim.x + threadIdx.x) / G;
     const int sub = threadIdx.x & (G - 1);
     const bool active = group < count;
@@ -369,6 +372,7 @@ __device__ __forceinline__ bool priority_filter_rows(std::int64_t count, const s
         if (active && sub == 0) {
             take = target >= 0 && gains[v] + correction >= 0;
             flags[v] = take ? labels[v] + 1 : 0;
+            if (take) mark_mover(state, v, target);
         }
     } else {
         correction = group_sum_i64<kWave>(correction);
@@ -379,6 +383,7 @@ __device__ __forceinline__ bool priority_filter_rows(std::int64_t count, const s
             for (int w = 0; w < kBlock / kWave; ++w) total += block_sum[w];
             take = target >= 0 && gains[v] + total >= 0;
             flags[v] = take ? labels[v] + 1 : 0;
+            if (take) mark_mover(state, v, target);
         }
     }
     *vertex = v;
@@ -395,21 +400,22 @@ __global__ void __launch_bounds__(kBlock) priority_filter_kernel(
     std::int64_t low_count, const std::int32_t* low, unsigned low_blocks, std::int64_t medium_count,
     const std::int32_t* medium, unsigned medium_blocks, std::int64_t high_count, const std::int32_t* high,
     const O* offsets, const std::int32_t* neighbors, const W* weights, const std::int32_t* labels,
-    const std::int32_t* targets, const long long* gains, std::int32_t* flags, std::int32_t* light,
-    std::int32_t* heavy, RoundState* st) {
+    const std::int32_t* targets, const long long* gains, std::int32_t* flags, unsigned char* state,
+    std::int32_t* light, std::int32_t* heavy, RoundState* st) {
     __shared__ long long block_sum[kBlock / kWave];
     const long long b = blockIdx.x;
     bool take;
     std::int32_t v = 0;
     if (b < low_blocks)
         take = priority_filter_rows<O, W, 8>(low_count, low, b, offsets, neighbors, weights, labels, targets, gains,
-                                             flags, block_sum, &v);
+                                             flags, state, block_sum, &v);
     else if (b < low_blocks + medium_blocks)
         take = priority_filter_rows<O, W, 64>(medium_count, medium, b - low_blocks, offsets, neighbors, weights,
-                                              labels, targets, gains, flags, block_sum, &v);
+                                              labels, targets, gains, flags, state, block_sum, &v);
     else
         take = priority_filter_rows<O, W, kBlock>(high_count, high, b - low_blocks - medium_blocks, offsets,
-                                                  neighbors, weights, labels, targets, gains, flags, block_sum, &v);
+                                                  neighbors, weights, labels, targets, gains, flags, state, block_sum,
+                                                  &v);
     if constexpr (Append) {
         __shared__ unsigned counts[2 * (kBlock / kWave)];
         __shared__ unsigned long long base[2];
@@ -454,11 +460,13 @@ __global__ void __launch_bounds__(kBlock) priority_filter_hub_kernel(const std::
 __global__ void priority_filter_hub_finish_kernel(std::int64_t count, const std::int64_t* chunk_start,
                                                   const std::int32_t* list, const std::int32_t* labels,
                                                   const std::int32_t* targets, const long long* gains,
-                                                  long long* sums, std::int32_t* flags) {
+                                                  long long* sums, std::int32_t* flags, unsigned char* state) {
     const std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= count || chunk_start[i] == chunk_start[i + 1]) return;
     const std::int32_t v = list[i];
-    flags[v] = targets[v] >= 0 && gains[v] + sums[i] >= 0 ? labels[v] + 1 : 0;
+    const bool take = targets[v] >= 0 && gains[v] + sums[i] >= 0;
+    flags[v] = take ? labels[v] + 1 : 0;
+    if (take) mark_mover(state, v, targets[v]);
     sums[i] = 0;
 }
 
@@ -656,6 +664,108 @@ __global__ void __launch_bounds__(kBlock) update_cache_kernel(
     }
 }
 
+// The end of a round without an incremental cache (refine_rows.hpp): commits, part
+// weights, the cut change and the status (as update_cache_kernel publishes it), in one
+// launch. A workgroup takes every gridDim-th heavy mover and spreads their entries over
+// its waves in segments of kGainSegment: the cut change is a plain sum, so a long row
+// need not stay with one wave. The light movers take 8 lanes each. Hub rows of the
+// cache are cleared on the way.
+constexpr int kGainSegment = 4 * kWave;
+template <typename O, typename W, int Form>
+__global__ void __launch_bounds__(kRowsThreads) gain_commit_kernel(
+    RoundState* st, const std::int32_t* light, const std::int32_t* heavy, RowLists lists, const unsigned char* states,
+    std::int64_t n, const O* offsets, const std::int32_t* neighbors, const W* weights, const W* vertex_weights,
+    std::int32_t* labels, const std::int32_t* targets, const std::int32_t* flags, std::int32_t* locks, int k,
+    unsigned* cache, unsigned long long* part_weights, unsigned long long* status, unsigned long long* counter) {
+    extern __shared__ unsigned lds[];
+    __shared__ long long wave_gain[kRowsWaves];
+    __shared__ PartMoves moves;
+    __shared__ int last;
+    __shared__ unsigned wave_segments[kRowsWaves];
+    __shared__ unsigned first_segment[kRowsThreads];  // of a pass's movers
+    __shared__ std::int32_t mover[kRowsThreads];
+    stage_states<Form>(states, n, lds);
+    moves.clear();  // its barrier also completes the states
+    const States<Form> state{lds, states};
+    const int t = threadIdx.x, lane = lane_id(), wave_in = t / kWave;
+    const std::int64_t groups = gridDim.x, heavies = st->heavy, lights = st->light;
+    long long gain = 0;
+    for (std::int64_t base = blockIdx.x; base < heavies; base += groups * kRowsThreads) {
+        const std::int64_t i = base + t * groups;
+        unsigned segments = 0;
+        std::int32_t v = 0;
+        if (i < heavies) {
+            v = heavy[i];
+            segments = static_cast<unsigned>((offsets[v + 1] - offsets[v] + kGainSegment - 1) / kGainSegment);
+            commit_mover(v, flags[v] - 1, targets[v], vertex_weights, labels, locks, moves);
+        }
+        const unsigned inclusive = wave_scan(segments);
+        if (lane == kWave - 1) wave_segments[wave_in] = inclusive;
+        __syncthreads();
+        unsigned before = 0, all = 0;
+        for (int w = 0; w < kRowsWaves; ++w) {
+            if (w == wave_in) before = all;
+            all += wave_segments[w];
+        }
+        first_segment[t] = before + inclusive - segments;
+        mover[t] = v;
+        __syncthreads();
+        // the last mover whose first segment is not behind s owns segment s
+        for (unsigned s = static_cast<unsigned>(wave_in); s < all; s += kRowsWaves) {
+            int lo = 0;
+#pragma unroll
+            for (int step = kRowsThreads / 2; step > 0; step /= 2)
+                if (first_segment[lo + step] <= s) lo += step;
+            const std::int32_t x = mover[lo];
+            const std::int64_t begin = static_cast<std::int64_t>(offsets[x]) +
+                                       static_cast<std::int64_t>(s - first_segment[lo]) * kGainSegment;
+            const auto row_end = static_cast<std::int64_t>(offsets[x + 1]);
+            const std::int64_t end = begin + kGainSegment < row_end ? begin + kGainSegment : row_end;
+            gain += mover_gain<kWave, kGainSegment / kWave>(x, flags[x] - 1, state.part(x), begin, end, lane, neighbors,
+                                                            weights, state, flags);
+        }
+        __syncthreads();
+    }
+    for (std::int64_t i = blockIdx.x + (t / 8) * groups; i < lights; i += groups * (kRowsThreads / 8)) {
+        const std::int32_t v = light[i], source = flags[v] - 1, target = targets[v];
+        if ((t & 7) == 0) commit_mover(v, source, target, vertex_weights, labels, locks, moves);
+        gain += mover_gain<8, 4>(v, source, target, static_cast<std::int64_t>(offsets[v]),
+                                 static_cast<std::int64_t>(offsets[v + 1]), t & 7, neighbors, weights, state, flags);
+    }
+    if (lists.chunk_total) {
+        const std::int64_t chunks = *lists.chunk_total;
+        for (std::int64_t c = static_cast<std::int64_t>(blockIdx.x) * kRowsWaves + wave_in; c < chunks;
+             c += groups * kRowsWaves) {
+            const std::int32_t i = lists.chunk_hub[c];
+            if (c == lists.chunk_start[i] && lane < k) cache[static_cast<std::int64_t>(lists.high[i]) * k + lane] = 0;
+        }
+    }
+    gain = group_sum_i64<kWave>(gain);
+    if (lane == 0) wave_gain[wave_in] = gain;
+    __syncthreads();  // also completes the LDS sums of the part weights
+    if (t == 0) {
+        long long total = 0;
+        for (int w = 0; w < kRowsWaves; ++w) total += wave_gain[w];
+        if (total) atomicAdd(reinterpret_cast<unsigned long long*>(&st->delta), static_cast<unsigned long long>(total));
+    }
+    moves.flush(k, part_weights);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (t == 0) {
+        const unsigned long long arrived = __hip_atomic_fetch_add(&st->arrivals, 1ULL, __ATOMIC_RELAXED,
+                                                                  __HIP_MEMORY_SCOPE_AGENT);
+        last = arrived + 1 == gridDim.x;
+    }
+    __syncthreads();
+    if (last && t < kWave) {
+        auto load = [](const unsigned long long* p) {
+            return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        const auto delta = static_cast<long long>(load(reinterpret_cast<const unsigned long long*>(&st->delta)));
+        publish_status(st, [&](int p) { return load(part_weights + p); }, delta, k, status, counter);
+    }
+}
+
 // Heavy movers (degree > kHeavyDegree) as one flattened entry range: heavy_start
 // holds the exclusive prefix of their degrees (count + 1 entries, the last one
 // the total), tiled as in tiles.hpp with the movers as rows.
@@ -796,10 +906,13 @@ struct OverloadedLoad {
 struct CandidateStore {
     std::int32_t* candidates;
     std::int32_t* flags;
+    const std::int32_t* labels;
+    unsigned char* state;  // refine_rows.hpp, or null
     std::int64_t n;
     RoundState* st;
     __device__ __forceinline__ void operator()(std::int64_t v, int prefix, int item) const {
         flags[v] = 0;
+        if (state) state[v] = static_cast<unsigned char>(labels[v]);
         if (item) candidates[prefix] = static_cast<std::int32_t>(v);
         if (v == n - 1) st->candidates = prefix + item;
     }
@@ -964,7 +1077,7 @@ __global__ void __launch_bounds__(kBlock) balance_vertices_kernel(RoundState* st
                                                                   int k, const unsigned long long* part_weights,
                                                                   std::uint64_t capacity, PowerTable powers,
                                                                   std::int32_t* targets, std::int32_t* choices,
-                                                                  std::int32_t* flags) {
+                                                                  std::int32_t* flags, unsigned char* state) {
     __shared__ unsigned long long pw[32];
     if (blockIdx.x == 0 && threadIdx.x < sizeof(RoundState) / 8)
         reinterpret_cast<unsigned long long*>(st)[threadIdx.x] = 0;
@@ -984,6 +1097,7 @@ __global__ void __launch_bounds__(kBlock) balance_vertices_kernel(RoundState* st
                                        : choice.bucket - source * kBalanceWidth + (source << kSourceShift) +
                                              (choice.target << kTargetShift);
         flags[v] = 0;
+        if (state) state[v] = static_cast<unsigned char>(source);  // refine_rows.hpp
     }
 }
 
@@ -1038,7 +1152,7 @@ template <typename O, typename W, int Items>
 __global__ void __launch_bounds__(kSelectThreads) balance_select_kernel(
     RoundState* st, std::int64_t n, const std::int32_t* choices, const W* vertex_weights, const O* offsets, int k,
     const unsigned long long* part_weights, std::uint64_t capacity, std::int32_t* light, std::int32_t* heavy,
-    std::int32_t* flags) {
+    std::int32_t* flags, unsigned char* state) {
     __shared__ SelectShared sh;
     const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
     const int first = wave * kWave * Items + lane;
@@ -1201,6 +1315,7 @@ __global__ void __launch_bounds__(kSelectThreads) balance_select_kernel(
             at += 1;
         }
         flags[v] = (item[i] >> kSourceShift & 31) + 1;
+        mark_mover(state, v, item[i] >> kTargetShift & 31);
     }
     if (t == 0) {
         st->light = static_cast<long long>(listed & 0xfffffU);
@@ -1413,7 +1528,7 @@ __global__ void __launch_bounds__(kBlock) balance_destinations_kernel(
     RoundState* st, const std::int32_t* cand, std::int32_t* dbucket, const W* vertex_weights, const O* offsets_csr,
     const unsigned long long* counts, const unsigned long long* offsets, const unsigned long long* thresholds,
     unsigned long long* block_sums, const std::int32_t* labels, std::int32_t* light, std::int32_t* heavy,
-    std::int32_t* flags) {
+    std::int32_t* flags, unsigned char* state) {
     __shared__ unsigned long long sums[32];
     __shared__ unsigned counts_lds[2 * (kBlock / kWave)];
     __shared__ unsigned long long base_lds[2];
@@ -1434,6 +1549,7 @@ __global__ void __launch_bounds__(kBlock) balance_destinations_kernel(
                 if (side == kTaken) {
                     take = true;
                     flags[v] = labels[v] + 1;
+                    mark_mover(state, v, part);
                 } else if (side == kBoundary) {
                     dbucket[i] = -3 - d;
                     atomicAdd(&sums[part], static_cast<unsigned long long>(vertex_weights[v]));
@@ -1451,7 +1567,7 @@ __global__ void __launch_bounds__(kBlock) balance_destination_ranks_kernel(
     RoundState* st, const std::int32_t* cand, const std::int32_t* dbucket, const W* vertex_weights,
     const O* offsets_csr, const unsigned long long* offsets, const unsigned long long* thresholds,
     const unsigned long long* column_prefix, const unsigned long long* block_sums, const std::int32_t* labels,
-    std::int32_t* light, std::int32_t* heavy, std::int32_t* flags) {
+    std::int32_t* light, std::int32_t* heavy, std::int32_t* flags, unsigned char* state) {
     __shared__ unsigned long long wave_total[kBlock / kWave][32];
     __shared__ unsigned long long running[32];
     __shared__ unsigned long long groups[kBlock / 32][32];
@@ -1477,7 +1593,10 @@ __global__ void __launch_bounds__(kBlock) balance_destination_ranks_kernel(
         }
         const unsigned long long rank = block_key_prefix<kBlock>(pending, part, w, wave_total, running);
         const bool take = pending && offsets[d] + rank + w <= thresholds[part];
-        if (take) flags[v] = labels[v] + 1;
+        if (take) {
+            flags[v] = labels[v] + 1;
+            mark_mover(state, v, part);
+        }
         append_movers(take, v, offsets_csr, light, heavy, st, counts_lds, base_lds);
     }
 }
@@ -1788,26 +1907,28 @@ struct Ops {
     static void filter_movers(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
                               const std::int32_t* labels, const std::int32_t* targets, const long long* gains,
                               std::int32_t* flags, bool append, std::int32_t* light, std::int32_t* heavy,
-                              RoundState* st) {
+                              RoundState* st, const gpart_refine_rows* rows) {
         const auto* off = static_cast<const O*>(g->offsets);
         const auto* w = static_cast<const W*>(g->edge_weights);
         profile_begin(ctx, GPART_PROFILE_REFINE_FILTER);
         const unsigned low_blocks = grid_for(c->low_count * 8), medium_blocks = grid_for(c->medium_count * 64);
         const auto high_blocks = static_cast<unsigned>(c->high_count);
         const unsigned blocks = low_blocks + medium_blocks + high_blocks;
+        unsigned char* state = rows ? rows->states.get() : nullptr;
         if (blocks > 0 && append)
             hipLaunchKernelGGL((priority_filter_kernel<O, W, true>), dim3(blocks), dim3(kBlock), 0, ctx->stream,
                                c->low_count, c->low, low_blocks, c->medium_count, c->medium, medium_blocks,
-                               c->high_count, c->high, off, g->neighbors, w, labels, targets, gains, flags, light,
+                               c->high_count, c->high, off, g->neighbors, w, labels, targets, gains, flags, state, light,
                                heavy, st);
         else if (blocks > 0)
             hipLaunchKernelGGL((priority_filter_kernel<O, W, false>), dim3(blocks), dim3(kBlock), 0, ctx->stream,
                                c->low_count, c->low, low_blocks, c->medium_count, c->medium, medium_blocks,
-                               c->high_count, c->high, off, g->neighbors, w, labels, targets, gains, flags, light,
+                               c->high_count, c->high, off, g->neighbors, w, labels, targets, gains, flags, state, light,
                                heavy, st);
         if (c->max_degree > kHubChunk) {
-            HubChunks chunks;
-            build_hub_chunks(ctx, off, c->high, c->high_count, c->high_edges, kHubChunk, chunks);
+            HubChunks own;
+            if (!rows) build_hub_chunks(ctx, off, c->high, c->high_count, c->high_edges, kHubChunk, own);
+            const HubChunks& chunks = rows ? rows->chunks : own;
             Scratch<long long> sums(ctx, c->high_count);
             fill_bytes(ctx, sums.get(), 0, static_cast<std::size_t>(c->high_count) * 8);
             hipLaunchKernelGGL((priority_filter_hub_kernel<O, W>), dim3(chunks.grid()), dim3(kBlock), 0, ctx->stream,
@@ -1815,11 +1936,97 @@ struct Ops {
                                labels, targets, gains, sums.get());
             hipLaunchKernelGGL(priority_filter_hub_finish_kernel, dim3(grid_for(c->high_count)), dim3(kBlock), 0,
                                ctx->stream, c->high_count, chunks.start.get(), c->high, labels, targets, gains,
-                               sums.get(), flags);
+                               sums.get(), flags, state);
         }
         GPART_LAUNCH_CHECK();
         const double nd = static_cast<double>(g->n), m = static_cast<double>(g->m);
         profile_end(ctx, GPART_PROFILE_REFINE_FILTER, (nd + 1) * sizeof(O) + m * (4 + sizeof(W)) + 16 * m + 20 * nd);
+    }
+
+    static RowLists row_lists(const gpart_degree_classes* c, const gpart_refine_rows* r) {
+        RowLists l{};
+        l.low = c->low;
+        l.medium = c->medium;
+        l.high = c->high;
+        l.low_count = c->low_count;
+        l.medium_count = c->medium_count;
+        l.high_count = c->high_count;
+        if (r->hubs) {
+            l.chunk_total = r->chunks.total();
+            l.chunk_start = r->chunks.start.get();
+            l.chunk_hub = r->chunks.hub.get();
+        }
+        return l;
+    }
+    // Workgroups of a pass over about `entries` entries: 256 entries a wave, at least
+    // a few workgroups so that a small level's rows spread over some CUs.
+    static unsigned rows_groups(std::int64_t entries, std::size_t lds) {
+        const std::int64_t per = std::int64_t{256} * kRowsWaves;
+        return static_cast<unsigned>(std::clamp<std::int64_t>((entries + per - 1) / per, 16,
+                                                              lds <= kRowsPairLds ? 2 * kRowsGroups : kRowsGroups));
+    }
+
+    // Before the first round of a level.
+    static void prepare_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
+                             gpart_refine_rows* r, const std::int32_t* labels, int k, C* cache) {
+        if constexpr (sizeof(C) == 4) {
+            if (r->ready) return;
+            hipLaunchKernelGGL(rows_prepare_kernel, dim3(std::min<unsigned>(grid_for(g->n), kRoundBlocks)), dim3(256), 0,
+                               ctx->stream, row_lists(c, r), g->n, labels, r->states.get(), k, cache);
+            GPART_LAUNCH_CHECK();
+            r->ready = true;
+        }
+    }
+
+    // The rows of every vertex, or (part_weights) of the parts above capacity.
+    static void rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
+                     const gpart_refine_rows* r, int k, C* cache, const unsigned long long* part_weights,
+                     std::uint64_t capacity) {
+        if constexpr (sizeof(C) == 4) {
+            profile_begin(ctx, GPART_PROFILE_REFINE_CACHE);
+            const std::size_t lds = kRowsWaveBytes + state_lds_bytes(g->n, r->form);
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(rows_groups(g->m, lds)), dim3(kRowsThreads), lds, ctx->stream,
+                                   row_lists(c, r), r->states.get(), g->n, static_cast<const O*>(g->offsets),
+                                   g->neighbors, static_cast<const W*>(g->edge_weights), k, cache, part_weights,
+                                   capacity);
+            };
+            if (r->form == kByteState) launch(rows_kernel<O, W, kByteState>);
+            else if (r->form == kNibbleState) launch(rows_kernel<O, W, kNibbleState>);
+            else launch(rows_kernel<O, W, kMemoryState>);
+            GPART_LAUNCH_CHECK();
+            const double n = static_cast<double>(g->n), m = static_cast<double>(g->m);
+            profile_end(ctx, GPART_PROFILE_REFINE_CACHE,
+                        part_weights ? 0.0 : (n + 1) * sizeof(O) + m * (4 + sizeof(W)) + n + 4 * n * k);
+        }
+    }
+
+    // gain_commit_kernel over the round's movers.
+    static void apply_rows(gpart_ctx* ctx, RoundRun& run, const gpart_csr_view* g, const gpart_degree_classes* c,
+                           const gpart_refine_rows* r, RoundState* st, const std::int32_t* light,
+                           const std::int32_t* heavy, std::int32_t* labels, const std::int32_t* targets,
+                           const std::int32_t* flags, int k, C* cache, unsigned long long* part_weights,
+                           std::int32_t* locks) {
+        if constexpr (sizeof(C) == 4) {
+            run.phase(GPART_PROFILE_CACHE_UPDATE, [&] {
+                profile_begin(ctx, GPART_PROFILE_CACHE_UPDATE);
+                const std::size_t lds = state_lds_bytes(g->n, r->form);
+                auto launch = [&](auto kernel) {
+                    // a tenth of the entries move in a round of a dense level
+                    hipLaunchKernelGGL(kernel, dim3(rows_groups(g->m / 8, lds)), dim3(kRowsThreads), lds, ctx->stream,
+                                       st, light, heavy, row_lists(c, r), r->states.get(), g->n, static_cast<const O*>(g->offsets), g->neighbors,
+                                       static_cast<const W*>(g->edge_weights),
+                                       static_cast<const W*>(g->vertex_weights), labels, targets, flags, locks, k,
+                                       cache, part_weights, reinterpret_cast<unsigned long long*>(ctx->status_device),
+                                       ctx->status_counter);
+                };
+                if (r->form == kByteState) launch(gain_commit_kernel<O, W, kByteState>);
+                else if (r->form == kNibbleState) launch(gain_commit_kernel<O, W, kNibbleState>);
+                else launch(gain_commit_kernel<O, W, kMemoryState>);
+                GPART_LAUNCH_CHECK();
+                profile_end(ctx, GPART_PROFILE_CACHE_UPDATE, 0.0);
+            });
+        }
     }
 
     // incremental_update_cache_and_cut + incremental_commit over the round's movers.
@@ -1893,7 +2100,8 @@ struct Ops {
 
     // The host's wait for the status that apply's last launch publishes, and its
     // reading.
-    static void finish(gpart_ctx* ctx, RoundRun& run, const gpart_csr_view* g, int k, gpart_refine_status* out) {
+    static void finish(gpart_ctx* ctx, RoundRun& run, const gpart_csr_view* g, int k, bool rows_form,
+                       gpart_refine_status* out) {
         run.end();
         const std::uint64_t seq = ++ctx->status_seq;
         wait_status(ctx, seq);
@@ -1905,10 +2113,16 @@ struct Ops {
         out->max_part_weight = h.max_weight;
         for (int p = 0; p < 32; ++p) out->part_weights[p] = p < k ? h.pw[p] : 0;
         out->mover_entries = h.edges;
-        const long long rebuild_above = rebuild_threshold(ctx, g);
+        const long long rebuild_above = rows_form ? -1 : rebuild_threshold(ctx, g);
         out->rebuilt = rebuild_above >= 0 && h.edges > rebuild_above ? 1 : 0;
         out->cut_after = 0;
-        if (!out->rebuilt) {
+        if (rows_form) {
+            // the movers' rows and ids, per entry a neighbour, a weight and the label,
+            // target and flag gathers
+            profile_add_bytes(ctx, GPART_PROFILE_CACHE_UPDATE,
+                              static_cast<double>(out->movers) * (2.0 * sizeof(O) + 16.0) +
+                                  static_cast<double>(h.edges) * (4.0 + sizeof(W) + 12.0));
+        } else if (!out->rebuilt) {
             // the movers' rows and ids, per entry a neighbour, a weight, two cache
             // atomics (read and write each) and the label, target and flag gathers
             const double movers = static_cast<double>(out->movers), entries = static_cast<double>(h.edges);
@@ -1927,22 +2141,24 @@ struct Ops {
     static void lp_round(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
                          C* cache, std::int32_t* labels, int k, double filter,
                          std::int32_t* locks, std::int32_t* targets, long long* gains, std::int32_t* flags,
-                         unsigned long long* part_weights, gpart_refine_status* out) {
+                         unsigned long long* part_weights, const gpart_refine_rows* r, gpart_refine_status* out) {
         const std::int64_t n = g->n;
         const auto* off = static_cast<const O*>(g->offsets);
-        RoundRun run(ctx, round_plan(ctx, n, round_key(ctx, g, c, cache, labels, k, targets, flags, part_weights,
+        RoundRun run(ctx, round_plan(ctx, n, round_key(ctx, g, c, cache, labels, k, targets, flags, part_weights, r,
                                                        {0, key_of(filter), key_of(locks), key_of(gains)})));
         // the proposals kernel zeroes the round state
         Scratch<RoundState> st(ctx, 1);
         Scratch<std::int32_t> light(ctx, n), heavy(ctx, n);
         const int G = group_for_k(k);
+        unsigned char* state = r ? r->states.get() : nullptr;
+        if (r) run.phase(GPART_PROFILE_REFINE_CACHE, [&] { rows(ctx, g, c, r, k, cache, nullptr, 0); });
         run.phase(GPART_PROFILE_REFINE_PROPOSALS, [&] {
             profile_begin(ctx, GPART_PROFILE_REFINE_PROPOSALS);
             const unsigned blocks = std::max<unsigned>(1, grid_for(n * G));
             switch (G) {
-                case 1: hipLaunchKernelGGL((lp_proposals_kernel<1, C>), dim3(blocks), dim3(kBlock), 0, ctx->stream, n, cache, labels, k, filter, locks, targets, gains, st.get()); break;
-                case 2: hipLaunchKernelGGL((lp_proposals_kernel<2, C>), dim3(blocks), dim3(kBlock), 0, ctx->stream, n, cache, labels, k, filter, locks, targets, gains, st.get()); break;
-                default: hipLaunchKernelGGL((lp_proposals_kernel<4, C>), dim3(blocks), dim3(kBlock), 0, ctx->stream, n, cache, labels, k, filter, locks, targets, gains, st.get()); break;
+                case 1: hipLaunchKernelGGL((lp_proposals_kernel<1, C>), dim3(blocks), dim3(kBlock), 0, ctx->stream, n, cache, labels, k, filter, locks, targets, gains, state, st.get()); break;
+                case 2: hipLaunchKernelGGL((lp_proposals_kernel<2, C>), dim3(blocks), dim3(kBlock), 0, ctx->stream, n, cache, labels, k, filter, locks, targets, gains, state, st.get()); break;
+                default: hipLaunchKernelGGL((lp_proposals_kernel<4, C>), dim3(blocks), dim3(kBlock), 0, ctx->stream, n, cache, labels, k, filter, locks, targets, gains, state, st.get()); break;
             }
             GPART_LAUNCH_CHECK();
             profile_end(ctx, GPART_PROFILE_REFINE_PROPOSALS, static_cast<double>(n) * (20.0 + sizeof(C) * k));
@@ -1952,7 +2168,7 @@ struct Ops {
         // uncoarsening 43 -> 49 ms), so their movers come from a scan of the flags.
         const bool append = n <= kSelectVertices && c->max_degree <= kHubChunk;
         run.phase(GPART_PROFILE_REFINE_FILTER, [&] {
-            filter_movers(ctx, g, c, labels, targets, gains, flags, append, light.get(), heavy.get(), st.get());
+            filter_movers(ctx, g, c, labels, targets, gains, flags, append, light.get(), heavy.get(), st.get(), r);
         });
         if (!append)
             run.phase(-1, [&] {
@@ -1960,9 +2176,13 @@ struct Ops {
                                                     MoverStore{light.get(), heavy.get(), n, st.get()}, n,
                                                     MoverPairOp{});
             });
-        apply(ctx, run, g, c, st.get(), light.get(), heavy.get(), labels, targets, flags, k, cache, part_weights,
-              locks);
-        finish(ctx, run, g, k, out);
+        if (r)
+            apply_rows(ctx, run, g, c, r, st.get(), light.get(), heavy.get(), labels, targets, flags, k, cache,
+                       part_weights, locks);
+        else
+            apply(ctx, run, g, c, st.get(), light.get(), heavy.get(), labels, targets, flags, k, cache, part_weights,
+                  locks);
+        finish(ctx, run, g, k, r != nullptr, out);
     }
 
     // Everything a round's launches depend on besides its own scratch.
@@ -1970,6 +2190,7 @@ struct Ops {
                                                 const gpart_degree_classes* c, const C* cache,
                                                 const std::int32_t* labels, int k, const std::int32_t* targets,
                                                 const std::int32_t* flags, const unsigned long long* part_weights,
+                                                const gpart_refine_rows* r,
                                                 std::initializer_list<std::uint64_t> extra) {
         std::vector<std::uint64_t> key{sizeof(O), sizeof(C), static_cast<std::uint64_t>(g->n),
                                        static_cast<std::uint64_t>(g->m), key_of(g->offsets), key_of(g->neighbors),
@@ -1981,7 +2202,10 @@ struct Ops {
                                        static_cast<std::uint64_t>(c->max_degree), key_of(cache), key_of(labels),
                                        static_cast<std::uint64_t>(k), key_of(targets), key_of(flags),
                                        key_of(part_weights), static_cast<std::uint64_t>(rebuild_threshold(ctx, g)),
-                                       key_of(ctx->status_device), key_of(ctx->status_counter)};
+                                       key_of(ctx->status_device), key_of(ctx->status_counter),
+                                       r ? key_of(r->states.get()) : 0, r ? static_cast<std::uint64_t>(r->form) : 0,
+                                       r && r->hubs ? key_of(r->chunks.start.get()) : 0,
+                                       r && r->hubs ? key_of(r->chunks.hub.get()) : 0};
         key.insert(key.end(), extra.begin(), extra.end());
         return key;
     }
@@ -1991,20 +2215,25 @@ struct Ops {
     static void rebalance_round_small(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
                                       C* cache, std::int32_t* labels, int k, unsigned long long* part_weights,
                                       std::uint64_t capacity, std::int32_t* targets, std::int32_t* flags,
-                                      const PowerTable& powers, gpart_refine_status* out) {
+                                      const PowerTable& powers, const gpart_refine_rows* r,
+                                      gpart_refine_status* out) {
         const std::int64_t n = g->n;
         const auto* off = static_cast<const O*>(g->offsets);
         const auto* vw = static_cast<const W*>(g->vertex_weights);
-        RoundRun run(ctx, round_plan(ctx, n, round_key(ctx, g, c, cache, labels, k, targets, flags, part_weights,
+        RoundRun run(ctx, round_plan(ctx, n, round_key(ctx, g, c, cache, labels, k, targets, flags, part_weights, r,
                                                        {2, capacity})));
         Scratch<RoundState> st(ctx, 1);
         Scratch<std::int32_t> choices(ctx, n), light(ctx, n), heavy(ctx, n);
+        unsigned char* state = r ? r->states.get() : nullptr;
         const int G = group_for_k(k);
+        if (r)
+            run.phase(GPART_PROFILE_REFINE_CACHE,
+                      [&] { rows(ctx, g, c, r, k, cache, part_weights, capacity); });
         run.phase(GPART_PROFILE_REBALANCE, [&] {
             profile_begin(ctx, GPART_PROFILE_REBALANCE);
 #define GPART_BALANCE_VERTICES(GG)                                                                                 \
     hipLaunchKernelGGL((balance_vertices_kernel<W, GG, C>), dim3(grid_for(n * GG)), dim3(kBlock), 0, ctx->stream, \
-                       st.get(), n, cache, labels, vw, k, part_weights, capacity, powers, targets, choices.get(), flags)
+                       st.get(), n, cache, labels, vw, k, part_weights, capacity, powers, targets, choices.get(), flags, state)
             switch (G) {
                 case 1: GPART_BALANCE_VERTICES(1); break;
                 case 2: GPART_BALANCE_VERTICES(2); break;
@@ -2018,16 +2247,20 @@ struct Ops {
 #define GPART_BALANCE_SELECT(ITEMS)                                                                              \
     hipLaunchKernelGGL((balance_select_kernel<O, W, ITEMS>), dim3(1), dim3(kSelectThreads), 0, ctx->stream,      \
                        st.get(), n, choices.get(), vw, off, k, part_weights, capacity, light.get(), heavy.get(), \
-                       flags)
+                       flags, state)
             if (n <= kSelectThreads) GPART_BALANCE_SELECT(1);
             else if (n <= 4 * kSelectThreads) GPART_BALANCE_SELECT(4);
             else GPART_BALANCE_SELECT(kSelectMaxItems);
 #undef GPART_BALANCE_SELECT
             GPART_LAUNCH_CHECK();
         });
-        apply(ctx, run, g, c, st.get(), light.get(), heavy.get(), labels, targets, flags, k, cache, part_weights,
-              nullptr);
-        finish(ctx, run, g, k, out);
+        if (r)
+            apply_rows(ctx, run, g, c, r, st.get(), light.get(), heavy.get(), labels, targets, flags, k, cache,
+                       part_weights, nullptr);
+        else
+            apply(ctx, run, g, c, st.get(), light.get(), heavy.get(), labels, targets, flags, k, cache, part_weights,
+                  nullptr);
+        finish(ctx, run, g, k, r != nullptr, out);
     }
 
     // One rebalance iteration: proposals, source and destination bucket quotas,
@@ -2035,12 +2268,14 @@ struct Ops {
     static void rebalance_round(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
                                 C* cache, std::int32_t* labels, int k,
                                 unsigned long long* part_weights, std::uint64_t capacity, std::int32_t* targets,
-                                std::int32_t* flags, gpart_refine_status* out) {
+                                std::int32_t* flags, const gpart_refine_rows* r, gpart_refine_status* out) {
         static const PowerTable powers = make_power_table();
         if (g->n <= kSelectVertices)
-            rebalance_round_small(ctx, g, c, cache, labels, k, part_weights, capacity, targets, flags, powers, out);
+            rebalance_round_small(ctx, g, c, cache, labels, k, part_weights, capacity, targets, flags, powers, r,
+                                  out);
         else
-            rebalance_round_large(ctx, g, c, cache, labels, k, part_weights, capacity, targets, flags, powers, out);
+            rebalance_round_large(ctx, g, c, cache, labels, k, part_weights, capacity, targets, flags, powers, r,
+                                  out);
         // per candidate: id, label, weight, cache row, target and bucket writes
         profile_add_bytes(ctx, GPART_PROFILE_REBALANCE,
                           static_cast<double>(out->candidates) * (16.0 + sizeof(W) + sizeof(C) * k));
@@ -2051,7 +2286,8 @@ struct Ops {
     static void rebalance_round_large(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
                                       C* cache, std::int32_t* labels, int k, unsigned long long* part_weights,
                                       std::uint64_t capacity, std::int32_t* targets, std::int32_t* flags,
-                                      const PowerTable& powers, gpart_refine_status* out) {
+                                      const PowerTable& powers, const gpart_refine_rows* r,
+                                      gpart_refine_status* out) {
         const std::int64_t n = g->n;
         const auto* off = static_cast<const O*>(g->offsets);
         const auto* vw = static_cast<const W*>(g->vertex_weights);
@@ -2070,7 +2306,7 @@ struct Ops {
         }
         if (!ctx->rebalance_counters_zero) fill_bytes(ctx, ctx->rebalance_counters, 0, ctx->rebalance_counter_bytes);
         ctx->rebalance_counters_zero = false;  // until this round completes
-        RoundRun run(ctx, round_plan(ctx, n, round_key(ctx, g, c, cache, labels, k, targets, flags, part_weights,
+        RoundRun run(ctx, round_plan(ctx, n, round_key(ctx, g, c, cache, labels, k, targets, flags, part_weights, r,
                                                        {1, capacity, key_of(ctx->rebalance_counters)})));
         Scratch<RoundState> st(ctx, 1);
         Scratch<unsigned long long> counts(ctx, 2 * width), offsets(ctx, 2 * width), thresholds(ctx, 64);
@@ -2088,15 +2324,19 @@ struct Ops {
         Scratch<unsigned long long> sums(ctx, static_cast<std::int64_t>(slices) * 32),
             prefix(ctx, static_cast<std::int64_t>(slices) * 32);
         // small grids sum the per-workgroup boundary weights in the ranks kernels
+        unsigned char* state = r ? r->states.get() : nullptr;
         const bool inline_columns = slices <= kInlineColumnBlocks;
         const unsigned long long* column_prefix = inline_columns ? nullptr : prefix.get();
 
         run.phase(-1, [&] {
             device_scan<int, SumOp<int>>(ctx, OverloadedLoad{labels, part_weights, capacity},
-                                         CandidateStore{cand.get(), flags, n, st_ptr}, n, SumOp<int>{});
+                                         CandidateStore{cand.get(), flags, labels, state, n, st_ptr}, n, SumOp<int>{});
         });
         const int G = group_for_k(k);
         const auto blocks = static_cast<unsigned>(std::min<std::int64_t>(grid_for(n * G), ctx->balance_blocks));
+        if (r)
+            run.phase(GPART_PROFILE_REFINE_CACHE,
+                      [&] { rows(ctx, g, c, r, k, cache, part_weights, capacity); });
         run.phase(GPART_PROFILE_REBALANCE, [&] {
         profile_begin(ctx, GPART_PROFILE_REBALANCE);
 #define GPART_BALANCE_PROPOSALS(GG)                                                                              \
@@ -2128,18 +2368,22 @@ struct Ops {
                            dst_counts, dst_offsets, part_weights, capacity, true, dst_thresholds);
         hipLaunchKernelGGL((balance_destinations_kernel<O, W>), dim3(slices), dim3(kBlock), 0, ctx->stream,
                            st_ptr, cand.get(), dbucket.get(), vw, off, dst_counts, dst_offsets, dst_thresholds,
-                           sums.get(), labels, light.get(), heavy.get(), flags);
+                           sums.get(), labels, light.get(), heavy.get(), flags, state);
         if (!inline_columns)
             hipLaunchKernelGGL(column_scan_kernel, dim3(k), dim3(kBucketScanThreads), 0, ctx->stream, sums.get(),
                                slices, prefix.get());
         hipLaunchKernelGGL((balance_destination_ranks_kernel<O, W>), dim3(slices), dim3(kBlock), 0, ctx->stream,
                            st_ptr, cand.get(), dbucket.get(), vw, off, dst_offsets, dst_thresholds, column_prefix,
-                           sums.get(), labels, light.get(), heavy.get(), flags);
+                           sums.get(), labels, light.get(), heavy.get(), flags, state);
         GPART_LAUNCH_CHECK();
         });
-        apply(ctx, run, g, c, st_ptr, light.get(), heavy.get(), labels, targets, flags, k, cache, part_weights,
-              nullptr);
-        finish(ctx, run, g, k, out);
+        if (r)
+            apply_rows(ctx, run, g, c, r, st_ptr, light.get(), heavy.get(), labels, targets, flags, k, cache,
+                       part_weights, nullptr);
+        else
+            apply(ctx, run, g, c, st_ptr, light.get(), heavy.get(), labels, targets, flags, k, cache, part_weights,
+                  nullptr);
+        finish(ctx, run, g, k, r != nullptr, out);
         ctx->rebalance_counters_zero = true;
     }
 };
@@ -2195,6 +2439,18 @@ using namespace gpart_hip;
             using OpsT = Ops<std::int64_t, std::uint64_t>;           \
             call;                                                    \
         }                                                            \
+    } while (0)
+
+// Width of the entry points without an incremental cache (4-byte rows).
+#define GPART_ROWS_DISPATCH(width, call)                                       \
+    do {                                                                       \
+        if ((width) == GPART_WIDTH_STANDARD) {                                  \
+            using OpsT = Ops<std::int32_t, std::uint32_t, unsigned>;           \
+            call;                                                              \
+        } else {                                                               \
+            using OpsT = Ops<std::int64_t, std::uint64_t, unsigned>;           \
+            call;                                                              \
+        }                                                                      \
     } while (0)
 
 // Width and cache entry type (4 or 8 bytes) of the refinement entry points.
@@ -2302,7 +2558,68 @@ int gpart_refine_lp_round(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_d
         GPART_CACHE_DISPATCH(g->width, cache_bytes,
                              OpsT::lp_round(ctx, g, classes, static_cast<CacheT*>(cache), labels, k, filter, locks,
                                             targets, reinterpret_cast<long long*>(gains), flags,
-                                            reinterpret_cast<unsigned long long*>(part_weights), status));
+                                            reinterpret_cast<unsigned long long*>(part_weights), nullptr, status));
+    });
+}
+
+int gpart_refine_rows_create(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes, int k,
+                             int cache_bytes, gpart_refine_rows** rows) {
+    return guarded([&] {
+        if (!ctx || !g || !classes || !rows) throw Error(GPART_ERR_INVALID_ARGUMENT, "null argument");
+        if (k < 1 || k > 32) throw Error(GPART_ERR_INVALID_ARGUMENT, "part count must be in [1, 32]");
+        *rows = nullptr;
+        if (cache_bytes != 4 || g->n <= 0 || g->m < kRowsMinDegree * g->n || g->n > kRowsMaxVertices) return;
+        auto made = std::make_unique<gpart_refine_rows>();
+        made->form = g->n <= kStateBytes ? kByteState
+                     : k <= 8 && g->n <= 2 * kStateBytes ? kNibbleState
+                                                         : kMemoryState;
+        made->states.reset(ctx, (g->n + 15) / 16 * 16);
+        made->hubs = classes->max_degree > kHubChunk;
+        if (made->hubs) {
+            if (g->width == GPART_WIDTH_STANDARD)
+                build_hub_chunks(ctx, static_cast<const std::int32_t*>(g->offsets), classes->high, classes->high_count,
+                                 classes->high_edges, kHubChunk, made->chunks);
+            else
+                build_hub_chunks(ctx, static_cast<const std::int64_t*>(g->offsets), classes->high, classes->high_count,
+                                 classes->high_edges, kHubChunk, made->chunks);
+        }
+        *rows = made.release();
+    });
+}
+
+void gpart_refine_rows_destroy(gpart_refine_rows* rows) { delete rows; }
+
+int gpart_refine_lp_round_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes,
+                               gpart_refine_rows* rows, uint32_t* cache, int32_t* labels, int k, double filter,
+                               int32_t* locks, int32_t* targets, int64_t* gains, int32_t* flags,
+                               uint64_t* part_weights, gpart_refine_status* status) {
+    return guarded([&] {
+        if (!rows) throw Error(GPART_ERR_INVALID_ARGUMENT, "null rows");
+        if (k < 1 || k > 32) throw Error(GPART_ERR_INVALID_ARGUMENT, "part count must be in [1, 32]");
+        if (g->n <= 0) throw Error(GPART_ERR_INVALID_ARGUMENT, "refinement round needs vertices");
+        GPART_ROWS_DISPATCH(g->width, {
+            OpsT::prepare_rows(ctx, g, classes, rows, labels, k, cache);
+            OpsT::lp_round(ctx, g, classes, cache, labels, k, filter, locks, targets,
+                           reinterpret_cast<long long*>(gains), flags,
+                           reinterpret_cast<unsigned long long*>(part_weights), rows, status);
+        });
+    });
+}
+
+int gpart_refine_rebalance_round_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes,
+                                      gpart_refine_rows* rows, uint32_t* cache, int32_t* labels, int k,
+                                      uint64_t* part_weights, uint64_t capacity, int32_t* targets, int32_t* flags,
+                                      gpart_refine_status* status) {
+    return guarded([&] {
+        if (!rows) throw Error(GPART_ERR_INVALID_ARGUMENT, "null rows");
+        if (k < 1 || k > 32) throw Error(GPART_ERR_INVALID_ARGUMENT, "part count must be in [1, 32]");
+        if (g->n <= 0) throw Error(GPART_ERR_INVALID_ARGUMENT, "refinement round needs vertices");
+        GPART_ROWS_DISPATCH(g->width, {
+            OpsT::prepare_rows(ctx, g, classes, rows, labels, k, cache);
+            OpsT::rebalance_round(ctx, g, classes, cache, labels, k,
+                                  reinterpret_cast<unsigned long long*>(part_weights), capacity, targets, flags,
+                                  rows, status);
+        });
     });
 }
 
@@ -2341,7 +2658,7 @@ int gpart_refine_rebalance_round(gpart_ctx* ctx, const gpart_csr_view* g, const 
         GPART_CACHE_DISPATCH(g->width, cache_bytes,
                              OpsT::rebalance_round(ctx, g, classes, static_cast<CacheT*>(cache), labels, k,
                                                    reinterpret_cast<unsigned long long*>(part_weights), capacity,
-                                                   targets, flags, status));
+                                                   targets, flags, nullptr, status));
     });
 }
 

@@ -12,6 +12,7 @@
 #include <cmath>
 #include <iostream>
 #include <limits>
+#include <memory>
 #include <numeric>
 #include <stdexcept>
 
@@ -104,7 +105,22 @@ RefineStats run_refinement(Level<Types>& level, const RefineOptions& options, in
     DeviceVector<std::uint8_t> cache(N * static_cast<std::size_t>(k) * static_cast<std::size_t>(cache_bytes));
     DeviceVector<std::int32_t> targets(N), locks(N, 0), flags(N, 0);
     DeviceVector<std::int64_t> gains(N);
-    GPART_CHECK(gpart_refine_build_cache(ctx, &view, &classes, level.partition.data(), k, cache.data(), cache_bytes));
+    int grid = 0;
+    if (!options.strict_verify)
+        GPART_CHECK(gpart_refine_engine_grid(ctx, &view, &classes, cache_bytes, &grid));
+    // Dense levels sum their rows where a round reads them; the others keep a cache.
+    struct RowsDelete {
+        void operator()(gpart_refine_rows* r) const { gpart_refine_rows_destroy(r); }
+    };
+    std::unique_ptr<gpart_refine_rows, RowsDelete> rows;
+    if (grid == 0) {
+        gpart_refine_rows* made = nullptr;
+        GPART_CHECK(gpart_refine_rows_create(ctx, &view, &classes, k, cache_bytes, &made));
+        rows.reset(made);
+    }
+    auto* row_cache = reinterpret_cast<std::uint32_t*>(cache.data());
+    if (!rows)
+        GPART_CHECK(gpart_refine_build_cache(ctx, &view, &classes, level.partition.data(), k, cache.data(), cache_bytes));
 
     RefineStats stats;
     stats.initial_cut = known_cut ? *known_cut : level.cut();
@@ -119,9 +135,6 @@ RefineStats run_refinement(Level<Types>& level, const RefineOptions& options, in
         return stats;
     };
     // Levels within the engine's tuning run the whole loop below in one launch.
-    int grid = 0;
-    if (!options.strict_verify)
-        GPART_CHECK(gpart_refine_engine_grid(ctx, &view, &classes, cache_bytes, &grid));
     if (grid > 0) {
         gpart_refine_level_stats e{};
         GPART_CHECK(gpart_refine_level(ctx, &view, &classes, cache.data(), cache_bytes, level.partition.data(), k,
@@ -160,6 +173,7 @@ RefineStats run_refinement(Level<Types>& level, const RefineOptions& options, in
         level.host_part_weights.assign(status.part_weights, status.part_weights + k);
         if (options.strict_verify) {
             if (level.cut() != current_cut) throw std::runtime_error("incremental cut differs from CSR scan");
+            if (rows) return;  // no cache is kept
             DeviceVector<std::uint8_t> check(cache.size());
             GPART_CHECK(gpart_refine_build_cache(ctx, &view, &classes, level.partition.data(), k, check.data(),
                                                  cache_bytes));
@@ -171,10 +185,15 @@ RefineStats run_refinement(Level<Types>& level, const RefineOptions& options, in
         for (int iteration = 0; iteration < 2 * k + 4 && level.maximum() > level.capacity; ++iteration) {
             ++stats.admission_iterations;
             gpart_refine_status status{};
-            GPART_CHECK(gpart_refine_rebalance_round(ctx, &view, &classes, cache.data(), cache_bytes,
-                                                     level.partition.data(), k,
-                                                     level.part_weights.data(), level.capacity, targets.data(),
-                                                     flags.data(), &status));
+            if (rows)
+                GPART_CHECK(gpart_refine_rebalance_round_rows(ctx, &view, &classes, rows.get(), row_cache,
+                                                              level.partition.data(), k, level.part_weights.data(),
+                                                              level.capacity, targets.data(), flags.data(), &status));
+            else
+                GPART_CHECK(gpart_refine_rebalance_round(ctx, &view, &classes, cache.data(), cache_bytes,
+                                                         level.partition.data(), k,
+                                                         level.part_weights.data(), level.capacity, targets.data(),
+                                                         flags.data(), &status));
             if (!status.movers) return false;
             absorb(status);
         }
@@ -184,10 +203,15 @@ RefineStats run_refinement(Level<Types>& level, const RefineOptions& options, in
     for (int phase = 0; phase < rounds && stale < options.stale_rounds; ++phase) {
         stats.rounds = phase + 1;
         gpart_refine_status status{};
-        GPART_CHECK(gpart_refine_lp_round(ctx, &view, &classes, cache.data(), cache_bytes, level.partition.data(),
-                                          k, filter,
-                                          locks.data(), targets.data(), gains.data(), flags.data(),
-                                          level.part_weights.data(), &status));
+        if (rows)
+            GPART_CHECK(gpart_refine_lp_round_rows(ctx, &view, &classes, rows.get(), row_cache,
+                                                   level.partition.data(), k, filter, locks.data(), targets.data(),
+                                                   gains.data(), flags.data(), level.part_weights.data(), &status));
+        else
+            GPART_CHECK(gpart_refine_lp_round(ctx, &view, &classes, cache.data(), cache_bytes, level.partition.data(),
+                                              k, filter,
+                                              locks.data(), targets.data(), gains.data(), flags.data(),
+                                              level.part_weights.data(), &status));
         stats.proposals += static_cast<std::uint64_t>(status.movers);
         if (!status.movers) {
             if (++empty >= 2) break;

@@ -472,6 +472,26 @@ int gpart_refine_rebalance_round(gpart_ctx* ctx, const gpart_csr_view* g,
                                  const gpart_degree_classes* classes, void* cache, int cache_bytes,
                                  int32_t* labels, int k, uint64_t* part_weights, uint64_t capacity,
                                  int32_t* targets, int32_t* flags, gpart_refine_status* status);
+/* The same rounds without an incremental cache: the connectivity rows are summed
+ * from the CSR where a round reads them (an LP round every row, a rebalance iteration
+ * the rows of overloaded parts), which is cheaper on dense levels than updating them.
+ * gpart_refine_rows_create gives the level's handle, or NULL in *rows where the level
+ * is better served by the cached rounds above (a sparse or very large level, or 8-byte
+ * entries); destroy it before its context. cache (n x k 4-byte entries, device) is the rounds'
+ * scratch and needs no gpart_refine_build_cache; it stays with one handle. Same
+ * labels, part weights and status as the cached rounds; rebuilt is 0. */
+typedef struct gpart_refine_rows gpart_refine_rows;
+int gpart_refine_rows_create(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes, int k,
+                             int cache_bytes, gpart_refine_rows** rows);
+void gpart_refine_rows_destroy(gpart_refine_rows* rows);
+int gpart_refine_lp_round_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes,
+                               gpart_refine_rows* rows, uint32_t* cache, int32_t* labels, int k, double filter,
+                               int32_t* locks, int32_t* targets, int64_t* gains, int32_t* flags,
+                               uint64_t* part_weights, gpart_refine_status* status);
+int gpart_refine_rebalance_round_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes,
+                                      gpart_refine_rows* rows, uint32_t* cache, int32_t* labels, int k,
+                                      uint64_t* part_weights, uint64_t capacity, int32_t* targets, int32_t* flags,
+                                      gpart_refine_status* status);
 /* Round graphs (no reference counterpart: the reference launches every kernel of a
  * round from the host). gpart_refine_lp_round and gpart_refine_rebalance_round
  * record the launches of a round the first time they see its level, arrays and
