@@ -238,10 +238,7 @@ template <typename Types>
 void partition_impl(GraphOf<Types>& g, int parts, double ratio, uint32_t seed, int verify, int mode, int32_t* labels,
                     gpart_partition_report* report) {
     auto partition = run_pipeline(g, parts, ratio, seed, verify, mode, report);
-    if (labels) {
-        const auto host = partition.to_host();
-        std::copy(host.begin(), host.end(), labels);
-    }
+    if (labels) partition.copy_to(labels);
 }
 
 }  // namespace
@@ -402,7 +399,8 @@ int gpart_graph_cut(gpart_graph* g, const int32_t* labels, uint64_t* cut) {
     return guard([&] {
         std::visit(
             [&](auto& x) {
-                gpart::DeviceVector<std::int32_t> d(std::vector<std::int32_t>(labels, labels + x.device.vertices()));
+                gpart::DeviceVector<std::int32_t> d;
+                d.assign(labels, static_cast<std::size_t>(x.device.vertices()));
                 const auto view = x.device.view();
                 GPART_CHECK(gpart_cut(gpart::detail::context(), &view, d.data(), cut));
             },
@@ -426,7 +424,8 @@ int gpart_graph_verify(gpart_graph* g, const int32_t* labels, int parts, const c
             [&](auto& x) {
                 const auto n = x.device.vertices();
                 if (n > 0 && !labels) throw std::invalid_argument("null labels");
-                gpart::DeviceVector<std::int32_t> d(std::vector<std::int32_t>(labels, labels + n));
+                gpart::DeviceVector<std::int32_t> d;
+                d.assign(labels, static_cast<std::size_t>(n));
                 const auto view = x.device.view();
                 const auto r = gpart::verify_partition(gpart::detail::context(), view, d.data(), labels, parts,
                                                        imbalance);
@@ -446,7 +445,8 @@ int gpart_graph_analyze(gpart_graph* g, const int32_t* labels, int parts, gpart_
             [&](auto& x) {
                 const auto n = x.device.vertices();
                 if (n > 0 && !labels) throw std::invalid_argument("null labels");
-                gpart::DeviceVector<std::int32_t> d(std::vector<std::int32_t>(labels, labels + n));
+                gpart::DeviceVector<std::int32_t> d;
+                d.assign(labels, static_cast<std::size_t>(n));
                 const auto view = x.device.view();
                 const auto r = gpart::analyze_partition(gpart::detail::context(), view, d.data(), parts);
                 if (per_part && per_part_capacity < r.parts)
@@ -597,10 +597,7 @@ int gpart_partition_batch(int count, gpart_graph* const* graphs, const int* part
             try {
                 if (!failed.load() && labels)
                     for (auto& [i, part] : done)
-                        if (labels[i]) {
-                            const auto host = part.to_host();
-                            std::copy(host.begin(), host.end(), labels[i]);
-                        }
+                        if (labels[i]) part.copy_to(labels[i]);
             } catch (...) {
                 fail();
             }
@@ -681,10 +678,20 @@ int gpart_graph_aggregate(gpart_graph* g, int parts, uint32_t seed, int level, i
                 gpart::SclpStats stats;
                 auto result = gpart::aggregate(x.device, workspace, parts, seed, level, stats, false,
                                                cluster_size_factor, pack_isolated != 0);
-                const auto mapping = result.map.to_host();
-                const auto weights = result.vertex_weights.to_host();
-                std::copy(mapping.begin(), mapping.end(), map);
-                for (std::size_t i = 0; i < weights.size(); ++i) cluster_weights[i] = static_cast<uint64_t>(weights[i]);
+                result.map.copy_to(map);
+                if constexpr (sizeof(typename T::WeightT) == sizeof(uint64_t)) {
+                    result.vertex_weights.copy_to(cluster_weights);
+                } else {
+                    // 32-bit weights land in the upper half of the 64-bit array and widen upwards
+                    const std::size_t count = result.vertex_weights.size();
+                    auto* narrow = reinterpret_cast<typename T::WeightT*>(cluster_weights) + count;
+                    result.vertex_weights.copy_to(narrow);
+                    for (std::size_t i = 0; i < count; ++i) {
+                        typename T::WeightT w;
+                        std::memcpy(&w, narrow + i, sizeof w);
+                        cluster_weights[i] = w;
+                    }
+                }
                 *coarse_vertices = static_cast<int64_t>(result.coarse_vertices);
                 *capacity = result.capacity;
                 *maximum_weight = result.maximum_weight;
@@ -807,12 +814,8 @@ int gpart_graph_initial_partition(gpart_graph* g, int parts, double ratio, uint3
                 auto l = gpart::initial_partition_gpu<Types>(x.device, parts, ratio, seed,
                                                              static_cast<gpart::SpectralMode>(spectral_mode),
                                                              coords ? &c : nullptr);
-                const auto host = l.to_host();
-                std::copy(host.begin(), host.end(), labels);
-                if (coords) {
-                    const auto hc = c.to_host();
-                    std::copy(hc.begin(), hc.end(), coords);
-                }
+                l.copy_to(labels);
+                if (coords) c.copy_to(coords);
             },
             g->g);
     });
@@ -855,10 +858,8 @@ int gpart_graph_refine(gpart_graph* g, int32_t* labels, int parts, double ratio,
                 o.max_rounds = max_rounds;
                 o.stale_rounds = stale_rounds;
                 o.strict_verify = verify != 0;
-                std::vector<std::int32_t> l(labels, labels + x.device.vertices());
                 gpart::RefineStats s;
-                gpart::refine_partition(host_of(x), l, o, &s);
-                std::copy(l.begin(), l.end(), labels);
+                gpart::refine_partition(x.device, labels, labels, o, &s);
                 if (report) {
                     report->rounds = s.rounds;
                     report->admission_iterations = s.admission_iterations;

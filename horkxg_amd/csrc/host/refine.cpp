@@ -412,6 +412,48 @@ void refine_partition(const WeightedGraph<Types>& graph, std::vector<typename Ty
 }
 
 template <typename Types>
+void refine_partition(const DeviceWeightedGraph<Types>& graph, const typename Types::VertexT* labels,
+                      typename Types::VertexT* refined, const RefineOptions& options, RefineStats* output_stats) {
+    const auto n = graph.vertices();
+    if (n <= 0) throw std::invalid_argument("invalid refinement options");
+    check_options(options);
+    const int k = options.parts;
+    const auto view = graph.view();
+    auto* ctx = detail::context();
+    bool valid = true;
+    for (std::int64_t v = 0; v < n; ++v) valid &= labels[v] >= 0 && labels[v] < k;
+    if constexpr (sizeof(typename Types::WeightT) == 8) {
+        // 64-bit weights whose sum does not fit (or labels that are no parts): the host
+        // form reports whichever it meets first
+        std::uint64_t total = 0, heaviest = 0, lightest = 0;
+        GPART_CHECK(gpart_vertex_weight_stats(ctx, &view, &total, &heaviest, &lightest));
+        if (total == std::numeric_limits<std::uint64_t>::max()) {
+            std::vector<typename Types::VertexT> copy(labels, labels + n);
+            refine_partition(copy_device_weighted(graph), copy, options, output_stats);
+            std::copy(copy.begin(), copy.end(), refined);
+            return;
+        }
+    }
+    if (!valid) throw std::invalid_argument("refinement partition has an invalid part id");
+    Level<Types> level;
+    level.graph.offsets = decltype(level.graph.offsets)::borrow(graph.offsets);
+    level.graph.neighbors = decltype(level.graph.neighbors)::borrow(graph.neighbors);
+    level.graph.edge_weights = decltype(level.graph.edge_weights)::borrow(graph.edge_weights);
+    level.graph.vertex_weights = decltype(level.graph.vertex_weights)::borrow(graph.vertex_weights);
+    level.partition.assign(labels, static_cast<std::size_t>(n));
+    level.part_weights.resize_discard(static_cast<std::size_t>(k));
+    GPART_CHECK(gpart_part_weights(ctx, &view, level.partition.data(), k, level.part_weights.data()));
+    level.host_part_weights = level.part_weights.to_host();
+    const auto total =
+        std::accumulate(level.host_part_weights.begin(), level.host_part_weights.end(), std::uint64_t{0});
+    level.capacity = partition_capacity(total, k, options.imbalance_ratio);
+    if (level.maximum() > level.capacity) throw std::invalid_argument("initial refinement partition is imbalanced");
+    const auto stats = run_refinement(level, options, options.max_rounds);
+    level.partition.copy_to(refined);
+    if (output_stats) *output_stats = stats;
+}
+
+template <typename Types>
 DeviceUncoarsenResult<Types> refine_hierarchy_device(const Hierarchy<Types>& hierarchy,
                                                      const std::vector<typename Types::VertexT>& partition,
                                                      const RefineOptions& options) {
@@ -428,6 +470,8 @@ DeviceUncoarsenResult<Types> refine_hierarchy_device(DeviceHierarchy<Types>& hie
 #define GPART_INSTANTIATE_REFINE(T)                                                                              \
     template void refine_partition<T>(const WeightedGraph<T>&, std::vector<typename T::VertexT>&,                \
                                       const RefineOptions&, RefineStats*);                                      \
+    template void refine_partition<T>(const DeviceWeightedGraph<T>&, const typename T::VertexT*,                 \
+                                      typename T::VertexT*, const RefineOptions&, RefineStats*);                \
     template DeviceUncoarsenResult<T> refine_hierarchy_device<T>(                                               \
         const Hierarchy<T>&, const std::vector<typename T::VertexT>&, const RefineOptions&);                    \
     template DeviceUncoarsenResult<T> refine_hierarchy_device<T>(DeviceHierarchy<T>&,                           \

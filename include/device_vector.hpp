@@ -109,6 +109,15 @@ public:
         if (!host.empty())
             GPART_CHECK(gpart_memcpy_htod(detail::context(), data_, host.data(), host.size() * sizeof(T)));
     }
+    // The same from a caller's array, without a copy on the host in between.
+    void assign(const T* host, std::size_t n) {
+        resize_discard(n);
+        if (n) GPART_CHECK(gpart_memcpy_htod(detail::context(), data_, host, n * sizeof(T)));
+    }
+    // Into a caller's array of size() elements.
+    void copy_to(T* host) const {
+        if (size_) GPART_CHECK(gpart_memcpy_dtoh(detail::context(), host, data_, size_ * sizeof(T)));
+    }
     void fill(const T& value);
     std::vector<T> to_host() const {
         std::vector<T> host(size_);

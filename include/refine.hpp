@@ -66,6 +66,13 @@ template <typename Types>
 void refine_partition(const WeightedGraph<Types>& graph, std::vector<typename Types::VertexT>& partition,
                       const RefineOptions& options, RefineStats* stats = nullptr);
 
+// The same for a graph that is on the device already (it is only read): labels are
+// vertices() entries on the host, refined receives as many and may be the same array.
+// No reference counterpart: the reference's overload uploads the graph on every call.
+template <typename Types>
+void refine_partition(const DeviceWeightedGraph<Types>& graph, const typename Types::VertexT* labels,
+                      typename Types::VertexT* refined, const RefineOptions& options, RefineStats* stats = nullptr);
+
 template <typename Types>
 DeviceUncoarsenResult<Types> refine_hierarchy_device(const Hierarchy<Types>& hierarchy,
                                                      const std::vector<typename Types::VertexT>& coarsest_partition,
