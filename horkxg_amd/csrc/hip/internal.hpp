@@ -84,6 +84,9 @@ struct gpart_ctx {
     void* rebalance_counters = nullptr;
     std::size_t rebalance_counter_bytes = 0;
     bool rebalance_counters_zero = false;
+    // The part weights that the last refinement round left (a hint: how many vertices
+    // the next rebalance iteration will move).
+    std::uint64_t round_part_weights[32] = {};
 };
 
 namespace gpart_hip {

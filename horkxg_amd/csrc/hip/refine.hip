@@ -307,7 +307,7 @@ __global__ void __launch_bounds__(kBlock) lp_proposals_kernel(std::int64_t n, co
 // Appends the taking threads' vertices to the light/heavy mover lists (one
 // global atomic per list per workgroup pass). Called by every thread of the
 // workgroup.
-template <typename O>
+template <int Threads, typename O>
 __device__ void append_movers(bool take, std::int32_t v, const O* offsets, std::int32_t* light,
                               std::int32_t* heavy, RoundState* st, unsigned* counts, unsigned long long* base) {
     const int lane = lane_id(), wave = threadIdx.x / kWave;
@@ -320,14 +320,14 @@ __device__ void append_movers(bool take, std::int32_t v, const O* offsets, std::
     const unsigned long long bl = __ballot(is_light), bh = __ballot(is_heavy);
     if (lane == 0) {
         counts[wave] = static_cast<unsigned>(__popcll(bl));
-        counts[kBlock / kWave + wave] = static_cast<unsigned>(__popcll(bh));
+        counts[Threads / kWave + wave] = static_cast<unsigned>(__popcll(bh));
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned tl = 0, th = 0;
-        for (int q = 0; q < kBlock / kWave; ++q) {
+        for (int q = 0; q < Threads / kWave; ++q) {
             tl += counts[q];
-            th += counts[kBlock / kWave + q];
+            th += counts[Threads / kWave + q];
         }
         base[0] = tl ? atomicAdd(reinterpret_cast<unsigned long long*>(&st->light), tl) : 0;
         base[1] = th ? atomicAdd(reinterpret_cast<unsigned long long*>(&st->heavy), th) : 0;
@@ -335,7 +335,7 @@ __device__ void append_movers(bool take, std::int32_t v, const O* offsets, std::
     __syncthreads();
     if (take) {
         unsigned before = 0;
-        const unsigned* row = is_heavy ? counts + kBlock / kWave : counts;
+        const unsigned* row = is_heavy ? counts + Threads / kWave : counts;
         for (int q = 0; q < wave; ++q) before += row[q];
         const unsigned long long mask = is_heavy ? bh : bl;
         before += static_cast<unsigned>(__popcll(mask & lanemask_lt()));
@@ -419,7 +419,7 @@ __global__ void __launch_bounds__(kBlock) priority_filter_kernel(
     if constexpr (Append) {
         __shared__ unsigned counts[2 * (kBlock / kWave)];
         __shared__ unsigned long long base[2];
-        if (__syncthreads_or(take)) append_movers(take, v, offsets, light, heavy, st, counts, base);
+        if (__syncthreads_or(take)) append_movers<kBlock>(take, v, offsets, light, heavy, st, counts, base);
     }
 }
 
@@ -892,8 +892,106 @@ struct MoverStore {
 // the weight of the lower-id members of their bucket (a blocked multisplit),
 // one legal outcome of the reference's atomicAdd ranking.
 
-// Candidates: vertices of overloaded parts, in id order. Every flag is cleared
-// on the way (movers are flagged later in the iteration).
+// The overloaded parts as a bit mask. Called by whole waves.
+__device__ __forceinline__ unsigned overloaded_parts(const unsigned long long* part_weights, int k,
+                                                     std::uint64_t capacity) {
+    const int lane = lane_id();
+    return static_cast<unsigned>(__ballot(lane < k && part_weights[lane < k ? lane : 0] > capacity));
+}
+
+// Candidates: vertices of overloaded parts, in id order, by a count per tile of
+// kBlock * Items vertices and a pass that lists them behind the counts below its tile.
+// A thread's vertices are kBlock apart (coalesced), a tile's order is (item, wave,
+// lane). The generic scan, with its gather of a part weight per vertex and pass, took
+// 5.3 + 8.6 us on the 128^3 mesh's levels on average.
+constexpr int kTileWaves = kBlock / kWave;
+constexpr std::int64_t kCandidateTiles = 1024;  // every workgroup sums the counts below its own
+
+template <int Items>
+__global__ void __launch_bounds__(kBlock) candidate_count_kernel(std::int64_t n, const std::int32_t* labels,
+                                                                 const unsigned long long* part_weights, int k,
+                                                                 std::uint64_t capacity, std::int32_t* tile_counts) {
+    __shared__ int wave_counts[kTileWaves];
+    const unsigned over = overloaded_parts(part_weights, k, capacity);
+    const std::int64_t base = static_cast<std::int64_t>(blockIdx.x) * kBlock * Items + threadIdx.x;
+    std::int32_t label[Items];
+#pragma unroll
+    for (int i = 0; i < Items; ++i) label[i] = base + i * kBlock < n ? labels[base + i * kBlock] : -1;
+    int count = 0;
+#pragma unroll
+    for (int i = 0; i < Items; ++i) count += __popcll(__ballot(label[i] >= 0 && (over >> label[i] & 1U)));
+    if (lane_id() == 0) wave_counts[threadIdx.x / kWave] = count;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int total = 0;
+        for (int w = 0; w < kTileWaves; ++w) total += wave_counts[w];
+        tile_counts[blockIdx.x] = total;
+    }
+}
+
+// Every flag is cleared on the way (movers are flagged later in the iteration), and
+// the states of refine_rows.hpp, where the level has them, are rewritten.
+template <int Items>
+__global__ void __launch_bounds__(kBlock) candidate_list_kernel(RoundState* st, std::int64_t n,
+                                                                const std::int32_t* labels,
+                                                                const unsigned long long* part_weights, int k,
+                                                                std::uint64_t capacity,
+                                                                const std::int32_t* tile_counts,
+                                                                std::int32_t* candidates, std::int32_t* flags,
+                                                                unsigned char* state) {
+    static_assert(Items * kTileWaves <= 2 * kWave, "one wave scans the counts, two per lane");
+    __shared__ int at[Items * kTileWaves];
+    __shared__ int below[kTileWaves];
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    const unsigned over = overloaded_parts(part_weights, k, capacity);
+    const std::int64_t base = static_cast<std::int64_t>(blockIdx.x) * kBlock * Items + threadIdx.x;
+    std::int32_t label[Items];
+#pragma unroll
+    for (int i = 0; i < Items; ++i) label[i] = base + i * kBlock < n ? labels[base + i * kBlock] : -1;
+    int carry = 0;
+    for (int t = threadIdx.x; t < static_cast<int>(blockIdx.x); t += kBlock) carry += tile_counts[t];
+    carry = wave_scan(carry);
+    if (lane == kWave - 1) below[wave] = carry;
+#pragma unroll
+    for (int i = 0; i < Items; ++i) {
+        const unsigned long long in = __ballot(label[i] >= 0 && (over >> label[i] & 1U));
+        if (lane == 0) at[i * kTileWaves + wave] = __popcll(in);
+    }
+    __syncthreads();
+    if (wave == 0) {
+        int first = 0;
+        for (int w = 0; w < kTileWaves; ++w) first += below[w];
+        constexpr int kPer = (Items * kTileWaves + kWave - 1) / kWave;
+        int counts[kPer], sum = 0;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            counts[i] = lane * kPer + i < Items * kTileWaves ? at[lane * kPer + i] : 0;
+            sum += counts[i];
+        }
+        const int inclusive = wave_scan(sum);
+        int running = first + inclusive - sum;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            if (lane * kPer + i < Items * kTileWaves) at[lane * kPer + i] = running;
+            running += counts[i];
+        }
+        if (lane == kWave - 1 && blockIdx.x == gridDim.x - 1) st->candidates = running;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < Items; ++i) {
+        const bool is = label[i] >= 0 && (over >> label[i] & 1U);
+        const unsigned long long in = __ballot(is);
+        const std::int64_t v = base + i * kBlock;
+        if (is) candidates[at[i * kTileWaves + wave] + __popcll(in & lanemask_lt())] = static_cast<std::int32_t>(v);
+        if (label[i] >= 0) {
+            flags[v] = 0;
+            if (state) state[v] = static_cast<unsigned char>(label[i]);
+        }
+    }
+}
+
+// The same for levels of more tiles, through the generic scan.
 struct OverloadedLoad {
     const std::int32_t* labels;
     const unsigned long long* part_weights;
@@ -920,42 +1018,70 @@ struct CandidateStore {
 
 // The choice of incremental_rebalance_proposals (:111-157) for one vertex of an
 // overloaded part, by a group of G lanes, lane j owning parts [8j, 8j + 8) of its
-// cache row: the destination (-1: none) and the source bucket (-1: none). pw: the
-// part weights (LDS). Every lane returns both.
+// cache row: the destination (-1: none) and the source bucket (-1: none). Every lane
+// returns both. U: the type of connectivities and slacks. 32 bits hold them, and every
+// sum of slacks, when cache entries have 4 bytes and k parts of the capacity fit; the
+// 64-bit form spent most of the finest mesh level's 62 us per launch in arithmetic.
 struct BalanceChoice {
     int target;
     int bucket;
 };
-template <int G, typename C>
+// The parts' slacks (0: no part, or full) and the bucket thresholds, in LDS.
+template <typename U>
+struct BalanceTables {
+    U slack[4 * kRowSpan];
+    double powers[48];
+    __device__ __forceinline__ void load(const unsigned long long* part_weights, int k, std::uint64_t capacity,
+                                         const PowerTable& table) {
+        const int t = threadIdx.x;
+        if (t < 4 * kRowSpan) {
+            const unsigned long long w = t < k ? part_weights[t] : capacity;
+            slack[t] = static_cast<U>(w < capacity ? capacity - w : 0);
+        }
+        if (t >= kWave && t < kWave + 48) powers[t - kWave] = table.value[t - kWave];
+    }
+};
+template <typename U>
+__device__ __forceinline__ U group_xor(U v, int mask, int width) {
+    if constexpr (sizeof(U) == 4) return lane_xor(v, mask, width);
+    else return shfl_xor_u64(v, mask, width);
+}
+template <typename U>
+__device__ __forceinline__ U saturated(U a, U b) {
+    if constexpr (sizeof(U) == 4) return a + b;  // every sum of slacks fits
+    else return ~U{0} - a < b ? ~U{0} : a + b;
+}
+template <int G, typename U, typename C>
 __device__ __forceinline__ BalanceChoice balance_choice(std::int64_t v, std::int32_t source, std::uint64_t weight,
-                                                        const C* cache, int j, int k, const unsigned long long* pw,
-                                                        std::uint64_t capacity, const PowerTable& powers) {
+                                                        const C* cache, int j, int k, const BalanceTables<U>& tables) {
     const C* row = cache + v * k;
-    unsigned long long slack[kRowSpan];
-    unsigned long long conn = 0, best_slack = 0, current = 0;
+    const U w = sizeof(U) == 4 && weight > 0xffffffffULL ? static_cast<U>(~U{0}) : static_cast<U>(weight);
+    U slack[kRowSpan];
+    U conn = 0, best_slack = 0, current = 0;
     int bp = 0x7fffffff;
-    unsigned long long span[kRowSpan];
+    U span[kRowSpan];
     load_span(row, j, k, span);
     // lane-local best by (conn, slack), lowest index on ties (ascending p)
 #pragma unroll
     for (int e = 0; e < kRowSpan; ++e) {
         const int p = j * kRowSpan + e;
-        const unsigned long long value = span[e];
+        const U value = span[e];
         if (p == source) current = value;
-        const bool ok = p < k && p != source && pw[p] < capacity && weight <= capacity - pw[p];
-        slack[e] = ok ? capacity - pw[p] : 0;
-        if (ok && (bp == 0x7fffffff || value > conn || (value == conn && slack[e] > best_slack))) {
+        const U room = tables.slack[p];
+        const bool ok = p != source && room > 0 && w <= room;
+        slack[e] = ok ? room : 0;
+        if (ok && (bp == 0x7fffffff || value > conn || (value == conn && room > best_slack))) {
             conn = value;
-            best_slack = slack[e];
+            best_slack = room;
             bp = p;
         }
     }
 #pragma unroll
     for (int m = G / 2; m > 0; m /= 2) {
-        const auto oc = shfl_xor_u64(conn, m, G);
-        const auto os = shfl_xor_u64(best_slack, m, G);
+        const U oc = group_xor(conn, m, G);
+        const U os = group_xor(best_slack, m, G);
         const int op = static_cast<int>(lane_xor(static_cast<unsigned>(bp), m, G));
-        const auto ocur = shfl_xor_u64(current, m, G);
+        const U ocur = group_xor(current, m, G);
         const bool ob = op != 0x7fffffff;
         const bool mine = bp != 0x7fffffff;
         if (ob && (!mine || oc > conn || (oc == conn && (os > best_slack || (os == best_slack && op < bp))))) {
@@ -972,31 +1098,27 @@ __device__ __forceinline__ BalanceChoice balance_choice(std::int64_t v, std::int
         // not depend on the order of addition, so the running total before part p
         // is the lane's running prefix plus the saturated total of lower lanes;
         // the walk stops at the first part whose running total exceeds the ticket.
-        unsigned long long running[kRowSpan];
-        unsigned long long lane_total = 0;
+        U running[kRowSpan];
+        U lane_total = 0;
 #pragma unroll
         for (int e = 0; e < kRowSpan; ++e) {
-            lane_total = ~0ULL - lane_total < slack[e] ? ~0ULL : lane_total + slack[e];
+            lane_total = saturated(lane_total, slack[e]);
             running[e] = lane_total;
         }
-        unsigned long long inclusive = lane_total;
+        // the totals of the group's lanes: up to four, exchanged by xor
+        U lower = 0, total = lane_total;
 #pragma unroll
-        for (int d = 1; d < G; d <<= 1) {
-            const auto other = shfl_up_u64(inclusive, d, G);
-            if (j >= d) inclusive = ~0ULL - inclusive < other ? ~0ULL : inclusive + other;
+        for (int m = 1; m < G; m <<= 1) {
+            const U other = group_xor(total, m, G);
+            if (j & m) lower = saturated(lower, other);
+            total = saturated(total, other);
         }
-        const unsigned long long before = G > 1 ? shfl_up_u64(inclusive, 1, G) : 0;
-        const unsigned long long lower = j > 0 ? before : 0;
-        const unsigned long long total = shfl_u64(inclusive, G - 1, G);  // > 0: some part is eligible
         const std::uint32_t hash = mix32(static_cast<std::uint32_t>(v));
-        const unsigned long long ticket =
-            total > 0xffffffffULL ? hash : hash % static_cast<std::uint32_t>(total);
+        const U ticket = sizeof(U) == 8 && total > 0xffffffffULL ? hash : hash % static_cast<std::uint32_t>(total);
         int hit = 0x7fffffff;
 #pragma unroll
-        for (int e = kRowSpan - 1; e >= 0; --e) {
-            const unsigned long long upto = ~0ULL - lower < running[e] ? ~0ULL : lower + running[e];
-            if (upto > ticket) hit = j * kRowSpan + e;
-        }
+        for (int e = kRowSpan - 1; e >= 0; --e)
+            if (saturated(lower, running[e]) > ticket) hit = j * kRowSpan + e;
 #pragma unroll
         for (int m = G / 2; m > 0; m /= 2) {
             const int other = static_cast<int>(lane_xor(static_cast<unsigned>(hit), m, G));
@@ -1009,7 +1131,7 @@ __device__ __forceinline__ BalanceChoice balance_choice(std::int64_t v, std::int
         const double gain =
             conn >= current ? static_cast<double>(conn - current) : -static_cast<double>(current - conn);
         const double per_weight = gain / static_cast<double>(weight);
-        bucket = source * kBalanceWidth + gain_bucket(per_weight, powers) * kBalanceSections +
+        bucket = source * kBalanceWidth + gain_bucket(per_weight, tables.powers) * kBalanceSections +
                  static_cast<int>(mix32(static_cast<std::uint32_t>(v)) % kBalanceSections);
     }
     return BalanceChoice{best, bucket};
@@ -1017,7 +1139,7 @@ __device__ __forceinline__ BalanceChoice balance_choice(std::int64_t v, std::int
 
 // incremental_rebalance_proposals (:111-157) + balance_source_histogram (:174-186).
 // One group of G lanes per candidate, lane j owning parts [8j, 8j + 8).
-template <typename W, int G, typename C>
+template <typename W, int G, typename U, typename C>
 __global__ void __launch_bounds__(kBlock) balance_proposals_kernel(RoundState* st, const std::int32_t* cand,
                                                                    const C* cache,
                                                                    const std::int32_t* labels, const W* vertex_weights,
@@ -1025,13 +1147,13 @@ __global__ void __launch_bounds__(kBlock) balance_proposals_kernel(RoundState* s
                                                                    std::uint64_t capacity, PowerTable powers,
                                                                    std::int32_t* targets, std::int32_t* cbucket,
                                                                    unsigned long long* replicas) {
-    __shared__ unsigned long long pw[32];
+    __shared__ BalanceTables<U> tables;
     __shared__ BucketTable table;
     // the round state past the candidate count starts at zero
     constexpr unsigned kCandidateWord = offsetof(RoundState, candidates) / 8;
     if (blockIdx.x == 0 && threadIdx.x < sizeof(RoundState) / 8 && threadIdx.x != kCandidateWord)
         reinterpret_cast<unsigned long long*>(st)[threadIdx.x] = 0;
-    if (threadIdx.x < 32) pw[threadIdx.x] = threadIdx.x < k ? part_weights[threadIdx.x] : 0;
+    tables.load(part_weights, k, capacity, powers);
     table_clear(table);
     __syncthreads();
     unsigned long long* counts = replicas + static_cast<long long>(blockIdx.x % kReplicas) * k * kBalanceWidth;
@@ -1043,7 +1165,7 @@ __global__ void __launch_bounds__(kBlock) balance_proposals_kernel(RoundState* s
         const std::int64_t v = cand[index];
         const std::int32_t source = labels[v];
         const std::uint64_t weight = static_cast<std::uint64_t>(vertex_weights[v]);
-        const BalanceChoice choice = balance_choice<G, C>(v, source, weight, cache, j, k, pw, capacity, powers);
+        const BalanceChoice choice = balance_choice<G, U>(v, source, weight, cache, j, k, tables);
         if (j == 0) {
             if (choice.bucket >= 0) table_add(table, static_cast<unsigned>(choice.bucket), weight, counts);
             targets[v] = choice.target;
@@ -1071,26 +1193,26 @@ __global__ void __launch_bounds__(kBlock) balance_proposals_kernel(RoundState* s
 constexpr int kNoCandidate = -2;
 constexpr int kBucketBits = 10, kSourceShift = 10, kTargetShift = 15;
 static_assert(kBalanceWidth <= 1 << kBucketBits, "a part's buckets fit their field");
-template <typename W, int G, typename C>
+template <typename W, int G, typename U, typename C>
 __global__ void __launch_bounds__(kBlock) balance_vertices_kernel(RoundState* st, std::int64_t n, const C* cache,
                                                                   const std::int32_t* labels, const W* vertex_weights,
                                                                   int k, const unsigned long long* part_weights,
                                                                   std::uint64_t capacity, PowerTable powers,
                                                                   std::int32_t* targets, std::int32_t* choices,
                                                                   std::int32_t* flags, unsigned char* state) {
-    __shared__ unsigned long long pw[32];
+    __shared__ BalanceTables<U> tables;
     if (blockIdx.x == 0 && threadIdx.x < sizeof(RoundState) / 8)
         reinterpret_cast<unsigned long long*>(st)[threadIdx.x] = 0;
-    if (threadIdx.x < 32) pw[threadIdx.x] = threadIdx.x < static_cast<unsigned>(k) ? part_weights[threadIdx.x] : 0;
+    tables.load(part_weights, k, capacity, powers);
+    const unsigned over = overloaded_parts(part_weights, k, capacity);
     __syncthreads();
     const std::int64_t v = (static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / G;
     if (v >= n) return;  // uniform per group
     const int j = threadIdx.x & (G - 1);
     const std::int32_t source = labels[v];
     BalanceChoice choice{-1, kNoCandidate};
-    if (pw[source] > capacity)  // uniform per group
-        choice = balance_choice<G, C>(v, source, static_cast<std::uint64_t>(vertex_weights[v]), cache, j, k, pw,
-                                      capacity, powers);
+    if (over >> source & 1U)  // uniform per group
+        choice = balance_choice<G, U>(v, source, static_cast<std::uint64_t>(vertex_weights[v]), cache, j, k, tables);
     if (j == 0) {
         targets[v] = choice.target;
         choices[v] = choice.bucket < 0 ? choice.bucket
@@ -1098,6 +1220,55 @@ __global__ void __launch_bounds__(kBlock) balance_vertices_kernel(RoundState* st
                                              (choice.target << kTargetShift);
         flags[v] = 0;
         if (state) state[v] = static_cast<unsigned char>(source);  // refine_rows.hpp
+    }
+}
+
+constexpr int kSelectThreads = 1024;
+constexpr int kSelectWaves = kSelectThreads / kWave;
+
+// What part p's members may weigh: its overload (sources) or its slack (destinations).
+__device__ __forceinline__ unsigned long long part_limit(unsigned long long w, std::uint64_t capacity,
+                                                         bool destinations) {
+    return destinations ? (w < capacity ? capacity - w : 0) : (w > capacity ? w - capacity : 0);
+}
+
+// For parts [base, base + parts), whose buckets' weights are in LDS (narrow, or wide):
+// the boundary bucket, the first at which the running weight reaches the limit, and the
+// weight before it. Members of lower buckets are all taken, those of higher ones refused
+// (source_side and destination_side state the same tests). A wave per part, 13 buckets
+// per lane; called by a workgroup of kSelectThreads threads.
+__device__ void part_boundaries(const unsigned* narrow, const unsigned long long* wide, int base, int parts,
+                                bool destinations, const unsigned long long* pw, std::uint64_t capacity,
+                                int* boundary, unsigned long long* before) {
+    constexpr int kPer = (kBalanceWidth + kWave - 1) / kWave;
+    const int lane = lane_id();
+    for (int q = threadIdx.x / kWave; q < parts; q += kSelectWaves) {
+        const unsigned long long limit = part_limit(pw[base + q], capacity, destinations);
+        if (!destinations && limit == 0) continue;  // not overloaded: no members
+        unsigned long long count[kPer], sum = 0;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int b = lane * kPer + i;
+            count[i] = b >= kBalanceWidth ? 0 : narrow ? narrow[q * kBalanceWidth + b] : wide[q * kBalanceWidth + b];
+            sum += count[i];
+        }
+        unsigned long long running = wave_scan(sum) - sum, at = 0;
+        int found = kBalanceWidth;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const bool reached = destinations ? running + count[i] > limit : running + count[i] >= limit;
+            if (reached && found == kBalanceWidth && lane * kPer + i < kBalanceWidth) {
+                found = lane * kPer + i;
+                at = running;
+            }
+            running += count[i];
+        }
+        const unsigned long long lanes = __ballot(found < kBalanceWidth);
+        const int owner = lanes ? __ffsll(static_cast<unsigned long long>(lanes)) - 1 : 0;
+        if (lane == owner) {
+            boundary[base + q] = found;
+            before[base + q] = at;
+        }
     }
 }
 
@@ -1111,10 +1282,8 @@ __global__ void __launch_bounds__(kBlock) balance_vertices_kernel(RoundState* st
 // taken, those behind it refused (source_side and destination_side state the same
 // tests). That bucket's own members of all parts are gathered in id order into the
 // histogram's space and ranked together, kSelectThreads at a time.
-constexpr int kSelectThreads = 1024;
 constexpr int kSelectMaxItems = 16;
 constexpr std::int64_t kSelectVertices = kSelectThreads * kSelectMaxItems;
-constexpr int kSelectWaves = kSelectThreads / kWave;
 struct SelectShared {
     union {
         unsigned narrow[32 * kBalanceWidth];
@@ -1177,10 +1346,6 @@ __global__ void __launch_bounds__(kSelectThreads) balance_select_kernel(
         in |= static_cast<unsigned>(item[i] >= 0) << i;
     }
 
-    auto threshold = [&](int p, bool destinations) -> unsigned long long {
-        const unsigned long long w = sh.pw[p];
-        return destinations ? (w < capacity ? capacity - w : 0) : (w > capacity ? w - capacity : 0);
-    };
     // Selects among the items in `in`, by the part at `shift`: the mask of the taken.
     auto select = [&](int shift, bool destinations) -> unsigned {
         for (int base = 0; base < k; base += window) {
@@ -1200,38 +1365,8 @@ __global__ void __launch_bounds__(kSelectThreads) balance_select_kernel(
                 else atomicAdd(&sh.u.wide[b], static_cast<unsigned long long>(weight[i]));
             }
             __syncthreads();
-            // a wave per part, 13 buckets per lane
-            constexpr int kPer = (kBalanceWidth + kWave - 1) / kWave;
-            for (int q = wave; q < parts; q += kSelectWaves) {
-                const unsigned long long limit = threshold(base + q, destinations);
-                if (!destinations && limit == 0) continue;  // not overloaded: no members
-                unsigned long long count[kPer], sum = 0;
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int b = lane * kPer + i;
-                    count[i] = b >= kBalanceWidth ? 0
-                               : narrow           ? sh.u.narrow[q * kBalanceWidth + b]
-                                                  : sh.u.wide[q * kBalanceWidth + b];
-                    sum += count[i];
-                }
-                unsigned long long running = wave_scan(sum) - sum, at = 0;
-                int found = kBalanceWidth;
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const bool reached = destinations ? running + count[i] > limit : running + count[i] >= limit;
-                    if (reached && found == kBalanceWidth && lane * kPer + i < kBalanceWidth) {
-                        found = lane * kPer + i;
-                        at = running;
-                    }
-                    running += count[i];
-                }
-                const unsigned long long lanes = __ballot(found < kBalanceWidth);
-                const int owner = lanes ? __ffsll(static_cast<unsigned long long>(lanes)) - 1 : 0;
-                if (lane == owner) {
-                    sh.boundary[base + q] = found;
-                    sh.running[base + q] = at;
-                }
-            }
+            part_boundaries(narrow ? sh.u.narrow : nullptr, sh.u.wide, base, parts, destinations, sh.pw, capacity,
+                            sh.boundary, sh.running);
             __syncthreads();
         }
         unsigned taken = 0, pending = 0;
@@ -1269,7 +1404,7 @@ __global__ void __launch_bounds__(kSelectThreads) balance_select_kernel(
             const unsigned long long w =
                 member ? static_cast<unsigned long long>(vertex_weights[sh.u.pending.vertex[x]]) : 0;
             const unsigned long long rank = block_key_prefix<kSelectThreads>(member, p, w, sh.wave_total, sh.running);
-            const unsigned long long limit = threshold(p, destinations);
+            const unsigned long long limit = part_limit(sh.pw[p], capacity, destinations);
             if (member) sh.u.pending.taken[x] = destinations ? rank + w <= limit : rank < limit;
         }
         __syncthreads();
@@ -1325,279 +1460,371 @@ __global__ void __launch_bounds__(kSelectThreads) balance_select_kernel(
     }
 }
 
-// balance_scan_buckets (:188-202): bucket totals (the kReplicas copies summed),
-// the exclusive sum over the 800 buckets of each part, and the part's threshold:
-// its overload (sources) or slack (destinations).
-// One workgroup per part, a thread per bucket: the 16 replica loads of a thread
-// are independent and all in flight at once.
+// ---------------------------------------------------------------- large levels
+//
+// Larger levels list their candidates, histogram the source buckets while they choose,
+// and then take four launches for the two selections: the sources' boundary buckets, a
+// pass that decides every candidate outside them, a pass that ranks the boundary
+// members and gathers the leaving vertices, and one workgroup that selects among
+// those. Mostly the leaving vertices are few (their weight is about the overload:
+// hundreds to thousands where the candidates are 10^4 to 10^6), so the destinations'
+// histogram, scan, ranks and mover lists take one workgroup 12 us; as launches over
+// the candidates they were four (six above 256 workgroups) of 4.4-6.2 us each. Where
+// the part weights of the last round say that more than kFewLeaving vertices leave, the
+// destinations too are selected by passes over the slices (R-MAT levels move up to a
+// tenth of their vertices at once: 4.2 M vertices, 1.5 against 4.3 ms an iteration).
+constexpr std::int64_t kFewLeaving = 16384;
+
+// balance_scan_buckets (:188-202): the boundary bucket of every overloaded part
+// (sources) or of every part (destinations) and the weight before it, from the
+// kReplicas copies of the counters, which are zeroed for the next round. One workgroup
+// per part, a thread per bucket: its 16 replica loads are independent and all in
+// flight at once.
 constexpr int kBucketScanThreads = 1024;
 static_assert(kBucketScanThreads >= kBalanceWidth, "a thread per bucket");
-static_assert(kRoundBlocks % kBucketScanThreads == 0, "column scan items per thread");
-__global__ void __launch_bounds__(kBucketScanThreads) balance_scan_kernel(unsigned long long* replicas, int k,
-                                                                    unsigned long long* counts,
-                                                                    unsigned long long* offsets,
-                                                                    const unsigned long long* part_weights,
-                                                                    std::uint64_t capacity, bool destinations,
-                                                                    unsigned long long* thresholds) {
+template <bool Destinations>
+__global__ void __launch_bounds__(kBucketScanThreads) bucket_boundaries_kernel(unsigned long long* replicas, int k,
+                                                                               const unsigned long long* part_weights,
+                                                                               std::uint64_t capacity, int* boundary,
+                                                                               unsigned long long* before) {
     __shared__ unsigned long long waves[kBucketScanThreads / kWave + 1];
-    constexpr int kPer = 1;
+    const unsigned long long limit = part_limit(part_weights[blockIdx.x], capacity, Destinations);
+    if (!Destinations && limit == 0) return;  // not overloaded: no members, its counters are zero
     const long long width = static_cast<long long>(k) * kBalanceWidth;
-    unsigned long long items[kPer];
-    unsigned long long local = 0;
+    const int b = threadIdx.x;
+    unsigned long long count = 0;
+    if (b < kBalanceWidth) {
+        unsigned long long* mine = replicas + static_cast<long long>(blockIdx.x) * kBalanceWidth + b;
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const int b = threadIdx.x * kPer + i;
-        unsigned long long total = 0;
-        if (b < kBalanceWidth) {
-            const long long bucket = static_cast<long long>(blockIdx.x) * kBalanceWidth + b;
+        for (int r = 0; r < kReplicas; ++r) count += mine[r * width];
 #pragma unroll
-            for (int r = 0; r < kReplicas; ++r) total += replicas[r * width + bucket];
-#pragma unroll
-            for (int r = 0; r < kReplicas; ++r) replicas[r * width + bucket] = 0;  // zero for the next round
-            counts[bucket] = total;
-        }
-        items[i] = total;
-        local += items[i];
+        for (int r = 0; r < kReplicas; ++r) mine[r * width] = 0;
     }
     unsigned long long total;
-    unsigned long long prefix = block_exclusive_scan(local, SumOp<unsigned long long>{}, &total, waves);
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const int b = threadIdx.x * kPer + i;
-        if (b < kBalanceWidth) offsets[static_cast<std::int64_t>(blockIdx.x) * kBalanceWidth + b] = prefix;
-        prefix += items[i];
+    const unsigned long long prefix = block_exclusive_scan(count, SumOp<unsigned long long>{}, &total, waves);
+    // the first bucket that reaches the limit; kBalanceWidth when none does
+    auto reached = [&](unsigned long long w) { return Destinations ? w > limit : w >= limit; };
+    if (b < kBalanceWidth && reached(prefix + count) && (b == 0 || !reached(prefix))) {
+        boundary[blockIdx.x] = b;
+        before[blockIdx.x] = prefix;
     }
-    if (threadIdx.x == 0) {
-        const unsigned long long w = part_weights[blockIdx.x];
-        thresholds[blockIdx.x] =
-            destinations ? (w < capacity ? capacity - w : 0) : (w > capacity ? w - capacity : 0);
+    if (b == 0 && !reached(total)) {
+        boundary[blockIdx.x] = kBalanceWidth;
+        before[blockIdx.x] = 0;
     }
 }
 
-// balance_select_sources (:204-217) for non-boundary buckets; boundary members
-// are summed per part and workgroup for the multisplit.
+// The selection passes over the candidates: at most kSliceBlocks workgroups, each with
+// one contiguous slice.
+constexpr int kSliceThreads = 1024;
+constexpr int kSliceBlocks = 256;
+
+// balance_select_sources (:204-217) outside the boundary buckets: leaving[i] is the
+// candidate's destination code (bucket | part << kBucketBits), kSourcePending for a
+// boundary member, whose weights are summed per part and workgroup, or kNoBucket.
 template <typename W>
-__global__ void __launch_bounds__(kBlock) balance_sources_kernel(const RoundState* st, const std::int32_t* cand,
-                                                                 const std::int32_t* cbucket, std::int32_t* dbucket,
-                                                                 const std::int32_t* targets,
-                                                                 const W* vertex_weights,
-                                                                 const unsigned long long* counts,
-                                                                 const unsigned long long* offsets,
-                                                                 const unsigned long long* thresholds,
-                                                                 unsigned long long* block_sums,
-                                                                 unsigned long long* dst_replicas, long long width) {
-    __shared__ BucketTable table;
+__global__ void __launch_bounds__(kSliceThreads) balance_sources_kernel(const RoundState* st, const std::int32_t* cand,
+                                                                        const std::int32_t* cbucket,
+                                                                        std::int32_t* leaving,
+                                                                        const std::int32_t* targets,
+                                                                        const W* vertex_weights, const int* boundary,
+                                                                        unsigned long long* block_sums) {
     __shared__ unsigned long long sums[32];
-    unsigned long long* dst_counts = dst_replicas + static_cast<long long>(blockIdx.x % kReplicas) * width;
-    table_clear(table);
-    if (threadIdx.x < 32) sums[threadIdx.x] = 0;
+    __shared__ int bounds[32];
+    if (threadIdx.x < 32) {
+        sums[threadIdx.x] = 0;
+        bounds[threadIdx.x] = boundary[threadIdx.x];  // set for overloaded parts, which all members belong to
+    }
     __syncthreads();
     long long begin, end;
     block_slice(st->candidates, begin, end);
-    for (long long i = begin + threadIdx.x; i < end; i += blockDim.x) {
+    for (long long i = begin + threadIdx.x; i < end; i += kSliceThreads) {
         const int b = cbucket[i];
-        int d = kNoBucket;
+        int code = kNoBucket;
         if (b >= 0) {
-            const int s = b / kBalanceWidth;
-            const std::int32_t v = cand[i];
-            const auto w = static_cast<unsigned long long>(vertex_weights[v]);
-            const BucketSide side = source_side(offsets[b], counts[b], thresholds[s]);
-            if (side == kTaken) {
-                d = targets[v] * kBalanceWidth + b % kBalanceWidth;
-                table_add(table, static_cast<unsigned>(d), w, dst_counts);
-            } else if (side == kBoundary) {
-                d = kSourcePending;
-                atomicAdd(&sums[s], w);
+            const int part = b / kBalanceWidth, bucket = b % kBalanceWidth;
+            if (bucket < bounds[part]) {
+                code = bucket | targets[cand[i]] << kBucketBits;
+            } else if (bucket == bounds[part]) {
+                code = kSourcePending;
+                atomicAdd(&sums[part], static_cast<unsigned long long>(vertex_weights[cand[i]]));
             }
         }
-        dbucket[i] = d;
+        leaving[i] = code;
     }
     __syncthreads();
-    table_flush(table, dst_counts);
     if (threadIdx.x < 32) block_sums[static_cast<long long>(blockIdx.x) * 32 + threadIdx.x] = sums[threadIdx.x];
 }
 
-// Exclusive scan of each part's column of per-workgroup sums (blocks <= 1024).
-__global__ void __launch_bounds__(kBucketScanThreads) column_scan_kernel(const unsigned long long* sums, int blocks,
-                                                                   unsigned long long* prefix) {
-    __shared__ unsigned long long waves[kBucketScanThreads / kWave + 1];
-    constexpr int kPer = kRoundBlocks / kBucketScanThreads;
-    const int column = blockIdx.x;
-    unsigned long long items[kPer];
-    unsigned long long local = 0;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const int b = threadIdx.x * kPer + i;
-        items[i] = b < blocks ? sums[static_cast<long long>(b) * 32 + column] : 0;
-        local += items[i];
+// The boundary weights of the workgroups below this one, per part, on top of the weight
+// before the boundary bucket where the part has a limit. Called by the workgroup.
+constexpr int kSliceRows = kSliceThreads / 32;
+__device__ __forceinline__ void slice_running(const unsigned long long* block_sums, const unsigned long long* before,
+                                              const unsigned long long* part_weights, int k, std::uint64_t capacity,
+                                              bool destinations, unsigned long long (*rows)[32],
+                                              unsigned long long* running, unsigned long long* limits) {
+    const int part = threadIdx.x & 31, row = threadIdx.x >> 5;
+    unsigned long long sum = 0;
+    for (int b = row; b < static_cast<int>(blockIdx.x); b += kSliceRows)
+        sum += block_sums[static_cast<long long>(b) * 32 + part];
+    rows[row][part] = sum;
+    __syncthreads();
+    if (threadIdx.x < 32) {
+        const bool is = threadIdx.x < static_cast<unsigned>(k);
+        const unsigned long long limit =
+            is ? part_limit(part_weights[threadIdx.x], capacity, destinations) : 0;
+        limits[threadIdx.x] = limit;
+        unsigned long long total = is && (destinations || limit) ? before[threadIdx.x] : 0;
+        for (int r = 0; r < kSliceRows; ++r) total += rows[r][threadIdx.x];
+        running[threadIdx.x] = total;
     }
-    unsigned long long total;
-    unsigned long long running = block_exclusive_scan(local, SumOp<unsigned long long>{}, &total, waves);
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const int b = threadIdx.x * kPer + i;
-        if (b < blocks) prefix[static_cast<long long>(b) * 32 + column] = running;
-        running += items[i];
-    }
+    __syncthreads();
 }
 
-// The exclusive prefix over the workgroups before this one of each of the 32
-// columns of block_sums (a row of 32 per workgroup) into running[]: read from
-// column_prefix when the column scan ran, else summed here from the rows, which
-// grids of at most kInlineColumnBlocks workgroups do instead of that launch
-// (thread t sums column t % 32 over the rows t / 32, t / 32 + 8, ...).
-constexpr int kInlineColumnBlocks = 256;
-__device__ __forceinline__ void column_running(const unsigned long long* column_prefix,
-                                               const unsigned long long* block_sums, unsigned long long* running,
-                                               unsigned long long (*groups)[32]) {
-    static_assert(kBlock == 256, "8 row groups of 32 columns");
-    if (column_prefix) {
-        if (threadIdx.x < 32)
-            running[threadIdx.x] = column_prefix[static_cast<long long>(blockIdx.x) * 32 + threadIdx.x];
-    } else {
-        const int column = threadIdx.x & 31, group = threadIdx.x >> 5;
-        unsigned long long sum = 0;
-        for (int row = group; row < static_cast<int>(blockIdx.x); row += kBlock / 32)
-            sum += block_sums[static_cast<long long>(row) * 32 + column];
-        groups[group][column] = sum;
+// Source boundary members: they leave while the weight before the bucket plus their
+// rank is below the overload. The slice's leaving vertices are gathered, in id order,
+// at the front of its range of left_vertex and left_code. Table: their weights are also
+// added to the destination buckets' counters.
+template <typename W, bool Table>
+__global__ void __launch_bounds__(kSliceThreads) balance_source_ranks_kernel(
+    const RoundState* st, const std::int32_t* cand, const std::int32_t* cbucket, const std::int32_t* leaving,
+    const std::int32_t* targets, const W* vertex_weights, const unsigned long long* part_weights, int k,
+    std::uint64_t capacity, const unsigned long long* before, const unsigned long long* block_sums,
+    std::int32_t* left_vertex, std::int32_t* left_code, std::int32_t* left_count, unsigned long long* replicas) {
+    constexpr int kWaves = kSliceThreads / kWave;
+    __shared__ unsigned long long wave_total[kWaves][32];
+    __shared__ unsigned long long running[32], limits[32];
+    __shared__ unsigned long long rows[kSliceRows][32];
+    __shared__ int wave_left[2][kWaves];
+    __shared__ std::conditional_t<Table, BucketTable, int> table;
+    unsigned long long* counts = replicas + static_cast<long long>(blockIdx.x % kReplicas) * k * kBalanceWidth;
+    if constexpr (Table) table_clear(table);
+    slice_running(block_sums, before, part_weights, k, capacity, false, rows, running, limits);
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    long long begin, end;
+    block_slice(st->candidates, begin, end);
+    int left = 0, turn = 0;
+    for (long long base = begin; base < end; base += kSliceThreads) {
+        const long long i = base + threadIdx.x;
+        int code = i < end ? leaving[i] : kNoBucket;
+        const bool pending = code == kSourcePending;
+        if (!__syncthreads_or(code != kNoBucket)) continue;
+        if (__syncthreads_or(pending)) {
+            const int b = pending ? cbucket[i] : 0, part = b / kBalanceWidth;
+            const std::int32_t v = pending ? cand[i] : 0;
+            const unsigned long long w = pending ? static_cast<unsigned long long>(vertex_weights[v]) : 0;
+            const unsigned long long rank = block_key_prefix<kSliceThreads>(pending, part, w, wave_total, running);
+            if (pending) code = rank < limits[part] ? b % kBalanceWidth | targets[v] << kBucketBits : kNoBucket;
+        }
+        const unsigned long long lanes = __ballot(code >= 0);
+        if (lane == 0) wave_left[turn][wave] = __popcll(lanes);
         __syncthreads();
-        if (threadIdx.x < 32) {
-            unsigned long long total = 0;
-#pragma unroll
-            for (int g = 0; g < kBlock / 32; ++g) total += groups[g][threadIdx.x];
-            running[threadIdx.x] = total;
+        int at = left;
+        for (int w = 0; w < kWaves; ++w) {
+            if (w < wave) at += wave_left[turn][w];
+            left += wave_left[turn][w];
         }
+        turn ^= 1;
+        if (code >= 0) {
+            at += __popcll(lanes & lanemask_lt());
+            const std::int32_t v = cand[i];
+            left_vertex[begin + at] = v;
+            left_code[begin + at] = code;
+            if constexpr (Table)
+                table_add(table,
+                          static_cast<unsigned>((code >> kBucketBits) * kBalanceWidth + (code & ((1 << kBucketBits) - 1))),
+                          static_cast<unsigned long long>(vertex_weights[v]), counts);
+        }
+    }
+    if (threadIdx.x == 0) left_count[blockIdx.x] = left;
+    if constexpr (Table) {
+        __syncthreads();
+        table_flush(table, counts);
     }
 }
 
-// Source boundary members: taken while offset + rank < overload.
-template <typename W>
-__global__ void __launch_bounds__(kBlock) balance_source_ranks_kernel(const RoundState* st, const std::int32_t* cand,
-                                                                      const std::int32_t* cbucket,
-                                                                      std::int32_t* dbucket,
-                                                                      const std::int32_t* targets,
-                                                                      const W* vertex_weights,
-                                                                      const unsigned long long* offsets,
-                                                                      const unsigned long long* thresholds,
-                                                                      const unsigned long long* column_prefix,
-                                                                      const unsigned long long* block_sums,
-                                                                      unsigned long long* dst_replicas,
-                                                                      long long width) {
-    __shared__ BucketTable table;
-    unsigned long long* dst_counts = dst_replicas + static_cast<long long>(blockIdx.x % kReplicas) * width;
-    __shared__ unsigned long long wave_total[kBlock / kWave][32];
-    __shared__ unsigned long long running[32];
-    __shared__ unsigned long long groups[kBlock / 32][32];
-    table_clear(table);
-    column_running(column_prefix, block_sums, running, groups);
-    __syncthreads();
-    long long begin, end;
-    block_slice(st->candidates, begin, end);
-    for (long long base = begin; base < end; base += blockDim.x) {
-        const long long i = base + threadIdx.x;
-        const bool pending = i < end && dbucket[i] == kSourcePending;
-        if (!__syncthreads_or(pending)) continue;
-        int b = 0, s = 0;
-        std::int32_t v = 0;
-        unsigned long long w = 0;
-        if (pending) {
-            b = cbucket[i];
-            s = b / kBalanceWidth;
-            v = cand[i];
-            w = static_cast<unsigned long long>(vertex_weights[v]);
-        }
-        const unsigned long long rank = block_key_prefix<kBlock>(pending, s, w, wave_total, running);
-        if (pending) {
-            if (offsets[b] + rank < thresholds[s]) {
-                const int d = targets[v] * kBalanceWidth + b % kBalanceWidth;
-                dbucket[i] = d;
-                table_add(table, static_cast<unsigned>(d), w, dst_counts);
-            } else {
-                dbucket[i] = kNoBucket;
-            }
-        }
-    }
-    __syncthreads();
-    table_flush(table, dst_counts);
-}
-
-// balance_select_destinations (:219-232) for non-boundary buckets: taken ones
-// become movers; boundary members are summed for the multisplit.
-template <typename O, typename W>
-__global__ void __launch_bounds__(kBlock) balance_destinations_kernel(
-    RoundState* st, const std::int32_t* cand, std::int32_t* dbucket, const W* vertex_weights, const O* offsets_csr,
-    const unsigned long long* counts, const unsigned long long* offsets, const unsigned long long* thresholds,
-    unsigned long long* block_sums, const std::int32_t* labels, std::int32_t* light, std::int32_t* heavy,
+// balance_select_destinations (:219-232) over the slices' leaving vertices, in two
+// passes. Ranks == false: those of buckets below the boundary move, the boundary
+// members' weights are summed per part and workgroup. Ranks == true: boundary members
+// move while the weight before the bucket, their rank and their own weight fit.
+template <typename O, typename W, bool Ranks>
+__global__ void __launch_bounds__(kSliceThreads) balance_slices_kernel(
+    RoundState* st, const std::int32_t* left_vertex, const std::int32_t* left_code, const std::int32_t* left_count,
+    const std::int32_t* labels, const W* vertex_weights, const O* offsets, int k,
+    const unsigned long long* part_weights, std::uint64_t capacity, const int* boundary,
+    const unsigned long long* before, unsigned long long* block_sums, std::int32_t* light, std::int32_t* heavy,
     std::int32_t* flags, unsigned char* state) {
-    __shared__ unsigned long long sums[32];
-    __shared__ unsigned counts_lds[2 * (kBlock / kWave)];
-    __shared__ unsigned long long base_lds[2];
-    if (threadIdx.x < 32) sums[threadIdx.x] = 0;
-    __syncthreads();
-    long long begin, end;
-    block_slice(st->candidates, begin, end);
-    for (long long base = begin; base < end; base += blockDim.x) {
-        const long long i = base + threadIdx.x;
-        bool take = false;
-        std::int32_t v = 0;
-        if (i < end) {
-            const int d = dbucket[i];
-            if (d >= 0) {
-                const int part = d / kBalanceWidth;
-                v = cand[i];
-                const BucketSide side = destination_side(offsets[d], counts[d], thresholds[part]);
-                if (side == kTaken) {
-                    take = true;
-                    flags[v] = labels[v] + 1;
-                    mark_mover(state, v, part);
-                } else if (side == kBoundary) {
-                    dbucket[i] = -3 - d;
-                    atomicAdd(&sums[part], static_cast<unsigned long long>(vertex_weights[v]));
-                }
-            }
-        }
-        append_movers(take, v, offsets_csr, light, heavy, st, counts_lds, base_lds);
+    constexpr int kWaves = kSliceThreads / kWave;
+    __shared__ unsigned long long wave_total[kWaves][32];
+    __shared__ unsigned long long running[32], limits[32];
+    __shared__ unsigned long long rows[kSliceRows][32];
+    __shared__ int bounds[32];
+    __shared__ unsigned counts[2 * kWaves];
+    __shared__ unsigned long long bases[2];
+    if (threadIdx.x < 32) bounds[threadIdx.x] = threadIdx.x < static_cast<unsigned>(k) ? boundary[threadIdx.x] : 0;
+    if constexpr (Ranks) {
+        slice_running(block_sums, before, part_weights, k, capacity, true, rows, running, limits);
+    } else {
+        if (threadIdx.x < 32) running[threadIdx.x] = 0;  // the workgroup's sums
+        __syncthreads();
     }
-    if (threadIdx.x < 32) block_sums[static_cast<long long>(blockIdx.x) * 32 + threadIdx.x] = sums[threadIdx.x];
-}
-
-// Destination boundary members: admitted while offset + rank + weight <= slack.
-template <typename O, typename W>
-__global__ void __launch_bounds__(kBlock) balance_destination_ranks_kernel(
-    RoundState* st, const std::int32_t* cand, const std::int32_t* dbucket, const W* vertex_weights,
-    const O* offsets_csr, const unsigned long long* offsets, const unsigned long long* thresholds,
-    const unsigned long long* column_prefix, const unsigned long long* block_sums, const std::int32_t* labels,
-    std::int32_t* light, std::int32_t* heavy, std::int32_t* flags, unsigned char* state) {
-    __shared__ unsigned long long wave_total[kBlock / kWave][32];
-    __shared__ unsigned long long running[32];
-    __shared__ unsigned long long groups[kBlock / 32][32];
-    __shared__ unsigned counts_lds[2 * (kBlock / kWave)];
-    __shared__ unsigned long long base_lds[2];
-    column_running(column_prefix, block_sums, running, groups);
-    __syncthreads();
     long long begin, end;
     block_slice(st->candidates, begin, end);
-    for (long long base = begin; base < end; base += blockDim.x) {
+    end = begin + left_count[blockIdx.x];
+    for (long long base = begin; base < end; base += kSliceThreads) {
         const long long i = base + threadIdx.x;
-        const int code = i < end ? dbucket[i] : kNoBucket;
-        const bool pending = code <= -3;
-        if (!__syncthreads_or(pending)) continue;
-        int d = 0, part = 0;
         std::int32_t v = 0;
-        unsigned long long w = 0;
-        if (pending) {
-            d = -3 - code;
-            part = d / kBalanceWidth;
-            v = cand[i];
-            w = static_cast<unsigned long long>(vertex_weights[v]);
+        int part = 0;
+        bool take = false, pending = false;
+        if (i < end) {
+            const int code = left_code[i], bucket = code & ((1 << kBucketBits) - 1);
+            part = code >> kBucketBits;
+            pending = bucket == bounds[part];
+            take = !Ranks && bucket < bounds[part];
+            if (take || pending) v = left_vertex[i];
         }
-        const unsigned long long rank = block_key_prefix<kBlock>(pending, part, w, wave_total, running);
-        const bool take = pending && offsets[d] + rank + w <= thresholds[part];
+        const unsigned long long w = pending ? static_cast<unsigned long long>(vertex_weights[v]) : 0;
+        if constexpr (Ranks) {
+            if (!__syncthreads_or(pending)) continue;
+            const unsigned long long rank = block_key_prefix<kSliceThreads>(pending, part, w, wave_total, running);
+            take = pending && rank + w <= limits[part];
+        } else if (pending) {
+            atomicAdd(&running[part], w);
+        }
         if (take) {
             flags[v] = labels[v] + 1;
             mark_mover(state, v, part);
         }
-        append_movers(take, v, offsets_csr, light, heavy, st, counts_lds, base_lds);
+        append_movers<kSliceThreads>(take, v, offsets, light, heavy, st, counts, bases);
+    }
+    if constexpr (!Ranks) {
+        __syncthreads();
+        if (threadIdx.x < 32) block_sums[static_cast<long long>(blockIdx.x) * 32 + threadIdx.x] = running[threadIdx.x];
+    }
+}
+
+// balance_select_destinations (:219-232) over all leaving vertices, by one workgroup: the
+// destination buckets' weights in LDS (as in balance_select_kernel), their boundary
+// buckets, then the vertices in id order, kSelectThreads at a time: those of lower
+// buckets move, boundary members while the weight before the bucket, their rank and
+// their own weight fit the slack.
+struct DestinationShared {
+    union {
+        unsigned narrow[32 * kBalanceWidth];
+        unsigned long long wide[16 * kBalanceWidth];
+    } u;
+    unsigned long long pw[32];
+    unsigned long long running[32];
+    int boundary[32];
+    unsigned long long wave_total[kSelectWaves][32];
+    int first[kSliceBlocks];  // of each slice's vertices in the order of all
+    int waves[kSelectWaves];
+    unsigned light, heavy;
+    unsigned long long edges;
+};
+template <typename O, typename W>
+__global__ void __launch_bounds__(kSelectThreads) balance_destinations_kernel(
+    RoundState* st, int slices, const std::int32_t* left_vertex, const std::int32_t* left_code,
+    const std::int32_t* left_count, const std::int32_t* labels, const W* vertex_weights, const O* offsets, int k,
+    const unsigned long long* part_weights, std::uint64_t capacity, std::int32_t* light, std::int32_t* heavy,
+    std::int32_t* flags, unsigned char* state) {
+    __shared__ DestinationShared sh;
+    const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
+    const long long candidates = st->candidates, per = (candidates + slices - 1) / slices;
+    const int mine = t < slices ? left_count[t] : 0;
+    if (t < 32) sh.pw[t] = t < k ? part_weights[t] : 0;
+    if (t == 0) {
+        sh.light = sh.heavy = 0;
+        sh.edges = 0;
+    }
+    const int inclusive = wave_scan(mine);
+    if (lane == kWave - 1) sh.waves[wave] = inclusive;
+    __syncthreads();
+    int below = 0, count = 0;
+    for (int w = 0; w < kSelectWaves; ++w) {
+        if (w == wave) below = count;
+        count += sh.waves[w];
+    }
+    if (t < kSliceBlocks) sh.first[t] = below + inclusive - mine;
+    unsigned long long total = 0;
+    for (int p = 0; p < k; ++p) total += sh.pw[p];
+    const bool narrow = total <= 0xffffffffULL;
+    const int window = narrow ? 32 : 16;
+    __syncthreads();
+    // the x-th leaving vertex: in the last slice that starts at or before it
+    auto locate = [&](int x) -> long long {
+        int lo = 0;
+#pragma unroll
+        for (int step = kSliceBlocks / 2; step > 0; step /= 2)
+            if (sh.first[lo + step] <= x) lo += step;
+        return lo * per + (x - sh.first[lo]);
+    };
+    for (int base = 0; base < k; base += window) {
+        const int parts = min(window, k - base);
+        if (narrow) {
+            for (int b = t; b < parts * kBalanceWidth; b += kSelectThreads) sh.u.narrow[b] = 0;
+        } else {
+            for (int b = t; b < parts * kBalanceWidth; b += kSelectThreads) sh.u.wide[b] = 0;
+        }
+        __syncthreads();
+        for (int x = t; x < count; x += kSelectThreads) {
+            const long long i = locate(x);
+            const int code = left_code[i], q = (code >> kBucketBits) - base;
+            if (q < 0 || q >= parts) continue;
+            const auto w = static_cast<unsigned long long>(vertex_weights[left_vertex[i]]);
+            const int b = q * kBalanceWidth + (code & ((1 << kBucketBits) - 1));
+            if (narrow) atomicAdd(&sh.u.narrow[b], static_cast<unsigned>(w));
+            else atomicAdd(&sh.u.wide[b], w);
+        }
+        __syncthreads();
+        part_boundaries(narrow ? sh.u.narrow : nullptr, sh.u.wide, base, parts, true, sh.pw, capacity, sh.boundary,
+                        sh.running);
+        __syncthreads();
+    }
+    unsigned long long edges = 0;
+    for (int start = 0; start < count; start += kSelectThreads) {
+        const int x = start + t;
+        int part = 0, v = 0;
+        bool take = false, pending = false;
+        if (x < count) {
+            const long long i = locate(x);
+            const int code = left_code[i], bucket = code & ((1 << kBucketBits) - 1);
+            v = left_vertex[i];
+            part = code >> kBucketBits;
+            take = bucket < sh.boundary[part];
+            pending = bucket == sh.boundary[part];
+        }
+        if (__syncthreads_or(pending)) {
+            const unsigned long long w = pending ? static_cast<unsigned long long>(vertex_weights[v]) : 0;
+            const unsigned long long rank = block_key_prefix<kSelectThreads>(pending, part, w, sh.wave_total, sh.running);
+            if (pending) take = rank + w <= part_limit(sh.pw[part], capacity, true);
+        }
+        const unsigned long long degree =
+            take ? static_cast<unsigned long long>(offsets[v + 1] - offsets[v]) : 0;
+        const unsigned long long bh = __ballot(take && degree > kHeavyDegree);
+        const unsigned long long bl = __ballot(take && degree <= kHeavyDegree);
+        unsigned at_light = 0, at_heavy = 0;
+        if (lane == 0) {
+            if (bl) at_light = atomicAdd(&sh.light, static_cast<unsigned>(__popcll(bl)));
+            if (bh) at_heavy = atomicAdd(&sh.heavy, static_cast<unsigned>(__popcll(bh)));
+        }
+        at_light = read_lane(at_light, 0);
+        at_heavy = read_lane(at_heavy, 0);
+        edges += degree;
+        if (take) {
+            if (degree > kHeavyDegree) heavy[at_heavy + __popcll(bh & lanemask_lt())] = v;
+            else light[at_light + __popcll(bl & lanemask_lt())] = v;
+            flags[v] = labels[v] + 1;
+            mark_mover(state, v, part);
+        }
+    }
+    edges = group_sum_u64<kWave>(edges);
+    if (lane == 0 && edges) atomicAdd(&sh.edges, edges);
+    __syncthreads();
+    if (t == 0) {
+        st->light = sh.light;
+        st->heavy = sh.heavy;
+        st->edges = static_cast<long long>(sh.edges);
     }
 }
 
@@ -2111,7 +2338,7 @@ struct Ops {
         out->cut_delta = h.delta;
         out->candidates = h.candidates;
         out->max_part_weight = h.max_weight;
-        for (int p = 0; p < 32; ++p) out->part_weights[p] = p < k ? h.pw[p] : 0;
+        for (int p = 0; p < 32; ++p) ctx->round_part_weights[p] = out->part_weights[p] = p < k ? h.pw[p] : 0;
         out->mover_entries = h.edges;
         const long long rebuild_above = rows_form ? -1 : rebuild_threshold(ctx, g);
         out->rebuilt = rebuild_above >= 0 && h.edges > rebuild_above ? 1 : 0;
@@ -2210,6 +2437,35 @@ struct Ops {
         return key;
     }
 
+    // Calls launch(lanes per row, a value of balance_choice's U): 32 bits when 4-byte
+    // cache entries and k parts of the capacity fit them.
+    template <typename Launch>
+    static void choose(int k, std::uint64_t capacity, Launch&& launch) {
+        auto with = [&](auto slack) {
+            switch (group_for_k(k)) {
+                case 1: launch(std::integral_constant<int, 1>{}, slack); break;
+                case 2: launch(std::integral_constant<int, 2>{}, slack); break;
+                default: launch(std::integral_constant<int, 4>{}, slack); break;
+            }
+        };
+        if constexpr (sizeof(C) == 4) {
+            if (capacity <= 0xffffffffULL / static_cast<unsigned>(k)) return with(unsigned{0});
+        }
+        with(0ULL);
+    }
+
+    // About how many vertices leave their parts in the next rebalance iteration, from the
+    // part weights of the context's last round (a wrong guess costs time only).
+    static std::int64_t expected_leaving(const gpart_ctx* ctx, std::int64_t n, int k, std::uint64_t capacity) {
+        double overload = 0, total = 0;
+        for (int p = 0; p < k; ++p) {
+            const auto w = ctx->round_part_weights[p];
+            total += static_cast<double>(w);
+            if (w > capacity) overload += static_cast<double>(w - capacity);
+        }
+        return total > 0 ? static_cast<std::int64_t>(overload / total * static_cast<double>(n)) : 0;
+    }
+
     // A rebalance iteration of a small level (balance_vertices_kernel,
     // balance_select_kernel, update).
     static void rebalance_round_small(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
@@ -2225,21 +2481,18 @@ struct Ops {
         Scratch<RoundState> st(ctx, 1);
         Scratch<std::int32_t> choices(ctx, n), light(ctx, n), heavy(ctx, n);
         unsigned char* state = r ? r->states.get() : nullptr;
-        const int G = group_for_k(k);
         if (r)
             run.phase(GPART_PROFILE_REFINE_CACHE,
                       [&] { rows(ctx, g, c, r, k, cache, part_weights, capacity); });
         run.phase(GPART_PROFILE_REBALANCE, [&] {
             profile_begin(ctx, GPART_PROFILE_REBALANCE);
-#define GPART_BALANCE_VERTICES(GG)                                                                                 \
-    hipLaunchKernelGGL((balance_vertices_kernel<W, GG, C>), dim3(grid_for(n * GG)), dim3(kBlock), 0, ctx->stream, \
-                       st.get(), n, cache, labels, vw, k, part_weights, capacity, powers, targets, choices.get(), flags, state)
-            switch (G) {
-                case 1: GPART_BALANCE_VERTICES(1); break;
-                case 2: GPART_BALANCE_VERTICES(2); break;
-                default: GPART_BALANCE_VERTICES(4); break;
-            }
-#undef GPART_BALANCE_VERTICES
+            choose(k, capacity, [&](auto group, auto slack) {
+                constexpr int kG = decltype(group)::value;
+                using U = decltype(slack);
+                hipLaunchKernelGGL((balance_vertices_kernel<W, kG, U, C>), dim3(grid_for(n * kG)), dim3(kBlock), 0,
+                                   ctx->stream, st.get(), n, cache, labels, vw, k, part_weights, capacity, powers, targets,
+                                   choices.get(), flags, state);
+            });
             GPART_LAUNCH_CHECK();
             profile_end(ctx, GPART_PROFILE_REBALANCE, 0.0);
         });
@@ -2292,9 +2545,9 @@ struct Ops {
         const auto* off = static_cast<const O*>(g->offsets);
         const auto* vw = static_cast<const W*>(g->vertex_weights);
         const std::int64_t width = static_cast<std::int64_t>(k) * kBalanceWidth;
-        // Both replica arrays live in the context between rounds and are zero at rest
-        // (the bucket scans clear what they read); the proposals kernel zeroes the
-        // round state after the candidate count.
+        // Both replica arrays live in the context between rounds and are zero at rest (the
+        // boundary search clears what it reads); the proposals kernel zeroes the round
+        // state after the candidate count.
         const std::size_t counter_bytes = static_cast<std::size_t>(2 * kReplicas * width) * 8;
         if (ctx->rebalance_counter_bytes < counter_bytes) {
             if (ctx->rebalance_counters) ctx_free(ctx, ctx->rebalance_counters);
@@ -2306,76 +2559,86 @@ struct Ops {
         }
         if (!ctx->rebalance_counters_zero) fill_bytes(ctx, ctx->rebalance_counters, 0, ctx->rebalance_counter_bytes);
         ctx->rebalance_counters_zero = false;  // until this round completes
+        const bool few = expected_leaving(ctx, n, k, capacity) <= kFewLeaving;
         RoundRun run(ctx, round_plan(ctx, n, round_key(ctx, g, c, cache, labels, k, targets, flags, part_weights, r,
-                                                       {1, capacity, key_of(ctx->rebalance_counters)})));
+                                                       {1, capacity, few, key_of(ctx->rebalance_counters)})));
         Scratch<RoundState> st(ctx, 1);
-        Scratch<unsigned long long> counts(ctx, 2 * width), offsets(ctx, 2 * width), thresholds(ctx, 64);
         auto* st_ptr = st.get();
-        auto* src_replicas = static_cast<unsigned long long*>(ctx->rebalance_counters);
-        unsigned long long* dst_replicas = src_replicas + kReplicas * width;
-        unsigned long long* src_counts = counts.get();
-        unsigned long long* dst_counts = counts.get() + width;
-        unsigned long long* src_offsets = offsets.get();
-        unsigned long long* dst_offsets = offsets.get() + width;
-        unsigned long long* src_thresholds = thresholds.get();
-        unsigned long long* dst_thresholds = thresholds.get() + 32;
-        Scratch<std::int32_t> cand(ctx, n), cbucket(ctx, n), dbucket(ctx, n), light(ctx, n), heavy(ctx, n);
-        const int slices = static_cast<int>(std::max<std::int64_t>(1, std::min<std::int64_t>(grid_for(n), kRoundBlocks)));
-        Scratch<unsigned long long> sums(ctx, static_cast<std::int64_t>(slices) * 32),
-            prefix(ctx, static_cast<std::int64_t>(slices) * 32);
-        // small grids sum the per-workgroup boundary weights in the ranks kernels
+        auto* replicas = static_cast<unsigned long long*>(ctx->rebalance_counters);
+        unsigned long long* destination_replicas = replicas + kReplicas * width;
+        Scratch<std::int32_t> cand(ctx, n), cbucket(ctx, n), leaving(ctx, n), left_vertex(ctx, n), left_code(ctx, n),
+            light(ctx, n), heavy(ctx, n), left_count(ctx, kSliceBlocks), tile_counts(ctx, kCandidateTiles);
+        const int slices =
+            static_cast<int>(std::min<std::int64_t>((n + kSliceThreads - 1) / kSliceThreads, kSliceBlocks));
+        Scratch<unsigned long long> sums(ctx, std::int64_t{kSliceBlocks} * 32), before(ctx, 32);
+        Scratch<int> boundary(ctx, 32);
         unsigned char* state = r ? r->states.get() : nullptr;
-        const bool inline_columns = slices <= kInlineColumnBlocks;
-        const unsigned long long* column_prefix = inline_columns ? nullptr : prefix.get();
 
         run.phase(-1, [&] {
-            device_scan<int, SumOp<int>>(ctx, OverloadedLoad{labels, part_weights, capacity},
-                                         CandidateStore{cand.get(), flags, labels, state, n, st_ptr}, n, SumOp<int>{});
+            auto listed = [&](auto items) {
+                constexpr int kItems = decltype(items)::value;
+                const auto tiles = static_cast<unsigned>((n + kBlock * kItems - 1) / (kBlock * kItems));
+                hipLaunchKernelGGL(candidate_count_kernel<kItems>, dim3(tiles), dim3(kBlock), 0, ctx->stream, n, labels,
+                                   part_weights, k, capacity, tile_counts.get());
+                hipLaunchKernelGGL(candidate_list_kernel<kItems>, dim3(tiles), dim3(kBlock), 0, ctx->stream, st_ptr, n,
+                                   labels, part_weights, k, capacity, tile_counts.get(), cand.get(), flags, state);
+                GPART_LAUNCH_CHECK();
+            };
+            if (n <= kCandidateTiles * kBlock * 8)
+                listed(std::integral_constant<int, 8>{});
+            else if (n <= kCandidateTiles * kBlock * 32)
+                listed(std::integral_constant<int, 32>{});
+            else
+                device_scan<int, SumOp<int>>(ctx, OverloadedLoad{labels, part_weights, capacity},
+                                             CandidateStore{cand.get(), flags, labels, state, n, st_ptr}, n,
+                                             SumOp<int>{});
         });
-        const int G = group_for_k(k);
-        const auto blocks = static_cast<unsigned>(std::min<std::int64_t>(grid_for(n * G), ctx->balance_blocks));
+        const auto blocks = static_cast<unsigned>(std::min<std::int64_t>(grid_for(n * group_for_k(k)), ctx->balance_blocks));
         if (r)
             run.phase(GPART_PROFILE_REFINE_CACHE,
                       [&] { rows(ctx, g, c, r, k, cache, part_weights, capacity); });
         run.phase(GPART_PROFILE_REBALANCE, [&] {
-        profile_begin(ctx, GPART_PROFILE_REBALANCE);
-#define GPART_BALANCE_PROPOSALS(GG)                                                                              \
-    hipLaunchKernelGGL((balance_proposals_kernel<W, GG, C>), dim3(blocks), dim3(kBlock), 0, ctx->stream, st_ptr,   \
-                       cand.get(), cache, labels, vw, k, part_weights, capacity, powers, targets, cbucket.get(), \
-                       src_replicas)
-        switch (G) {
-            case 1: GPART_BALANCE_PROPOSALS(1); break;
-            case 2: GPART_BALANCE_PROPOSALS(2); break;
-            default: GPART_BALANCE_PROPOSALS(4); break;
-        }
-#undef GPART_BALANCE_PROPOSALS
-        GPART_LAUNCH_CHECK();
-        profile_end(ctx, GPART_PROFILE_REBALANCE, 0.0);
+            profile_begin(ctx, GPART_PROFILE_REBALANCE);
+            choose(k, capacity, [&](auto group, auto slack) {
+                constexpr int kG = decltype(group)::value;
+                using U = decltype(slack);
+                hipLaunchKernelGGL((balance_proposals_kernel<W, kG, U, C>), dim3(blocks), dim3(kBlock), 0, ctx->stream,
+                                   st_ptr, cand.get(), cache, labels, vw, k, part_weights, capacity, powers, targets,
+                                   cbucket.get(), replicas);
+            });
+            GPART_LAUNCH_CHECK();
+            profile_end(ctx, GPART_PROFILE_REBALANCE, 0.0);
         });
         run.phase(-1, [&] {
-        hipLaunchKernelGGL(balance_scan_kernel, dim3(k), dim3(kBucketScanThreads), 0, ctx->stream, src_replicas, k,
-                           src_counts, src_offsets, part_weights, capacity, false, src_thresholds);
-        hipLaunchKernelGGL(balance_sources_kernel<W>, dim3(slices), dim3(kBlock), 0, ctx->stream, st_ptr,
-                           cand.get(), cbucket.get(), dbucket.get(), targets, vw, src_counts, src_offsets,
-                           src_thresholds, sums.get(), dst_replicas, width);
-        if (!inline_columns)
-            hipLaunchKernelGGL(column_scan_kernel, dim3(k), dim3(kBucketScanThreads), 0, ctx->stream, sums.get(),
-                               slices, prefix.get());
-        hipLaunchKernelGGL(balance_source_ranks_kernel<W>, dim3(slices), dim3(kBlock), 0, ctx->stream, st_ptr,
-                           cand.get(), cbucket.get(), dbucket.get(), targets, vw, src_offsets, src_thresholds,
-                           column_prefix, sums.get(), dst_replicas, width);
-        hipLaunchKernelGGL(balance_scan_kernel, dim3(k), dim3(kBucketScanThreads), 0, ctx->stream, dst_replicas, k,
-                           dst_counts, dst_offsets, part_weights, capacity, true, dst_thresholds);
-        hipLaunchKernelGGL((balance_destinations_kernel<O, W>), dim3(slices), dim3(kBlock), 0, ctx->stream,
-                           st_ptr, cand.get(), dbucket.get(), vw, off, dst_counts, dst_offsets, dst_thresholds,
-                           sums.get(), labels, light.get(), heavy.get(), flags, state);
-        if (!inline_columns)
-            hipLaunchKernelGGL(column_scan_kernel, dim3(k), dim3(kBucketScanThreads), 0, ctx->stream, sums.get(),
-                               slices, prefix.get());
-        hipLaunchKernelGGL((balance_destination_ranks_kernel<O, W>), dim3(slices), dim3(kBlock), 0, ctx->stream,
-                           st_ptr, cand.get(), dbucket.get(), vw, off, dst_offsets, dst_thresholds, column_prefix,
-                           sums.get(), labels, light.get(), heavy.get(), flags, state);
-        GPART_LAUNCH_CHECK();
+            hipLaunchKernelGGL(bucket_boundaries_kernel<false>, dim3(k), dim3(kBucketScanThreads), 0, ctx->stream, replicas, k,
+                               part_weights, capacity, boundary.get(), before.get());
+            hipLaunchKernelGGL(balance_sources_kernel<W>, dim3(slices), dim3(kSliceThreads), 0, ctx->stream, st_ptr,
+                               cand.get(), cbucket.get(), leaving.get(), targets, vw, boundary.get(), sums.get());
+            auto ranks = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(slices), dim3(kSliceThreads), 0, ctx->stream, st_ptr, cand.get(),
+                                   cbucket.get(), leaving.get(), targets, vw, part_weights, k, capacity, before.get(),
+                                   sums.get(), left_vertex.get(), left_code.get(), left_count.get(),
+                                   destination_replicas);
+            };
+            if (few) {
+                ranks(balance_source_ranks_kernel<W, false>);
+                hipLaunchKernelGGL((balance_destinations_kernel<O, W>), dim3(1), dim3(kSelectThreads), 0, ctx->stream,
+                                   st_ptr, slices, left_vertex.get(), left_code.get(), left_count.get(), labels, vw, off,
+                                   k, part_weights, capacity, light.get(), heavy.get(), flags, state);
+            } else {
+                ranks(balance_source_ranks_kernel<W, true>);
+                hipLaunchKernelGGL(bucket_boundaries_kernel<true>, dim3(k), dim3(kBucketScanThreads), 0, ctx->stream,
+                                   destination_replicas, k, part_weights, capacity, boundary.get(), before.get());
+                auto slice = [&](auto kernel) {
+                    hipLaunchKernelGGL(kernel, dim3(slices), dim3(kSliceThreads), 0, ctx->stream, st_ptr,
+                                       left_vertex.get(), left_code.get(), left_count.get(), labels, vw, off, k,
+                                       part_weights, capacity, boundary.get(), before.get(), sums.get(), light.get(),
+                                       heavy.get(), flags, state);
+                };
+                slice(balance_slices_kernel<O, W, false>);
+                slice(balance_slices_kernel<O, W, true>);
+            }
+            GPART_LAUNCH_CHECK();
         });
         if (r)
             apply_rows(ctx, run, g, c, r, st_ptr, light.get(), heavy.get(), labels, targets, flags, k, cache,

@@ -24,9 +24,9 @@ constexpr int kRowSpan = 8;
 // The lane's kRowSpan entries of a cache row, entries at or past k as 0: 16-byte
 // loads when the span lies inside the row and is 16-byte aligned (k a multiple of
 // 4 or 2 entries), else one load per entry.
-template <typename C>
-__device__ __forceinline__ void load_span(const C* row, int j, int k, unsigned long long (&out)[kRowSpan]) {
-    static_assert(sizeof(C) == 4 || sizeof(C) == 8, "4- or 8-byte cache entries");
+template <typename C, typename U>
+__device__ __forceinline__ void load_span(const C* row, int j, int k, U (&out)[kRowSpan]) {
+    static_assert((sizeof(C) == 4 || sizeof(C) == 8) && sizeof(U) >= sizeof(C), "4- or 8-byte cache entries");
     const int first = j * kRowSpan;
     const C* span = row + first;
     if (first + kRowSpan <= k && (reinterpret_cast<std::uintptr_t>(span) & 15) == 0) {
@@ -40,13 +40,13 @@ __device__ __forceinline__ void load_span(const C* row, int j, int k, unsigned l
                 out[4 * q + 2] = x.z;
                 out[4 * q + 3] = x.w;
             } else {
-                out[2 * q] = static_cast<unsigned long long>(x.x) | static_cast<unsigned long long>(x.y) << 32;
-                out[2 * q + 1] = static_cast<unsigned long long>(x.z) | static_cast<unsigned long long>(x.w) << 32;
+                out[2 * q] = static_cast<U>(x.x) | static_cast<U>(x.y) << 32;
+                out[2 * q + 1] = static_cast<U>(x.z) | static_cast<U>(x.w) << 32;
             }
         }
     } else {
 #pragma unroll
-        for (int e = 0; e < kRowSpan; ++e) out[e] = first + e < k ? static_cast<unsigned long long>(span[e]) : 0;
+        for (int e = 0; e < kRowSpan; ++e) out[e] = first + e < k ? static_cast<U>(span[e]) : 0;
     }
 }
 
@@ -79,15 +79,15 @@ struct PowerTable {
 };
 
 // balance_gain_bucket (:167-171): clamp(25 + ceil(log_1.5(-g)), 2, 49) for g < 0,
-// evaluated as the smallest j with -g <= 1.5^j.
-__device__ __forceinline__ int gain_bucket(double gain, const PowerTable& t) {
+// evaluated as the smallest j with -g <= 1.5^j. powers: PowerTable's values.
+__device__ __forceinline__ int gain_bucket(double gain, const double* powers) {
     if (gain > 0) return 0;
     if (gain == 0) return 1;
     const double x = -gain;
     int lo = 0, hi = 48;
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        if (x <= t.value[mid]) hi = mid;
+        if (x <= powers[mid]) hi = mid;
         else lo = mid + 1;
     }
     const int j = lo == 48 ? 25 : lo - 23;

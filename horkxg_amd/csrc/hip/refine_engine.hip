@@ -507,7 +507,7 @@ __device__ void stage_balance_proposals(const EngineArgs<O, W, C>& a, std::int64
                 const double gain =
                     conn >= current ? static_cast<double>(conn - current) : -static_cast<double>(current - conn);
                 const double per_weight = gain / static_cast<double>(weight);
-                bucket = source * kBalanceWidth + gain_bucket(per_weight, a.powers) * kBalanceSections +
+                bucket = source * kBalanceWidth + gain_bucket(per_weight, a.powers.value) * kBalanceSections +
                          static_cast<int>(mix32(static_cast<std::uint32_t>(v)) % kBalanceSections);
                 table_add(sh.table, static_cast<unsigned>(bucket), weight, a.src_counts);
             }
