@@ -39,6 +39,7 @@ __device__ __forceinline__ std::uint64_t lanemask_lt() {
 // Every lane that a pattern reads must be active, as with __shfl_*.
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppRowRor8 = 0x128;
 constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
+constexpr int kDppRowShl = 0x100;  // + 1..15
 constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;
 
 // Lanes without a source (and rows outside RowMask) receive 0.

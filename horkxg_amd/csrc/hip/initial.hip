@@ -15,7 +15,8 @@
 //
 // Plain form: the reference's launch structure, one task at a time (start, then
 // per step: SpMV, finish_moments, normalize).
-// Batched form: all tasks of one recursion depth share every launch. A depth is
+// Batched form: all tasks of one recursion depth share every launch (small sparse
+// tasks a single one, the solo form below). Else a depth is
 // 66 launches whatever its task count: start, 64 steps (each also finishing the
 // previous step's moments and normalising on read), and one 1024-thread
 // workgroup per task for the (x, id) sort (LDS bitonic), the weight prefix, the
@@ -52,8 +53,10 @@ __global__ void __launch_bounds__(256) spectral_start_kernel(int count, const in
         Moments m{0, 0, 0};
         if (i < count) {
             const int v = ids[i];
-            // CSR entries each diffusion step scans (for the family's algorithmic bytes)
-            atomicAdd(entries, static_cast<unsigned long long>(offsets[v + 1] - offsets[v]));
+            // CSR entries each diffusion step scans, for the family's algorithmic bytes:
+            // counted under profiling only, the atomics of all rows meet in one word
+            // (7,429 rows: 48 us of the launch's 52)
+            if (entries) atomicAdd(entries, static_cast<unsigned long long>(offsets[v + 1] - offsets[v]));
             const double a = static_cast<double>(mix32(static_cast<unsigned>(v) ^ seed)) / 4294967296.0 - 0.5;
             degree[v] = d;
             x[v] = a;
@@ -186,7 +189,7 @@ __global__ void __launch_bounds__(256) depth_start_kernel(DepthTasks dt, const i
         Moments m{0, 0, 0};
         if (i < task.count) {
             const int v = ids[i];
-            atomicAdd(entries, static_cast<unsigned long long>(offsets[v + 1] - offsets[v]));
+            if (entries) atomicAdd(entries, static_cast<unsigned long long>(offsets[v + 1] - offsets[v]));
             const double a = static_cast<double>(mix32(static_cast<unsigned>(v) ^ tseed)) / 4294967296.0 - 0.5;
             degree[v] = d;
             x[v] = static_cast<T>(a);
@@ -226,15 +229,7 @@ __global__ void __launch_bounds__(256) depth_step_kernel(DepthTasks dt, const in
             if (labels[u] == group) sum = VecTraits<T>::fmadd(static_cast<T>(weights[e]), normalized(x, u, norm), sum);
         }
     }
-    double sd;
-    if constexpr (sizeof(T) == 8) {
-        sd = tree32(static_cast<double>(sum));
-    } else {
-        float f = sum;
-#pragma unroll
-        for (int s2 = 16; s2; s2 >>= 1) f += __shfl_down(f, s2, kHalf);
-        sd = static_cast<double>(f);
-    }
+    const double sd = static_cast<double>(tree32(sum));
     if (lane == 0) {
         Moments m{0, 0, 0};
         if (i < task.count) {
@@ -281,6 +276,278 @@ __global__ void __launch_bounds__(kBatchThreads) depth_finish_kernel(DepthTasks 
     if (st && threadIdx.x == 0) atomicMax(status, st);
 }
 
+// ------------------------------------------------------------------- solo form
+//
+// A step of a small sparse task is a few microseconds of launch and of dependent loads
+// (id, row, neighbour, label, value) around a few hundred nanoseconds of work: 5.0-6.5
+// us per launch, 64 per depth. Here one workgroup does a task's whole depth, start,
+// steps and split, in one launch. The vector stays in LDS; a thread owns up to four
+// rows, and their entries, resolved to positions inside the task once, lie in slots of
+// one lane each (sliced ELL: rows of a wave share the width of the longest), so that a
+// step reads them in runs from the L2. Values are bit-identical to the launch form: a
+// thread sums its row's 32 strided accumulators and their tree itself (absent entries
+// and other tasks' neighbours are zero terms), eight neighbouring lanes form a block's
+// partial, and finish_block is the same. A step waits for its two barriers and the
+// normalisation's chain (1.3 us at 460 rows), from about 2,000 rows on for the slots and
+// the LDS reads. Bisection of a 7,429-vertex weighted mesh into 32, with its four depths
+// below the root: 3.29 -> 2.33 ms.
+constexpr int kSoloThreads = 1024;
+constexpr int kSoloRows = kMaxBatchedTask / kSoloThreads;  // rows per thread
+constexpr int kSoloGroups = kMaxBatchedTask / kWave;       // groups of 64 rows, one width each
+// Entries of a task, estimated by its share of the graph's vertices, up to which the
+// solo form is taken. Weighted 3D meshes, FP64, a depth of tasks of 3,700 vertices and
+// 21,000 entries: 500 us, the launch form 500; of 1,860 and 10,500: 300 and 500; of 930
+// and 5,300: 190 and 490; of 460 and 2,600: 145 and 490.
+constexpr double kSoloEntries = 16384;
+
+struct SoloTasks {
+    int count;
+    long long first_slot[kMaxDepthTasks + 1];  // of each task's slots, in rows of 64
+    gpart_bisect_task task[kMaxDepthTasks];
+};
+
+// The sum of a row's terms in the reference's order: accumulator l takes terms l,
+// l + 32, ..., then a tree (16, 8, 4, 2, 1) whose absent leaves would add zero.
+// terms(first, part) adds the terms from `first` on to a run of accumulators, whose
+// loads are so under way together.
+template <typename A, int N, int Run, typename Terms>
+__device__ __forceinline__ A tree_sum(int width, Terms terms) {
+    A v[N];
+#pragma unroll
+    for (int l = 0; l < N; ++l) v[l] = A(0);
+    for (int first = 0; first < width; first += N) {
+#pragma unroll
+        for (int c = 0; c < N; c += Run) {
+            A part[Run];
+#pragma unroll
+            for (int l = 0; l < Run; ++l) part[l] = v[c + l];
+            terms(first + c, part);
+#pragma unroll
+            for (int l = 0; l < Run; ++l) v[c + l] = part[l];
+            // no more than a run's loads at once: the registers do not hold them
+            if constexpr (Run < N) __builtin_amdgcn_sched_barrier(0);
+        }
+        if (N < 32) break;
+    }
+#pragma unroll
+    for (int h = 16; h > 0; h /= 2)
+#pragma unroll
+        for (int l = 0; l < h; ++l)
+            if (l + h < N) v[l] += v[l + h];
+    return v[0];
+}
+// over slots, the same width for a wave
+template <typename A, typename Terms>
+__device__ __forceinline__ A row_sum(int width, Terms terms) {
+    if (width <= 4) return tree_sum<A, 4, 4>(width, terms);
+    if (width <= 8) return tree_sum<A, 8, 8>(width, terms);
+    if (width <= 12) return tree_sum<A, 12, 12>(width, terms);
+    if (width <= 16) return tree_sum<A, 16, 8>(width, terms);
+    if (width <= 24) return tree_sum<A, 24, 8>(width, terms);
+    return tree_sum<A, 32, 8>(width, terms);
+}
+// the slots that row_sum reads for a row of `width` entries
+__device__ __forceinline__ int padded_width(int width) {
+    if (width <= 16) return (width + 3) / 4 * 4;
+    return width <= 24 ? 24 : (width + 31) / 32 * 32;
+}
+
+// A slot: position in the low 12 bits, weight above. Of 4 bytes while a group's weights
+// are below 2^20 (a step's time is the slots' way from the L2), else of 8, up to 2^52.
+constexpr int kSlotShift = 12;
+static_assert(kMaxBatchedTask <= 1 << kSlotShift, "a task's positions fit");
+
+template <typename T>
+struct SoloShared {
+    BatchShared batch;  // its keys hold the degrees until the split
+    T x[kMaxBatchedTask];   // normalised
+    T y[kMaxBatchedTask];   // a step's result
+    Moments partials[kMaxBatchedTask / 8];
+    int width[kSoloGroups];  // of a group of 64 rows: its longest
+    long long slots[kSoloGroups];  // its first slot, in rows of 64; -1: it has none
+    int slot_bytes[kSoloGroups];   // 0: its entries are read from the CSR
+};
+
+template <typename O, typename W, typename T>
+__global__ void __launch_bounds__(kSoloThreads) depth_solo_kernel(
+    SoloTasks st, int* labels, int* order, const O* offsets, const int* neighbors, const W* weights,
+    const std::uint64_t* vertex_weights, unsigned seed, std::uint64_t capacity, double* coords, int* position,
+    std::uint64_t* slot, gpart_bisect_task* next, int* next_count, int* status,
+    unsigned long long* entries) {
+    __shared__ SoloShared<T> sh;
+    const gpart_bisect_task task = st.task[blockIdx.x];
+    const int count = task.count, group = task.first_part, blocks = (count + 7) / 8;
+    const int rounds = (count + kSoloThreads - 1) / kSoloThreads;
+    int* ids = order + task.begin;
+    double* degree = reinterpret_cast<double*>(sh.batch.keys);
+    const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
+    unsigned long long scanned = 0;
+    if (t < kSoloGroups) sh.width[t] = 0;
+    __syncthreads();
+    for (int r = t, g = wave; g < rounds * (kSoloThreads / kWave); r += kSoloThreads, g += kSoloThreads / kWave) {
+        int width = 0;
+        if (r < count) {
+            const int v = ids[r];
+            position[v] = r;
+            width = static_cast<int>(offsets[v + 1] - offsets[v]);
+        }
+        scanned += static_cast<unsigned long long>(width);
+#pragma unroll
+        for (int m = kWave / 2; m > 0; m /= 2) width = max(width, __shfl_xor(width, m, kWave));
+        if (lane == 0) sh.width[g] = width;
+    }
+    scanned = group_sum_u64<kWave>(scanned);
+    if (entries && lane == 0 && scanned) atomicAdd(entries, scanned);
+    __syncthreads();  // widths and positions
+    if (wave == 0) {
+        const int width = padded_width(sh.width[lane]);
+        const long long inclusive = wave_scan(static_cast<long long>(width));
+        const long long first = st.first_slot[blockIdx.x] + inclusive - width;
+        sh.slots[lane] = first + width <= st.first_slot[blockIdx.x + 1] ? first : -1;
+    }
+    __syncthreads();
+    static_assert(kSoloGroups == kWave, "one wave places the groups");
+    // four terms of row r from the CSR: weight (0: no entry, or another task's neighbour) and position
+    auto resolve = [&](int r, int first, W (&w)[4], int (&pos)[4]) {
+        std::int64_t e = 0, end = 0;
+        if (r < count) {
+            const int v = ids[r];
+            e = static_cast<std::int64_t>(offsets[v]) + first;
+            end = static_cast<std::int64_t>(offsets[v + 1]);
+        }
+        int u[4];
+#pragma unroll
+        for (int l = 0; l < 4; ++l) u[l] = e + l < end ? neighbors[e + l] : -1;
+#pragma unroll
+        for (int l = 0; l < 4; ++l) w[l] = u[l] >= 0 ? weights[e + l] : W(0);
+#pragma unroll
+        for (int l = 0; l < 4; ++l)
+            if (u[l] >= 0 && labels[u[l]] != group) u[l] = -1;
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            pos[l] = u[l] >= 0 ? position[u[l]] : 0;
+            w[l] = u[l] >= 0 ? w[l] : W(0);
+        }
+    };
+    // row r's entries into its slots; returns all its weights or-ed
+    auto fill = [&](int r, auto* slots) {
+        using S = std::remove_pointer_t<decltype(slots)>;
+        const int width = __builtin_amdgcn_readfirstlane(padded_width(sh.width[r / kWave]));
+        std::uint64_t bits = 0;
+#pragma unroll 1
+        for (int first = 0; first < width; first += 4) {
+            W w[4];
+            int pos[4];
+            resolve(r, first, w, pos);
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                bits |= w[l];
+                slots[(first + l) * kWave + lane] = static_cast<S>(w[l]) << 12 | static_cast<S>(pos[l]);
+            }
+        }
+        return bits;
+    };
+    // the sum of term(weight, position, accumulator) over row r
+    auto over_row = [&](int r, auto zero, auto term) {
+        using A = decltype(zero);
+        const int g = r / kWave;
+        const int width = __builtin_amdgcn_readfirstlane(sh.width[g]);
+        auto stored = [&](const auto* at) {
+            return row_sum<A>(width, [&](int first, auto& acc) {
+                constexpr int N = sizeof(acc) / sizeof(A);
+                std::remove_cv_t<std::remove_pointer_t<decltype(at)>> s[N];
+#pragma unroll
+                for (int l = 0; l < N; ++l) s[l] = at[(first + l) * kWave];
+#pragma unroll
+                for (int l = 0; l < N; ++l)
+                    acc[l] = term(s[l] >> kSlotShift, static_cast<int>(s[l] & ((1 << kSlotShift) - 1)), acc[l]);
+            });
+        };
+        const int bytes = __builtin_amdgcn_readfirstlane(sh.slot_bytes[g]);
+        const std::uint64_t* at = slot + sh.slots[g] * kWave;
+        if (bytes == 4) return stored(reinterpret_cast<const std::uint32_t*>(at) + lane);
+        if (bytes == 8) return stored(at + lane);
+        return tree_sum<A, 32, 4>(width, [&](int first, A (&acc)[4]) {
+            W w[4];
+            int pos[4];
+            resolve(r, first, w, pos);
+#pragma unroll
+            for (int l = 0; l < 4; ++l) acc[l] = term(w[l], pos[l], acc[l]);
+        });
+    };
+    // a row's moments into its block of eight rows
+    auto absorb = [&](int r, double mass, double a) {
+        Moments m{0, 0, 0};
+        if (r < count) m = Moments{mass, mass * a, mass * a * a};
+        auto total = [](double v) {
+            v = z(v);
+            v += lane_down<4>(v);
+            v += lane_down<2>(v);
+            return v + lane_down<1>(v);
+        };
+        m = Moments{total(m.mass), total(m.sum), total(m.squares)};
+        if ((t & 7) == 0 && r / 8 < blocks) sh.partials[r / 8] = m;
+    };
+    // spectral_start (:81-107)
+    const unsigned tseed = seed ^ static_cast<unsigned>(task.first_part);
+#pragma unroll 1
+    for (int r = t; r < rounds * kSoloThreads; r += kSoloThreads) {
+        const int g = r / kWave;
+        std::uint64_t* slots = sh.slots[g] >= 0 ? slot + sh.slots[g] * kWave : nullptr;
+        int bytes = 0;
+        if (slots) {
+            const std::uint64_t bits = fill(r, reinterpret_cast<std::uint32_t*>(slots));
+            bytes = 4;
+            if (__any(bits >> (32 - kSlotShift) != 0)) {
+                fill(r, slots);
+                bytes = __any(bits >> (64 - kSlotShift) != 0) ? 0 : 8;
+            }
+        }
+        if (lane == 0) sh.slot_bytes[g] = bytes;
+        const double d = over_row(r, 0.0, [](auto w, int, double acc) { return acc + static_cast<double>(w); });
+        T x = 0;
+        if (r < count) {
+            x = static_cast<T>(static_cast<double>(mix32(static_cast<unsigned>(ids[r]) ^ tseed)) / 4294967296.0 - 0.5);
+            degree[r] = d;
+            sh.y[r] = x;
+        }
+        absorb(r, d > 0 ? d : 1.0, static_cast<double>(x));
+    }
+    __syncthreads();
+    // finish_moments (:65-79), normalize (:138-142) and spectral_step (:109-136)
+#pragma unroll 1
+    for (int step = 0;; ++step) {
+        const Norm norm = finish_block(sh.partials, blocks, sh.batch.shared8, &sh.batch.norm);
+        for (int r = t; r < count; r += kSoloThreads)
+            sh.x[r] = static_cast<T>((static_cast<double>(sh.y[r]) - norm.mean) * norm.scale);
+        __syncthreads();
+        if (step == 64) break;
+#pragma unroll 1
+        for (int r = t; r < rounds * kSoloThreads; r += kSoloThreads) {
+            const T sum = over_row(r, T(0), [&](auto w, int pos, T acc) {
+                return VecTraits<T>::fmadd(static_cast<T>(w), sh.x[pos], acc);
+            });
+            double a = 0, d = 0;
+            if (r < count) {
+                d = degree[r];
+                const T x = sh.x[r];
+                if constexpr (sizeof(T) == 8) {
+                    a = d > 0 ? 0.5 * (x + sum / d) : x;
+                } else {
+                    a = static_cast<double>(d > 0 ? 0.5f * (x + sum / static_cast<float>(d)) : x);
+                }
+                sh.y[r] = static_cast<T>(a);
+            }
+            absorb(r, d > 0 ? d : 1.0, a);
+        }
+        __syncthreads();
+    }
+    const int failed = split_task<T>(
+        task, ids, labels, vertex_weights, capacity, coords, sh.batch, [&](int i, int) { return sh.x[i]; },
+        [&](const gpart_bisect_task& child) { next[atomicAdd(next_count, 1)] = child; });
+    if (failed && t == 0) atomicMax(status, failed);
+}
+
 template <typename O, typename W>
 void plain_task(gpart_ctx* ctx, const gpart_csr_view* g, const int32_t* labels, int32_t* order,
                 const std::uint64_t* vertex_weights, const gpart_bisect_task* task, uint32_t seed, double* x,
@@ -299,7 +566,8 @@ void plain_task(gpart_ctx* ctx, const gpart_csr_view* g, const int32_t* labels, 
     profile_begin(ctx, GPART_PROFILE_SPECTRAL);
     hipLaunchKernelGGL((spectral_start_kernel<O, W>), dim3(spectral_blocks), dim3(256), 0, ctx->stream, count, ids,
                        labels, task->first_part, off, g->neighbors, w, degree, x,
-                       seed ^ static_cast<unsigned>(task->first_part), partials.get(), entries.get());
+                       seed ^ static_cast<unsigned>(task->first_part), partials.get(),
+                       ctx->profile[GPART_PROFILE_SPECTRAL].enabled ? entries.get() : nullptr);
     hipLaunchKernelGGL(finish_moments_kernel, dim3(1), dim3(256), 0, ctx->stream, spectral_blocks, partials.get(),
                        norm.get());
     GPART_LAUNCH_CHECK();
@@ -400,7 +668,7 @@ int gpart_spectral_depth(gpart_ctx* ctx, const gpart_csr_view* g, int32_t* label
         Scratch<unsigned long long> counters(ctx, 2);
         fill_bytes(ctx, counters.get(), 0, 16);
         int* next_and_status = reinterpret_cast<int*>(counters.get());
-        unsigned long long* entries = counters.get() + 1;
+        unsigned long long* entries = ctx->profile[GPART_PROFILE_SPECTRAL].enabled ? counters.get() + 1 : nullptr;
         int vertices = 0;
         for (int t = 0; t < task_count; ++t) vertices += tasks[t].count;
         profile_begin(ctx, GPART_PROFILE_SPECTRAL);
@@ -427,14 +695,41 @@ int gpart_spectral_depth(gpart_ctx* ctx, const gpart_csr_view* g, int32_t* label
                                next_and_status + 1);
             GPART_LAUNCH_CHECK();
         };
-        const bool fp32 = precision == GPART_SPECTRAL_FP32;
-        if (g->width == GPART_WIDTH_STANDARD) {
-            if (fp32) launch(std::int32_t{}, std::uint32_t{}, float{});
-            else launch(std::int32_t{}, std::uint32_t{}, double{});
-        } else {
-            if (fp32) launch(std::int64_t{}, std::uint64_t{}, float{});
-            else launch(std::int64_t{}, std::uint64_t{}, double{});
+        // one workgroup per task where every task is small and sparse enough
+        SoloTasks solo{};
+        solo.count = task_count;
+        bool alone = true;
+        for (int t = 0; t < task_count; ++t) {
+            const double share = static_cast<double>(g->m) * tasks[t].count / static_cast<double>(n);
+            alone = alone && share <= kSoloEntries;
+            solo.task[t] = tasks[t];
+            // twice the estimate in whole rows of 64, and as much again for uneven widths
+            solo.first_slot[t + 1] =
+                solo.first_slot[t] + static_cast<long long>(4.0 * share / kWave) + kSoloGroups * 8;
         }
+        const std::int64_t slots = alone ? solo.first_slot[task_count] * kWave : 0;
+        Scratch<int> position(ctx, alone ? n : 0);
+        Scratch<std::uint64_t> slot(ctx, slots);
+        auto launch_solo = [&](auto o_tag, auto w_tag, auto t_tag) {
+            using O = decltype(o_tag);
+            using W = decltype(w_tag);
+            using T = decltype(t_tag);
+            hipLaunchKernelGGL((depth_solo_kernel<O, W, T>), dim3(task_count), dim3(kSoloThreads), 0, ctx->stream, solo,
+                               labels, order, static_cast<const O*>(g->offsets), g->neighbors,
+                               static_cast<const W*>(g->edge_weights), vertex_weights, seed, capacity, coords,
+                               position.get(), slot.get(), next,
+                               next_and_status, next_and_status + 1, entries);
+            GPART_LAUNCH_CHECK();
+        };
+        const bool fp32 = precision == GPART_SPECTRAL_FP32;
+        auto run = [&](auto o_tag, auto w_tag) {
+            if (alone && fp32) launch_solo(o_tag, w_tag, float{});
+            else if (alone) launch_solo(o_tag, w_tag, double{});
+            else if (fp32) launch(o_tag, w_tag, float{});
+            else launch(o_tag, w_tag, double{});
+        };
+        if (g->width == GPART_WIDTH_STANDARD) run(std::int32_t{}, std::uint32_t{});
+        else run(std::int64_t{}, std::uint64_t{});
         profile_end(ctx, GPART_PROFILE_SPECTRAL, 0.0);
         unsigned long long h[2];
         read_back(ctx, h, counters.get(), sizeof(h));

@@ -21,9 +21,37 @@ struct Moments {
     double mass, sum, squares;
 };
 
-__device__ __forceinline__ double tree32(double v) {
-#pragma unroll
-    for (int s = 16; s; s >>= 1) v += __shfl_down(v, s, kHalf);
+// v of the lane `Distance` further on (1, 2, 4 or 8, inside a row of 16; 16: of lanes
+// 0..15 and 32..47 only). Lanes without a source receive something.
+template <int Distance>
+__device__ __forceinline__ unsigned lane_down(unsigned v) {
+    if constexpr (Distance == 16)
+        return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+    else
+        return dpp_or_zero<kDppRowShl + Distance>(v);
+}
+template <int Distance>
+__device__ __forceinline__ double lane_down(double v) {
+    const auto bits = static_cast<std::uint64_t>(__double_as_longlong(v));
+    const std::uint64_t lo = lane_down<Distance>(static_cast<unsigned>(bits));
+    const std::uint64_t hi = lane_down<Distance>(static_cast<unsigned>(bits >> 32));
+    return __longlong_as_double(static_cast<long long>(hi << 32 | lo));
+}
+template <int Distance>
+__device__ __forceinline__ float lane_down(float v) {
+    return __uint_as_float(lane_down<Distance>(__float_as_uint(v)));
+}
+
+// The reference's 32-lane tree (distances 16, 8, 4, 2, 1): the total on lane 0 of each
+// half-wave. Lane moves in the VALU: a wave's step waits for five of them in turn, and
+// through the LDS each was about 60 ns.
+template <typename T>
+__device__ __forceinline__ T tree32(T v) {
+    v += lane_down<16>(v);
+    v += lane_down<8>(v);
+    v += lane_down<4>(v);
+    v += lane_down<2>(v);
+    v += lane_down<1>(v);
     return v;
 }
 
@@ -138,6 +166,7 @@ struct BatchShared {
     int ids[kMaxBatchedTask];
     double shared8[24];
     Norm norm;
+    std::uint64_t wave_weight[kBatchThreads / kWave];
     int boundary;
     int status;
 };
@@ -208,14 +237,19 @@ __device__ int split_task(const gpart_bisect_task& task, int* ids, int* labels, 
         sh.keys[i] = vertex_weights[sh.ids[i]];
     }
     __syncthreads();
-    for (int offset = 1; offset < count; offset <<= 1) {
-        std::uint64_t add[kMaxBatchedTask / kBatchThreads] = {};
-        int slot = 0;
-        for (int i = threadIdx.x; i < count; i += kBatchThreads, ++slot)
-            add[slot] = i >= offset ? sh.keys[i - offset] : 0;
+    std::uint64_t before = 0;
+    for (int first = 0; first < count; first += kBatchThreads) {
+        const int i = first + threadIdx.x, wave = threadIdx.x / kWave;
+        const std::uint64_t inclusive = wave_scan(i < count ? sh.keys[i] : 0);
+        if (lane_id() == kWave - 1) sh.wave_weight[wave] = inclusive;
         __syncthreads();
-        slot = 0;
-        for (int i = threadIdx.x; i < count; i += kBatchThreads, ++slot) sh.keys[i] += add[slot];
+        std::uint64_t total = 0, mine = before;
+        for (int w = 0; w < kBatchThreads / kWave; ++w) {
+            if (w == wave) mine += total;
+            total += sh.wave_weight[w];
+        }
+        if (i < count) sh.keys[i] = mine + inclusive;
+        before += total;
         __syncthreads();
     }
     // split selection (src/initial_partition_gpu.cu:233-248)

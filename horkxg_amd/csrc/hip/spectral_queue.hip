@@ -250,14 +250,7 @@ __device__ __forceinline__ void row_sums(const QueueStep<T>& s, const int* local
 
 template <typename T>
 __device__ __forceinline__ double half_wave_total(T v) {
-    if constexpr (sizeof(T) == 8) {
-        return tree32(static_cast<double>(v));
-    } else {
-        float f = v;
-#pragma unroll
-        for (int s2 = 16; s2; s2 >>= 1) f += __shfl_down(f, s2, kHalf);
-        return static_cast<double>(f);
-    }
+    return static_cast<double>(tree32(v));
 }
 
 // One member's share of one task: start, 64 steps, and (member 0) the split.
