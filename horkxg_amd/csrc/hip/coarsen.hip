@@ -138,7 +138,7 @@ struct ClassStore {
     std::int32_t* medium;
     std::int32_t* high;
     std::int64_t n;
-    unsigned long long* counts;
+    Publication counts;
     __device__ __forceinline__ void operator()(std::int64_t v, const DegreeScan& prefix,
                                                const DegreeScan& item) const {
         if (item.c[0]) low[prefix.c[0]] = static_cast<std::int32_t>(v);
@@ -146,10 +146,11 @@ struct ClassStore {
         else high[prefix.c[2]] = static_cast<std::int32_t>(v);
         if (v == n - 1) {
             const DegreeScan total = DegreeScanOp{}(prefix, item);
-            for (int j = 0; j < 3; ++j) counts[j] = static_cast<unsigned long long>(total.c[j]);
-            counts[3] = static_cast<unsigned long long>(total.high_edges);
-            counts[4] = static_cast<unsigned long long>(total.max_degree);
-            counts[5] = static_cast<unsigned long long>(total.isolated);
+            for (int j = 0; j < 3; ++j) counts.words[1 + j] = static_cast<unsigned long long>(total.c[j]);
+            counts.words[4] = static_cast<unsigned long long>(total.high_edges);
+            counts.words[5] = static_cast<unsigned long long>(total.max_degree);
+            counts.words[6] = static_cast<unsigned long long>(total.isolated);
+            publish_sequence(counts);
         }
     }
 };
@@ -871,20 +872,23 @@ struct ValidLoad {
 struct IdStore {
     std::int32_t* out;
     std::int64_t n;
-    std::int64_t* count;
+    Publication count;
     __device__ __forceinline__ void operator()(std::int64_t v, std::int64_t prefix, std::int64_t item) const {
         if (item) out[prefix] = static_cast<std::int32_t>(v);
-        if (v == n - 1) *count = prefix + item;
+        if (v == n - 1) {
+            count.words[1] = static_cast<unsigned long long>(prefix + item);
+            publish_sequence(count);
+        }
     }
 };
-void compact_valid(gpart_ctx* ctx, std::int64_t n, const std::int32_t* targets, std::int32_t* out,
-                   std::int64_t* d_count) {
-    if (n <= 0) {
-        fill_bytes(ctx, d_count, 0, sizeof(std::int64_t));
-        return;
-    }
-    device_scan<std::int64_t, SumOp<std::int64_t>>(ctx, ValidLoad{targets}, IdStore{out, n, d_count}, n,
+// The scan's last element sends the count to the host itself.
+std::int64_t compact_valid(gpart_ctx* ctx, std::int64_t n, const std::int32_t* targets, std::int32_t* out) {
+    std::int64_t count = 0;
+    if (n <= 0) return count;
+    device_scan<std::int64_t, SumOp<std::int64_t>>(ctx, ValidLoad{targets}, IdStore{out, n, publication(ctx)}, n,
                                                    SumOp<std::int64_t>{});
+    read_published(ctx, &count, sizeof(count));
+    return count;
 }
 
 // Key components of the admission order (target asc, gain desc, tie desc, id asc).
@@ -940,10 +944,13 @@ struct SegOneLoad {
 struct ExclusiveTotalStore {
     std::int64_t* out;
     std::int64_t n;
-    std::int64_t* total;
+    Publication total;
     __device__ __forceinline__ void operator()(std::int64_t i, std::int64_t prefix, std::int64_t item) const {
         out[i] = prefix;
-        if (i == n - 1) *total = prefix + item;
+        if (i == n - 1) {
+            total.words[1] = static_cast<unsigned long long>(prefix + item);
+            publish_sequence(total);
+        }
     }
 };
 struct SegInclusiveStore {
@@ -1247,9 +1254,9 @@ std::int32_t* admission_sort(gpart_ctx* ctx, std::int64_t n, std::int64_t p, std
 }
 
 unsigned long long count_nonempty(gpart_ctx* ctx, std::int64_t n, const unsigned long long* weights) {
-    Scratch<unsigned long long> c(ctx, 1);
-    device_reduce<unsigned long long>(ctx, NonzeroLoad{weights}, n, SumU64{}, c.get());
-    return read_scalar(ctx, c.get());
+    unsigned long long count = 0;
+    reduce_read<SumU64>(ctx, NonzeroLoad{weights}, n, &count);
+    return count;
 }
 
 template <typename O, typename W>
@@ -1408,16 +1415,14 @@ void launch_proposals(gpart_ctx* ctx, const gpart_csr_view* g, const std::int32_
 
 template <typename O, typename W>
 void build_classes(gpart_ctx* ctx, const gpart_csr_view* g, gpart_degree_classes* c) {
-    Scratch<unsigned long long> counters(ctx, 6);
-    fill_bytes(ctx, counters.get(), 0, 48);
+    unsigned long long h[6] = {};
     if (g->n > 0) {
         const auto* off = static_cast<const O*>(g->offsets);
         device_scan<DegreeScan, DegreeScanOp>(
-            ctx, ClassLoad<O>{off}, ClassStore<O>{off, c->low, c->medium, c->high, g->n, counters.get()}, g->n,
+            ctx, ClassLoad<O>{off}, ClassStore<O>{off, c->low, c->medium, c->high, g->n, publication(ctx)}, g->n,
             DegreeScanOp{});
+        read_published(ctx, h, sizeof(h));
     }
-    unsigned long long h[6];
-    read_back(ctx, h, counters.get(), sizeof(h));
     c->low_count = static_cast<std::int64_t>(h[0]);
     c->medium_count = static_cast<std::int64_t>(h[1]);
     c->high_count = static_cast<std::int64_t>(h[2]);
@@ -1429,9 +1434,10 @@ void build_classes(gpart_ctx* ctx, const gpart_csr_view* g, gpart_degree_classes
 template <typename O, typename W>
 void record_bounds_impl(gpart_ctx* ctx, const gpart_csr_view* g, std::uint64_t* row_bounds,
                         std::uint64_t* maximum, int* unsorted) {
-    Scratch<unsigned long long> meta(ctx, 2);
-    fill_bytes(ctx, meta.get(), 0, 16);
+    unsigned long long h[2] = {0, 0};  // unsorted, maximum
     if (g->n > 0) {
+        Scratch<unsigned long long> found(ctx, 1);
+        fill_bytes(ctx, found.get(), 0, 8);
         Scratch<std::int32_t> low(ctx, g->n), medium(ctx, g->n), high(ctx, g->n);
         gpart_degree_classes c{low.get(), medium.get(), high.get(), 0, 0, 0, 0, 0, 0};
         build_classes<O, W>(ctx, g, &c);
@@ -1440,20 +1446,18 @@ void record_bounds_impl(gpart_ctx* ctx, const gpart_csr_view* g, std::uint64_t* 
         auto* rb = reinterpret_cast<unsigned long long*>(row_bounds);
         if (c.low_count)
             hipLaunchKernelGGL((record_bound_kernel<O, W, 8>), dim3(grid_for(c.low_count * 8)), dim3(kBlock), 0,
-                               ctx->stream, c.low_count, c.low, off, g->neighbors, w, rb, meta.get());
+                               ctx->stream, c.low_count, c.low, off, g->neighbors, w, rb, found.get());
         if (c.medium_count)
             hipLaunchKernelGGL((record_bound_kernel<O, W, 64>), dim3(grid_for(c.medium_count * 64)), dim3(kBlock), 0,
-                               ctx->stream, c.medium_count, c.medium, off, g->neighbors, w, rb, meta.get());
+                               ctx->stream, c.medium_count, c.medium, off, g->neighbors, w, rb, found.get());
         if (c.high_count)
             hipLaunchKernelGGL((record_bound_kernel<O, W, 64>), dim3(grid_for(c.high_count * 64)), dim3(kBlock), 0,
-                               ctx->stream, c.high_count, c.high, off, g->neighbors, w, rb, meta.get());
+                               ctx->stream, c.high_count, c.high, off, g->neighbors, w, rb, found.get());
         GPART_LAUNCH_CHECK();
-        device_reduce<unsigned long long>(ctx, U64Load{rb}, g->n, MaxU64{}, meta.get());
+        reduce_read<MaxU64>(ctx, U64Load{rb}, g->n, h, found.get(), 1);
     }
-    unsigned long long h[2];
-    read_back(ctx, h, meta.get(), sizeof(h));
-    *maximum = h[0];
-    *unsorted = h[1] != 0;
+    *maximum = h[1];
+    *unsorted = h[0] != 0;
 }
 
 }  // namespace
@@ -1486,26 +1490,23 @@ int gpart_contract_record_bounds(gpart_ctx* ctx, int64_t n, const int32_t* map, 
         fill_bytes(ctx, coarse_bounds, 0, static_cast<std::size_t>(n_coarse) * 8);
         auto* cb = reinterpret_cast<unsigned long long*>(coarse_bounds);
         const auto* fb = reinterpret_cast<const unsigned long long*>(fine_bounds);
-        Scratch<unsigned long long> meta(ctx, 2);  // maximum, wrapped
-        fill_bytes(ctx, meta.get(), 0, 16);
+        Scratch<unsigned long long> wrapped(ctx, 1);
+        fill_bytes(ctx, wrapped.get(), 0, 8);
         if (n > 0) {
             hipLaunchKernelGGL(contract_bounds_add_kernel, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, n, map,
-                               fb, cb, meta.get() + 1);
+                               fb, cb, wrapped.get());
             GPART_LAUNCH_CHECK();
         }
-        if (n_coarse > 0) device_reduce<unsigned long long>(ctx, U64Load{cb}, n_coarse, MaxU64{}, meta.get());
-        unsigned long long h[2];
-        read_back(ctx, h, meta.get(), sizeof(h));
-        if (h[1]) {
+        unsigned long long h[2];  // wrapped, maximum
+        reduce_read<MaxU64>(ctx, U64Load{cb}, n_coarse, h, wrapped.get(), 1);
+        if (h[0]) {
             fill_bytes(ctx, coarse_bounds, 0, static_cast<std::size_t>(n_coarse) * 8);
-            fill_bytes(ctx, meta.get(), 0, 8);
             hipLaunchKernelGGL(contract_bounds_kernel, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, n, map, fb,
                                cb);
             GPART_LAUNCH_CHECK();
-            if (n_coarse > 0) device_reduce<unsigned long long>(ctx, U64Load{cb}, n_coarse, MaxU64{}, meta.get());
-            h[0] = read_scalar(ctx, meta.get());
+            reduce_read<MaxU64>(ctx, U64Load{cb}, n_coarse, h + 1);
         }
-        *maximum = h[0];
+        *maximum = h[1];
     });
 }
 
@@ -1529,9 +1530,7 @@ int gpart_sclp_admit(gpart_ctx* ctx, int64_t n, const int32_t* proposals, const 
         auto* cw = reinterpret_cast<unsigned long long*>(cluster_weights);
         const auto* gn = reinterpret_cast<const unsigned long long*>(gains);
         Scratch<std::int32_t> order(ctx, n), order_alt(ctx, n);
-        Scratch<std::int64_t> d_count(ctx, 1);
-        compact_valid(ctx, n, proposals, order.get(), d_count.get());
-        const std::int64_t p = read_scalar(ctx, d_count.get());
+        const std::int64_t p = compact_valid(ctx, n, proposals, order.get());
         *valid = p;
         *accepted = 0;
         if (p > 0) {
@@ -1539,7 +1538,7 @@ int gpart_sclp_admit(gpart_ctx* ctx, int64_t n, const int32_t* proposals, const 
                                                   gain_bound);
             Scratch<std::int32_t> ordered_targets(ctx, p), accept(ctx, p);
             Scratch<std::uint64_t> ordered_weights(ctx, p), prefix(ctx, p);
-            Scratch<unsigned long long> acc(ctx, 3);  // accepted, predicted gain, non-empty clusters
+            Scratch<unsigned long long> acc(ctx, 2);  // accepted, predicted gain
             // the gather also clears the commit's two counters
             hipLaunchKernelGGL(gather_order_kernel, dim3(grid_for(p)), dim3(kBlock), 0, ctx->stream, p, sorted,
                                proposals, vertex_weights, ordered_targets.get(), ordered_weights.get(), acc.get(), 2);
@@ -1556,9 +1555,8 @@ int gpart_sclp_admit(gpart_ctx* ctx, int64_t n, const int32_t* proposals, const 
             GPART_LAUNCH_CHECK();
             profile_end(ctx, GPART_PROFILE_SCLP_COMMIT, 0.0);
             // the non-empty cluster count comes back with the commit's counters
-            device_reduce<unsigned long long>(ctx, NonzeroLoad{cw}, n, SumU64{}, acc.get() + 2);
             unsigned long long h[3];
-            read_back(ctx, h, acc.get(), sizeof(h));
+            reduce_read<SumU64>(ctx, NonzeroLoad{cw}, n, h, acc.get(), 2);
             *accepted = static_cast<std::int64_t>(h[0]);
             *nonempty = static_cast<std::int64_t>(h[2]);
             // per proposal its order, target, weight and decision; per accepted move
@@ -1624,8 +1622,7 @@ int gpart_sclp_two_hop(gpart_ctx* ctx, int64_t n, const int32_t* proposals, cons
         hipLaunchKernelGGL(favorite_kernel, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, n, vertex_weights, cw,
                            clusters, proposals, favorites.get());
         GPART_LAUNCH_CHECK();
-        compact_valid(ctx, n, favorites.get(), order.get(), d_count.get());
-        const std::int64_t p = read_scalar(ctx, d_count.get());
+        const std::int64_t p = compact_valid(ctx, n, favorites.get(), order.get());
         *candidates = p;
         *pairable = 0;
         *merged = 0;
@@ -1646,21 +1643,21 @@ int gpart_sclp_two_hop(gpart_ctx* ctx, int64_t n, const int32_t* proposals, cons
             GPART_LAUNCH_CHECK();
             // positions and, in one read-back, the pair count
             device_scan<std::int64_t, SumOp<std::int64_t>>(ctx, ArrayLoad<std::int64_t>{pair_flags.get()},
-                                                           ExclusiveTotalStore{positions.get(), p, d_count.get()},
+                                                           ExclusiveTotalStore{positions.get(), p, publication(ctx)},
                                                            p, SumOp<std::int64_t>{});
-            const std::int64_t pair_count = read_scalar(ctx, d_count.get());
+            std::int64_t pair_count = 0;
+            read_published(ctx, &pair_count, sizeof(pair_count));
             *pairable = pair_count;
             const auto budget = static_cast<std::uint64_t>(std::max<std::int64_t>(0, merge_budget));
             if (pair_count > 0 && budget > 0) {
-                Scratch<unsigned long long> m(ctx, 2);  // merged pairs, non-empty clusters
-                fill_bytes(ctx, m.get(), 0, 16);
+                Scratch<unsigned long long> m(ctx, 1);  // merged pairs
+                fill_bytes(ctx, m.get(), 0, 8);
                 hipLaunchKernelGGL(two_hop_commit_kernel, dim3(grid_for(p)), dim3(kBlock), 0, ctx->stream, p, sorted,
                                    pair_flags.get(), positions.get(), budget, ordered_weights.get(), clusters, cw,
                                    m.get());
                 GPART_LAUNCH_CHECK();
-                device_reduce<unsigned long long>(ctx, NonzeroLoad{cw}, n, SumU64{}, m.get() + 1);
                 unsigned long long h[2];
-                read_back(ctx, h, m.get(), sizeof(h));
+                reduce_read<SumU64>(ctx, NonzeroLoad{cw}, n, h, m.get(), 1);
                 *merged = static_cast<std::int64_t>(h[0]);
                 *nonempty = static_cast<std::int64_t>(h[1]);
                 return;
@@ -1680,25 +1677,23 @@ int gpart_sclp_compact(gpart_ctx* ctx, int64_t n, const int32_t* clusters, const
                                                        SumOp<std::int64_t>{});
         const std::size_t wbytes = g->width == GPART_WIDTH_STANDARD ? 4 : 8;
         fill_bytes(ctx, coarse_vertex_weights, 0, static_cast<std::size_t>(n_coarse) * wbytes);
-        Scratch<unsigned long long> mx(ctx, 1);
-        fill_bytes(ctx, mx.get(), 0, 8);
+        unsigned long long largest = 0;
         if (g->width == GPART_WIDTH_STANDARD) {
             hipLaunchKernelGGL(map_and_weights_kernel<std::uint32_t>, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream,
                                n, clusters, compact.get(), static_cast<const std::uint32_t*>(g->vertex_weights), map,
                                static_cast<std::uint32_t*>(coarse_vertex_weights));
-            device_reduce<unsigned long long>(
-                ctx, WidenLoad<std::uint32_t>{static_cast<const std::uint32_t*>(coarse_vertex_weights)}, n_coarse,
-                MaxU64{}, mx.get());
+            GPART_LAUNCH_CHECK();
+            reduce_read<MaxU64>(ctx, WidenLoad<std::uint32_t>{static_cast<const std::uint32_t*>(coarse_vertex_weights)},
+                                n_coarse, &largest);
         } else {
             hipLaunchKernelGGL(map_and_weights_kernel<std::uint64_t>, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream,
                                n, clusters, compact.get(), static_cast<const std::uint64_t*>(g->vertex_weights), map,
                                static_cast<std::uint64_t*>(coarse_vertex_weights));
-            device_reduce<unsigned long long>(
-                ctx, WidenLoad<std::uint64_t>{static_cast<const std::uint64_t*>(coarse_vertex_weights)}, n_coarse,
-                MaxU64{}, mx.get());
+            GPART_LAUNCH_CHECK();
+            reduce_read<MaxU64>(ctx, WidenLoad<std::uint64_t>{static_cast<const std::uint64_t*>(coarse_vertex_weights)},
+                                n_coarse, &largest);
         }
-        GPART_LAUNCH_CHECK();
-        *maximum_weight = read_scalar(ctx, mx.get());
+        *maximum_weight = largest;
     });
 }
 

@@ -418,9 +418,9 @@ void contract_impl(gpart_ctx* ctx, const gpart_csr_view* fine, const gpart_degre
         // 16-byte records through the sort; the result is the same).
         const Layout packed = choose_layout(n_coarse, 0);
         if (packed.weight_bits) {
-            Scratch<unsigned long long> largest(ctx, 1);
-            device_reduce<unsigned long long>(ctx, WidenLoad<W>{ew}, m, MaxU64{}, largest.get());
-            if (read_scalar(ctx, largest.get()) <= packed.weight_mask) layout = packed;
+            unsigned long long largest = 0;
+            reduce_read<MaxU64>(ctx, WidenLoad<W>{ew}, m, &largest);
+            if (largest <= packed.weight_mask) layout = packed;
         }
     }
     Scratch<std::uint64_t> keys(ctx, std::max<std::int64_t>(m, 1)), keys_alt(ctx, std::max<std::int64_t>(m, 1));

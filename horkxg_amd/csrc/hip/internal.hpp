@@ -49,7 +49,9 @@ struct gpart_ctx {
     // word and publish its value (so a captured launch needs no new argument per
     // call); the host counts the same publications in status_seq.
     std::uint64_t status_seq = 0;
-    unsigned long long* status_counter = nullptr;  // device word
+    // Device words: that counter, and the workgroups of the reduction under way that
+    // have finished (its last one leaves 0; one stream, so one reduction at a time).
+    unsigned long long* status_counter = nullptr;
     gpart_hip::ScratchRecorder* recorder = nullptr;
     // The refinement's recorded round graphs (refine.hip), dropped before the
     // cache releases memory or the context ends; round_graphs switches them.
@@ -181,6 +183,16 @@ void read_back(gpart_ctx* ctx, void* host, const void* device, std::size_t bytes
 // Waits until status word 0 equals seq: polls for a short while, then synchronises
 // the stream (which also reports a failed kernel) and checks again.
 void wait_status(gpart_ctx* ctx, std::uint64_t seq);
+
+// Where a kernel publishes values to the host by itself, in place of a copy launch
+// after it: the values from word 1 on, then the sequence number (publish_sequence).
+// After each such launch comes one read_published, which waits for it.
+struct Publication {
+    unsigned long long* words;
+    unsigned long long* counter;
+};
+Publication publication(gpart_ctx* ctx);
+void read_published(gpart_ctx* ctx, void* host, std::size_t bytes);
 constexpr int kStatusWords = 512;  // 4 KiB of status memory per context
 
 template <typename T>

@@ -12,7 +12,7 @@
 //      tile is staged in LDS in digit order and written out so that consecutive
 //      threads store consecutive addresses of one digit run.
 // Inputs of at most 8192 keys (four tiles) are sorted in one launch instead:
-// three or more launches per 8-bit pass cost more than the whole sort in LDS.
+// three or more launches per 8-bit pass cost more than comparing all pairs.
 #include "internal.hpp"
 #include "scan.hpp"
 

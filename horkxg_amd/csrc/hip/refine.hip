@@ -2059,33 +2059,30 @@ template <typename O, typename W, typename C = unsigned long long>
 struct Ops {
     static void cut(gpart_ctx* ctx, const gpart_csr_view* g, const std::int32_t* labels, std::uint64_t* out) {
         const std::int64_t tiles = g->n > 0 && g->m > 0 ? tile_count(g->m) : 0;
-        Scratch<unsigned long long> d(ctx, 1);
         Scratch<std::int32_t> tile_row(ctx, tiles);
         Scratch<unsigned long long> partials(ctx, std::min<std::int64_t>(tiles, kReduceMaxBlocks));
-        cut_with(ctx, g, labels, d.get(), tile_row.get(), partials.get(), out);
+        cut_with(ctx, g, labels, tile_row.get(), partials.get(), out);
     }
 
-    // The cut over caller-provided device scratch: total (1 word), tile_row
-    // (tile_count(m) entries) and partials (min(tiles, kReduceMaxBlocks) words).
+    // The cut over caller-provided device scratch: tile_row (tile_count(m) entries) and
+    // partials (min(tiles, kReduceMaxBlocks) words, folded by one workgroup).
     static void cut_with(gpart_ctx* ctx, const gpart_csr_view* g, const std::int32_t* labels,
-                         unsigned long long* total, std::int32_t* tile_row, unsigned long long* partials,
-                         std::uint64_t* out) {
-        fill_bytes(ctx, total, 0, 8);
+                         std::int32_t* tile_row, unsigned long long* partials, std::uint64_t* out) {
+        unsigned long long directed = 0;
         const auto* off = static_cast<const O*>(g->offsets);
         const auto* w = static_cast<const W*>(g->edge_weights);
         if (g->n > 0 && g->m > 0) {
-            // edge tiles, capped grid, partials folded by one workgroup
+            // edge tiles, capped grid
             const std::int64_t tiles = tile_count(g->m);
             hipLaunchKernelGGL(tile_rows_kernel<O>, dim3(grid_for(g->n)), dim3(kBlock), 0, ctx->stream, g->n, off,
                                tile_row);
             const int blocks = static_cast<int>(std::min<std::int64_t>(tiles, kReduceMaxBlocks));
             hipLaunchKernelGGL((cut_kernel<O, W>), dim3(blocks), dim3(kTileLanes), 0, ctx->stream, g->n, g->m, tiles,
                                off, tile_row, g->neighbors, w, labels, partials);
-            hipLaunchKernelGGL((reduce_finish_kernel<unsigned long long, SumU64>), dim3(1), dim3(kReduceThreads), 0,
-                               ctx->stream, partials, blocks, SumU64{}, total);
             GPART_LAUNCH_CHECK();
+            static_assert(kReduceMaxBlocks <= kReduceThreads * kReduceLoads, "one workgroup: no scratch");
+            reduce_read<SumU64>(ctx, WidenLoad<unsigned long long>{partials}, blocks, &directed);
         }
-        const auto directed = read_scalar(ctx, total);
         if (directed & 1ULL) throw Error(GPART_ERR_RUNTIME, "refinement cut is not symmetric");
         *out = directed / 2;
     }
@@ -2661,10 +2658,9 @@ struct Ops {
 namespace gpart_hip {
 namespace {
 constexpr std::int64_t kCutScratchTiles = std::int64_t{1} << 20;  // CSRs up to 2^20 * 4096 entries
-constexpr std::size_t kCutScratchTotalOffset = 0;
-constexpr std::size_t kCutScratchPartialsOffset = 256;
+constexpr std::size_t kCutScratchPartialsOffset = 0;
 constexpr std::size_t kCutScratchTilesOffset = kCutScratchPartialsOffset + 8 * kReduceMaxBlocks;
-constexpr std::size_t kCutScratchBytes = kCutScratchTilesOffset + 4 * kCutScratchTiles;  // 4 MiB + 8.25 KiB
+constexpr std::size_t kCutScratchBytes = kCutScratchTilesOffset + 4 * kCutScratchTiles;  // 4 MiB + 8 KiB
 constexpr int kCutScratchDevices = 64;
 
 std::mutex& cut_scratch_mutex() {
@@ -2767,10 +2763,9 @@ int gpart_cut_noalloc(gpart_ctx* ctx, const gpart_csr_view* g, const int32_t* la
         }
         if (!base) throw Error(GPART_ERR_RUNTIME, "gpart_cut_noalloc: scratch of this device was not set up");
         auto* bytes = static_cast<unsigned char*>(base);
-        auto* total = reinterpret_cast<unsigned long long*>(bytes + kCutScratchTotalOffset);
         auto* partials = reinterpret_cast<unsigned long long*>(bytes + kCutScratchPartialsOffset);
         auto* tile_row = reinterpret_cast<std::int32_t*>(bytes + kCutScratchTilesOffset);
-        GPART_WIDTH_DISPATCH(g->width, OpsT::cut_with(ctx, g, labels, total, tile_row, partials, cut));
+        GPART_WIDTH_DISPATCH(g->width, OpsT::cut_with(ctx, g, labels, tile_row, partials, cut));
     });
 }
 
@@ -2927,39 +2922,19 @@ int gpart_refine_rebalance_round(gpart_ctx* ctx, const gpart_csr_view* g, const 
 
 int gpart_max_edge_weight(gpart_ctx* ctx, const gpart_csr_view* g, uint64_t* maximum) {
     return guarded([&] {
-        Scratch<unsigned long long> out(ctx, 1);
-        fill_bytes(ctx, out.get(), 0, 8);
-        if (g->m > 0) {
-            if (g->width == GPART_WIDTH_STANDARD)
-                device_reduce<unsigned long long>(
-                    ctx, WidenLoad<std::uint32_t>{static_cast<const std::uint32_t*>(g->edge_weights)}, g->m, MaxU64{},
-                    out.get());
-            else
-                device_reduce<unsigned long long>(
-                    ctx, WidenLoad<std::uint64_t>{static_cast<const std::uint64_t*>(g->edge_weights)}, g->m, MaxU64{},
-                    out.get());
-        }
-        *maximum = read_scalar(ctx, out.get());
+        unsigned long long h = 0;
+        if (g->m > 0)
+            with_weights(g->width, g->edge_weights, [&](auto load) { reduce_read<MaxU64>(ctx, load, g->m, &h); });
+        *maximum = h;
     });
 }
 
 int gpart_edge_weight_sum(gpart_ctx* ctx, const gpart_csr_view* g, uint64_t* checked, uint64_t* limited) {
     return guarded([&] {
-        Scratch<unsigned long long> out(ctx, 2);
-        fill_bytes(ctx, out.get(), 0, 16);
-        if (g->m > 0) {
-            if (g->width == GPART_WIDTH_STANDARD) {
-                const WidenLoad<std::uint32_t> load{static_cast<const std::uint32_t*>(g->edge_weights)};
-                device_reduce<unsigned long long>(ctx, load, g->m, CheckedSumU64{}, out.get());
-                device_reduce<unsigned long long>(ctx, load, g->m, LimitedSumU64{}, out.get() + 1);
-            } else {
-                const WidenLoad<std::uint64_t> load{static_cast<const std::uint64_t*>(g->edge_weights)};
-                device_reduce<unsigned long long>(ctx, load, g->m, CheckedSumU64{}, out.get());
-                device_reduce<unsigned long long>(ctx, load, g->m, LimitedSumU64{}, out.get() + 1);
-            }
-        }
-        unsigned long long h[2];
-        read_back(ctx, h, out.get(), sizeof(h));
+        unsigned long long h[2] = {0, 0};
+        if (g->m > 0)
+            with_weights(g->width, g->edge_weights,
+                         [&](auto load) { reduce_read<CheckedSumU64, LimitedSumU64>(ctx, load, g->m, h); });
         *checked = h[0];
         *limited = h[1];
     });
@@ -2968,23 +2943,10 @@ int gpart_edge_weight_sum(gpart_ctx* ctx, const gpart_csr_view* g, uint64_t* che
 int gpart_vertex_weight_stats(gpart_ctx* ctx, const gpart_csr_view* g, uint64_t* total, uint64_t* maximum,
                               uint64_t* minimum) {
     return guarded([&] {
-        Scratch<unsigned long long> out(ctx, 3);
-        fill_bytes(ctx, out.get(), 0, 24);
-        if (g->n > 0) {
-            if (g->width == GPART_WIDTH_STANDARD) {
-                const WidenLoad<std::uint32_t> load{static_cast<const std::uint32_t*>(g->vertex_weights)};
-                device_reduce<unsigned long long>(ctx, load, g->n, CheckedSumU64{}, out.get());
-                device_reduce<unsigned long long>(ctx, load, g->n, MaxU64{}, out.get() + 1);
-                device_reduce<unsigned long long>(ctx, load, g->n, MinU64{}, out.get() + 2);
-            } else {
-                const WidenLoad<std::uint64_t> load{static_cast<const std::uint64_t*>(g->vertex_weights)};
-                device_reduce<unsigned long long>(ctx, load, g->n, CheckedSumU64{}, out.get());
-                device_reduce<unsigned long long>(ctx, load, g->n, MaxU64{}, out.get() + 1);
-                device_reduce<unsigned long long>(ctx, load, g->n, MinU64{}, out.get() + 2);
-            }
-        }
-        unsigned long long h[3];
-        read_back(ctx, h, out.get(), sizeof(h));
+        unsigned long long h[3] = {0, 0, 0};
+        if (g->n > 0)
+            with_weights(g->width, g->vertex_weights,
+                         [&](auto load) { reduce_read<CheckedSumU64, MaxU64, MinU64>(ctx, load, g->n, h); });
         *total = h[0];
         *maximum = h[1];
         *minimum = h[2];

@@ -147,6 +147,15 @@ void wait_status(gpart_ctx* ctx, std::uint64_t seq) {
         throw Error(GPART_ERR_RUNTIME, "round status did not reach the host");
 }
 
+Publication publication(gpart_ctx* ctx) {
+    return Publication{reinterpret_cast<unsigned long long*>(ctx->status_device), ctx->status_counter};
+}
+
+void read_published(gpart_ctx* ctx, void* host, std::size_t bytes) {
+    wait_status(ctx, ++ctx->status_seq);
+    std::memcpy(host, ctx->status_host + 1, bytes);
+}
+
 // Small read-backs: a one-wave kernel copies the bytes into the fine-grained
 // status words and stores the sequence number after them; the host polls for it
 // (no copy engine, no blocking wait).
@@ -268,8 +277,8 @@ int gpart_ctx_create(int device, gpart_ctx** out) {
                                           hipHostMallocCoherent | hipHostMallocMapped));
             GPART_HIP_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&ctx->status_device), ctx->status_host, 0));
             std::memset(ctx->status_host, 0, kStatusWords * 8);
-            GPART_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&ctx->status_counter), sizeof(unsigned long long)));
-            GPART_HIP_CHECK(hipMemset(ctx->status_counter, 0, sizeof(unsigned long long)));
+            GPART_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&ctx->status_counter), 2 * sizeof(unsigned long long)));
+            GPART_HIP_CHECK(hipMemset(ctx->status_counter, 0, 2 * sizeof(unsigned long long)));
             SegmentSource source;
             source.allocate = [ctx](std::size_t bytes) -> void* {
                 void* p = nullptr;
