@@ -5,7 +5,7 @@
 // 1336-1339,1550; src/refine_incremental.cuh:277).
 //
 // Radix sort: stable LSD over 8-bit digits. Per pass:
-//   1. digit histogram of each 2048-key tile (LDS counters);
+//   1. digit histogram of each 2048- or 4096-key tile (LDS counters);
 //   2. exclusive scan of the digit-major [256 x tiles] histogram (global bases);
 //   3. scatter: each wave ranks its keys with a 64-lane multisplit (eight
 //      ballots give the lanes sharing a digit), waves are combined in LDS, the
@@ -19,22 +19,36 @@
 namespace gpart_hip {
 namespace {
 
-constexpr int kSortThreads = 256;
-constexpr int kSortWaves = kSortThreads / kWave;
-constexpr int kSortItems = 8;  // per lane
-constexpr int kSortTile = kSortThreads * kSortItems;
+// A tile's shape: the threads of its workgroup and the keys of each.
+template <int Threads, int Items>
+struct Tile {
+    static constexpr int kThreads = Threads;
+    static constexpr int kItems = Items;
+    static constexpr int kWaves = Threads / kWave;
+    static constexpr int kKeys = Threads * Items;
+    __device__ static __forceinline__ std::int64_t item(int wave, int it, int lane) {
+        return static_cast<std::int64_t>(wave) * (kWave * Items) + it * kWave + lane;
+    }
+};
+using SmallTile = Tile<256, 8>;
+using LargeTile = Tile<512, 8>;
+// From here on large tiles: a digit's run in a tile is twice as long and the digit-major
+// histograms, stored and scanned 4 bytes apart by tiles, are half as many. A pass over
+// 32 Mi keys, histogram and scatter: 84 + 174 -> 69 + 166 us, with 4-byte values
+// 84 + 296 -> 69 + 265; tiles of 8,192 keys lose more in the scatter (176, 213) than the
+// histogram gains (57). 4 Mi keys: 10.4 + 21.0 -> 7.5 + 20.9 us; 1 Mi keys: no difference;
+// smaller sorts need the tiles to fill the chip.
+constexpr std::int64_t kLargeSort = std::int64_t{1} << 21;
 constexpr int kDigits = 256;
 // Sorts of at most this many tiles scan the digit histograms inside each scatter
 // workgroup (at most 256 x 64 loads) instead of two scan launches per pass.
 constexpr std::int64_t kInlineHistogramTiles = 64;
 
-__device__ __forceinline__ std::int64_t tile_item(int wave, int it, int lane) {
-    return static_cast<std::int64_t>(wave) * (kWave * kSortItems) + it * kWave + lane;
-}
-
-__global__ void __launch_bounds__(kSortThreads) radix_histogram_kernel(const std::uint64_t* keys, std::int64_t n, int shift,
-                                                                       std::uint64_t mask, std::uint32_t* hist,
-                                                                       std::int64_t tiles) {
+template <typename S>
+__global__ void __launch_bounds__(S::kThreads) radix_histogram_kernel(const std::uint64_t* keys, std::int64_t n, int shift,
+                                                                      std::uint64_t mask, std::uint32_t* hist,
+                                                                      std::int64_t tiles) {
+    constexpr int kSortThreads = S::kThreads, kSortWaves = S::kWaves, kSortItems = S::kItems, kSortTile = S::kKeys;
     __shared__ std::uint32_t counts[kSortWaves][kDigits];
     for (int i = threadIdx.x; i < kSortWaves * kDigits; i += kSortThreads)
         (&counts[0][0])[i] = 0;
@@ -43,7 +57,7 @@ __global__ void __launch_bounds__(kSortThreads) radix_histogram_kernel(const std
     const std::int64_t tile_start = static_cast<std::int64_t>(blockIdx.x) * kSortTile;
 #pragma unroll
     for (int it = 0; it < kSortItems; ++it) {
-        const std::int64_t idx = tile_start + tile_item(wave, it, lane);
+        const std::int64_t idx = tile_start + S::item(wave, it, lane);
         if (idx < n) {
             const int d = static_cast<int>((keys[idx] >> shift) & mask);
             atomicAdd(&counts[wave][d], 1U);
@@ -61,12 +75,13 @@ __global__ void __launch_bounds__(kSortThreads) radix_histogram_kernel(const std
 // offsets: the digit-major exclusive scan of the tiles' histograms, or, with
 // raw_histogram, the histograms themselves, which each workgroup then scans
 // for its own tile (grids of at most kInlineHistogramTiles tiles).
-template <typename V, bool HasValues>
-__global__ void __launch_bounds__(kSortThreads) radix_scatter_kernel(const std::uint64_t* keys_in, std::uint64_t* keys_out,
-                                                                     const V* values_in, V* values_out, std::int64_t n,
-                                                                     int shift, std::uint64_t mask,
-                                                                     const std::uint32_t* offsets, std::int64_t tiles,
-                                                                     int raw_histogram) {
+template <typename S, typename V, bool HasValues>
+__global__ void __launch_bounds__(S::kThreads) radix_scatter_kernel(const std::uint64_t* keys_in, std::uint64_t* keys_out,
+                                                                    const V* values_in, V* values_out, std::int64_t n,
+                                                                    int shift, std::uint64_t mask,
+                                                                    const std::uint32_t* offsets, std::int64_t tiles,
+                                                                    int raw_histogram) {
+    constexpr int kSortThreads = S::kThreads, kSortWaves = S::kWaves, kSortItems = S::kItems, kSortTile = S::kKeys;
     __shared__ std::uint32_t wave_counts[kSortWaves][kDigits];
     __shared__ std::uint32_t digit_start[kDigits + 1];
     __shared__ std::uint32_t global_base[kDigits];
@@ -85,27 +100,30 @@ __global__ void __launch_bounds__(kSortThreads) radix_scatter_kernel(const std::
     V value[kSortItems];
     int digit[kSortItems];
     std::uint32_t rank[kSortItems];
-    const std::uint64_t below = lanemask_lt();
 #pragma unroll
     for (int it = 0; it < kSortItems; ++it) {
-        const std::int64_t idx = tile_start + tile_item(wave, it, lane);
+        const std::int64_t idx = tile_start + S::item(wave, it, lane);
         const bool valid = idx < n;
         key[it] = valid ? keys_in[idx] : 0;
         if constexpr (HasValues) value[it] = valid ? values_in[idx] : V{};
         const int d = valid ? static_cast<int>((key[it] >> shift) & mask) : 0;
         digit[it] = valid ? d : -1;
-        std::uint64_t peers = __ballot(valid);
+        // the lanes of the same digit, bit by bit: ~(ballot ^ own bit), in 32-bit halves
+        const std::uint64_t in_tile = __ballot(valid);
+        unsigned low = static_cast<unsigned>(in_tile), high = static_cast<unsigned>(in_tile >> 32);
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
-            const std::uint64_t bits = __ballot((d >> b) & 1);
-            peers &= ((d >> b) & 1) ? bits : ~bits;
+            const int own = (d << (31 - b)) >> 31;  // all ones where bit b is set
+            const std::uint64_t set = __ballot(own != 0);
+            low &= ~(static_cast<unsigned>(set) ^ static_cast<unsigned>(own));
+            high &= ~(static_cast<unsigned>(set >> 32) ^ static_cast<unsigned>(own));
         }
         std::uint32_t before = 0;
         if (valid) before = wave_counts[wave][d];
-        const std::uint32_t mine = static_cast<std::uint32_t>(__popcll(peers & below));
+        const std::uint32_t mine = __builtin_amdgcn_mbcnt_hi(high, __builtin_amdgcn_mbcnt_lo(low, 0U));
         rank[it] = before + mine;
         // the lowest peer publishes the new running count
-        if (valid && mine == 0) wave_counts[wave][d] = before + static_cast<std::uint32_t>(__popcll(peers));
+        if (valid && mine == 0) wave_counts[wave][d] = before + __popc(low) + __popc(high);
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
@@ -168,7 +186,7 @@ __global__ void __launch_bounds__(kSortThreads) radix_scatter_kernel(const std::
 // keys: 5.6, 6.4, 9.8 and 21 us (a bitonic network in one workgroup: 17, 25, 46 and 96);
 // of 16,384 keys 61 us and of 32,768 keys 210 us, where the passes of 8 bits below take
 // 160 and 170 us, 90 us for 31 bits and 45 us for 16: the line is drawn at 8,192.
-constexpr int kRankSortMax = 4 * kSortTile;
+constexpr int kRankSortMax = 8192;
 constexpr int kRankEntries = 16;
 constexpr int kRankWaves = 16;
 
@@ -239,11 +257,42 @@ __global__ void __launch_bounds__(kRankWaves* kWave) rank_sort_kernel(const std:
     }
 }
 
+template <typename S, typename V, bool HasValues>
+bool radix_passes(gpart_ctx* ctx, std::uint64_t* keys, std::uint64_t* keys_alt, V* values, V* values_alt,
+                  std::int64_t n, int begin_bit, int end_bit) {
+    const std::int64_t tiles = (n + S::kKeys - 1) / S::kKeys;
+    Scratch<std::uint32_t> hist(ctx, tiles * kDigits);
+    std::uint64_t* src_k = keys;
+    std::uint64_t* dst_k = keys_alt;
+    V* src_v = values;
+    V* dst_v = values_alt;
+    bool in_alt = false;
+    for (int shift = begin_bit; shift < end_bit; shift += 8) {
+        const int bits = end_bit - shift < 8 ? end_bit - shift : 8;
+        const std::uint64_t mask = (1ULL << bits) - 1;
+        hipLaunchKernelGGL(radix_histogram_kernel<S>, dim3(static_cast<unsigned>(tiles)), dim3(S::kThreads), 0,
+                           ctx->stream, src_k, n, shift, mask, hist.get(), tiles);
+        GPART_LAUNCH_CHECK();
+        const bool raw = tiles <= kInlineHistogramTiles;
+        if (!raw)
+            device_scan<std::uint32_t, SumOp<std::uint32_t>>(ctx, ArrayLoad<std::uint32_t>{hist.get()},
+                                                             ExclusiveStore<std::uint32_t>{hist.get()},
+                                                             tiles * kDigits, SumOp<std::uint32_t>{});
+        hipLaunchKernelGGL((radix_scatter_kernel<S, V, HasValues>), dim3(static_cast<unsigned>(tiles)), dim3(S::kThreads),
+                           0, ctx->stream, src_k, dst_k, src_v, dst_v, n, shift, mask, hist.get(), tiles, raw ? 1 : 0);
+        GPART_LAUNCH_CHECK();
+        std::swap(src_k, dst_k);
+        std::swap(src_v, dst_v);
+        in_alt = !in_alt;
+    }
+    return in_alt;
+}
+
 template <typename V, bool HasValues>
 bool radix_sort_impl(gpart_ctx* ctx, std::uint64_t* keys, std::uint64_t* keys_alt, V* values, V* values_alt,
                      std::int64_t n, int begin_bit, int end_bit) {
     if (n <= 1 || end_bit <= begin_bit) return false;
-    if (n > (std::int64_t{1} << 32) - kSortTile)
+    if (n > (std::int64_t{1} << 32) - SmallTile::kKeys)
         throw Error(GPART_ERR_INVALID_ARGUMENT, "radix sort supports fewer than 2^32 keys per call");
     if (n <= kRankSortMax) {
         const int width = end_bit - begin_bit;
@@ -258,32 +307,9 @@ bool radix_sort_impl(gpart_ctx* ctx, std::uint64_t* keys, std::uint64_t* keys_al
         GPART_LAUNCH_CHECK();
         return true;
     }
-    const std::int64_t tiles = (n + kSortTile - 1) / kSortTile;
-    Scratch<std::uint32_t> hist(ctx, tiles * kDigits);
-    std::uint64_t* src_k = keys;
-    std::uint64_t* dst_k = keys_alt;
-    V* src_v = values;
-    V* dst_v = values_alt;
-    bool in_alt = false;
-    for (int shift = begin_bit; shift < end_bit; shift += 8) {
-        const int bits = end_bit - shift < 8 ? end_bit - shift : 8;
-        const std::uint64_t mask = (1ULL << bits) - 1;
-        hipLaunchKernelGGL(radix_histogram_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kSortThreads), 0,
-                           ctx->stream, src_k, n, shift, mask, hist.get(), tiles);
-        GPART_LAUNCH_CHECK();
-        const bool raw = tiles <= kInlineHistogramTiles;
-        if (!raw)
-            device_scan<std::uint32_t, SumOp<std::uint32_t>>(ctx, ArrayLoad<std::uint32_t>{hist.get()},
-                                                             ExclusiveStore<std::uint32_t>{hist.get()},
-                                                             tiles * kDigits, SumOp<std::uint32_t>{});
-        hipLaunchKernelGGL((radix_scatter_kernel<V, HasValues>), dim3(static_cast<unsigned>(tiles)), dim3(kSortThreads),
-                           0, ctx->stream, src_k, dst_k, src_v, dst_v, n, shift, mask, hist.get(), tiles, raw ? 1 : 0);
-        GPART_LAUNCH_CHECK();
-        std::swap(src_k, dst_k);
-        std::swap(src_v, dst_v);
-        in_alt = !in_alt;
-    }
-    return in_alt;
+    if (n < kLargeSort)
+        return radix_passes<SmallTile, V, HasValues>(ctx, keys, keys_alt, values, values_alt, n, begin_bit, end_bit);
+    return radix_passes<LargeTile, V, HasValues>(ctx, keys, keys_alt, values, values_alt, n, begin_bit, end_bit);
 }
 
 struct FlagLoad {
