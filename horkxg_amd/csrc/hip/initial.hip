@@ -254,6 +254,16 @@ __global__ void __launch_bounds__(256) depth_step_kernel(DepthTasks dt, const in
     if (threadIdx.x == 0) partials[blockIdx.x] = block_partial(vm, 0, 8);
 }
 
+// The last normalisation of one task, in place.
+__global__ void __launch_bounds__(256) depth_normalize_kernel(int count, const int* ids, double* x,
+                                                              const Moments* partials, int blocks) {
+    __shared__ double shared8[24];
+    __shared__ Norm shared_norm;
+    const Norm norm = finish_block(partials, blocks, shared8, &shared_norm);
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count) x[ids[i]] = normalized(x, ids[i], norm);
+}
+
 // The last normalisation, the (x, id) sort (:143-148, :230), the weight prefix and
 // feasible split (:231-248) and the label assignment (:149-153): one workgroup per
 // task, emitting the child tasks of the next depth.
@@ -292,8 +302,7 @@ __global__ void __launch_bounds__(kBatchThreads) depth_finish_kernel(DepthTasks 
 // the LDS reads. Bisection of a 7,429-vertex weighted mesh into 32, with its four depths
 // below the root: 3.29 -> 2.33 ms.
 constexpr int kSoloThreads = 1024;
-constexpr int kSoloRows = kMaxBatchedTask / kSoloThreads;  // rows per thread
-constexpr int kSoloGroups = kMaxBatchedTask / kWave;       // groups of 64 rows, one width each
+constexpr int kSoloGroups = kMaxBatchedTask / kWave;  // groups of 64 rows, one width each
 // Entries of a task, estimated by its share of the graph's vertices, up to which the
 // solo form is taken. Weighted 3D meshes, FP64, a depth of tasks of 3,700 vertices and
 // 21,000 entries: 500 us, the launch form 500; of 1,860 and 10,500: 300 and 500; of 930
@@ -548,6 +557,13 @@ __global__ void __launch_bounds__(kSoloThreads) depth_solo_kernel(
     if (failed && t == 0) atomicMax(status, failed);
 }
 
+// Single tasks of at most this size take their steps through the depth's fused launches:
+// one per step, of 5.5 us at 7,429 vertices, where step, moments and normalisation were
+// three, of 9.7 us. Each workgroup reads all partials, 3 bytes a vertex, so the form's
+// cost grows with the square of the size: the line is where a step's reads reach 25 MB
+// of L2 traffic.
+constexpr int kMaxFusedTask = 8192;
+
 template <typename O, typename W>
 void plain_task(gpart_ctx* ctx, const gpart_csr_view* g, const int32_t* labels, int32_t* order,
                 const std::uint64_t* vertex_weights, const gpart_bisect_task* task, uint32_t seed, double* x,
@@ -564,22 +580,43 @@ void plain_task(gpart_ctx* ctx, const gpart_csr_view* g, const int32_t* labels, 
     Scratch<unsigned long long> entries(ctx, 1);
     fill_bytes(ctx, entries.get(), 0, 8);
     profile_begin(ctx, GPART_PROFILE_SPECTRAL);
-    hipLaunchKernelGGL((spectral_start_kernel<O, W>), dim3(spectral_blocks), dim3(256), 0, ctx->stream, count, ids,
-                       labels, task->first_part, off, g->neighbors, w, degree, x,
-                       seed ^ static_cast<unsigned>(task->first_part), partials.get(),
-                       ctx->profile[GPART_PROFILE_SPECTRAL].enabled ? entries.get() : nullptr);
-    hipLaunchKernelGGL(finish_moments_kernel, dim3(1), dim3(256), 0, ctx->stream, spectral_blocks, partials.get(),
-                       norm.get());
-    GPART_LAUNCH_CHECK();
-    for (int iteration = 0; iteration <= 64; ++iteration) {
-        hipLaunchKernelGGL(normalize_kernel, dim3(blocks), dim3(256), 0, ctx->stream, count, ids, x, norm.get());
-        if (iteration == 64) break;
-        hipLaunchKernelGGL((spectral_step_kernel<O, W, double>), dim3(spectral_blocks), dim3(256), 0, ctx->stream,
-                           count, ids, labels, task->first_part, off, g->neighbors, w, degree, x, y, partials.get());
+    unsigned long long* scanned = ctx->profile[GPART_PROFILE_SPECTRAL].enabled ? entries.get() : nullptr;
+    if (count <= kMaxFusedTask) {
+        DepthTasks dt{};
+        dt.count = 1;
+        dt.first_block[1] = spectral_blocks;
+        dt.task[0] = *task;
+        Scratch<Moments> partials_alt(ctx, spectral_blocks);
+        Moments* p = partials.get();
+        Moments* q = partials_alt.get();
+        hipLaunchKernelGGL((depth_start_kernel<O, W, double>), dim3(spectral_blocks), dim3(256), 0, ctx->stream, dt,
+                           order, labels, off, g->neighbors, w, seed, degree, x, p, scanned);
+        for (int step = 0; step < 64; ++step) {
+            hipLaunchKernelGGL((depth_step_kernel<O, W, double>), dim3(spectral_blocks), dim3(256), 0, ctx->stream, dt,
+                               order, labels, off, g->neighbors, w, degree, x, y, p, q);
+            std::swap(x, y);
+            std::swap(p, q);
+        }
+        hipLaunchKernelGGL(depth_normalize_kernel, dim3(blocks), dim3(256), 0, ctx->stream, count, ids, x, p,
+                           spectral_blocks);
+        GPART_LAUNCH_CHECK();
+    } else {
+        hipLaunchKernelGGL((spectral_start_kernel<O, W>), dim3(spectral_blocks), dim3(256), 0, ctx->stream, count, ids,
+                           labels, task->first_part, off, g->neighbors, w, degree, x,
+                           seed ^ static_cast<unsigned>(task->first_part), partials.get(), scanned);
         hipLaunchKernelGGL(finish_moments_kernel, dim3(1), dim3(256), 0, ctx->stream, spectral_blocks, partials.get(),
                            norm.get());
         GPART_LAUNCH_CHECK();
-        std::swap(x, y);
+        for (int iteration = 0; iteration <= 64; ++iteration) {
+            hipLaunchKernelGGL(normalize_kernel, dim3(blocks), dim3(256), 0, ctx->stream, count, ids, x, norm.get());
+            if (iteration == 64) break;
+            hipLaunchKernelGGL((spectral_step_kernel<O, W, double>), dim3(spectral_blocks), dim3(256), 0, ctx->stream,
+                               count, ids, labels, task->first_part, off, g->neighbors, w, degree, x, y, partials.get());
+            hipLaunchKernelGGL(finish_moments_kernel, dim3(1), dim3(256), 0, ctx->stream, spectral_blocks, partials.get(),
+                               norm.get());
+            GPART_LAUNCH_CHECK();
+            std::swap(x, y);
+        }
     }
     profile_end(ctx, GPART_PROFILE_SPECTRAL, 0.0);
     if (ctx->profile[GPART_PROFILE_SPECTRAL].enabled)

@@ -45,6 +45,10 @@ CASES = {
     "n1023": (lattice, (1023, 2), "standard"),
     "n1025": (lattice, (1025, 1), "big"),
     "n4096": (lattice, (4096, 2), "standard"),
+    # roots too large for a depth: steps of one launch up to 8192 vertices, of three above
+    "n4097": (lattice, (4097, 2), "big"),
+    "n8192": (lattice, (8192, 1), "standard"),
+    "n8193": (lattice, (8193, 1), "standard"),
     # slots per row: 8, 12, 16, 24, 32, more than 32 terms
     "deg8": (lattice, (700, 4), "standard"),
     "deg12": (lattice, (700, 6), "standard"),
