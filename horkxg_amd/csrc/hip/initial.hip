@@ -15,12 +15,12 @@
 //
 // Plain form: the reference's launch structure, one task at a time (start, then
 // per step: SpMV, finish_moments, normalize).
-// Batched form: all tasks of one recursion depth share every launch (small sparse
-// tasks a single one, the solo form below). Else a depth is
-// 66 launches whatever its task count: start, 64 steps (each also finishing the
-// previous step's moments and normalising on read), and one 1024-thread
-// workgroup per task for the (x, id) sort (LDS bitonic), the weight prefix, the
-// feasible split and the label assignment, emitting the child tasks.
+// Batched form: all tasks of one recursion depth share every launch. Small sparse tasks
+// take a single one (the solo form below), else a depth is 66 launches whatever its task
+// count: start, 64 steps (each also finishing the previous step's moments and
+// normalising on read), and one 1024-thread workgroup per task for the (x, id) sort
+// (LDS bitonic), the weight prefix, the feasible split and the label assignment,
+// emitting the child tasks.
 #include "internal.hpp"
 #include "scan.hpp"
 #include "spectral_device.hpp"
