@@ -309,6 +309,8 @@ constexpr int kSoloGroups = kMaxBatchedTask / kWave;  // groups of 64 rows, one 
 // and 5,300: 190 and 490; of 460 and 2,600: 145 and 490.
 constexpr double kSoloEntries = 16384;
 
+constexpr int kSoloWidth = 256;  // longest row of a group with slots
+
 struct SoloTasks {
     int count;
     long long first_slot[kMaxDepthTasks + 1];  // of each task's slots, in rows of 64
@@ -409,10 +411,11 @@ __global__ void __launch_bounds__(kSoloThreads) depth_solo_kernel(
     if (entries && lane == 0 && scanned) atomicAdd(entries, scanned);
     __syncthreads();  // widths and positions
     if (wave == 0) {
-        const int width = padded_width(sh.width[lane]);
+        const int padded = padded_width(sh.width[lane]);
+        const int width = padded <= kSoloWidth ? padded : 0;  // a long row's group does without
         const long long inclusive = wave_scan(static_cast<long long>(width));
         const long long first = st.first_slot[blockIdx.x] + inclusive - width;
-        sh.slots[lane] = first + width <= st.first_slot[blockIdx.x + 1] ? first : -1;
+        sh.slots[lane] = width > 0 && first + width <= st.first_slot[blockIdx.x + 1] ? first : -1;
     }
     __syncthreads();
     static_assert(kSoloGroups == kWave, "one wave places the groups");
@@ -476,13 +479,26 @@ __global__ void __launch_bounds__(kSoloThreads) depth_solo_kernel(
         const std::uint64_t* at = slot + sh.slots[g] * kWave;
         if (bytes == 4) return stored(reinterpret_cast<const std::uint32_t*>(at) + lane);
         if (bytes == 8) return stored(at + lane);
-        return tree_sum<A, 32, 4>(width, [&](int first, A (&acc)[4]) {
-            W w[4];
-            int pos[4];
-            resolve(r, first, w, pos);
-#pragma unroll
-            for (int l = 0; l < 4; ++l) acc[l] = term(w[l], pos[l], acc[l]);
-        });
+        // without slots a half-wave takes a row, as in the launch form
+        A result = A(0);
+#pragma unroll 1
+        for (int first = 0; first < (width > 0 ? kWave : 0); first += 2) {
+            const int row = g * kWave + first + lane / kHalf;
+            A acc = A(0);
+            if (row < count) {
+                const int v = ids[row];
+                const auto end = static_cast<std::int64_t>(offsets[v + 1]);
+                for (std::int64_t e = static_cast<std::int64_t>(offsets[v]) + lane % kHalf; e < end; e += kHalf) {
+                    const int u = neighbors[e];
+                    if (labels[u] == group) acc = term(weights[e], position[u], acc);
+                }
+            }
+            acc = tree32(acc);
+            const A even = __shfl(acc, 0, kWave), odd = __shfl(acc, kHalf, kWave);
+            if (lane == first) result = even;
+            if (lane == first + 1) result = odd;
+        }
+        return result;
     };
     // a row's moments into its block of eight rows
     auto absorb = [&](int r, double mass, double a) {

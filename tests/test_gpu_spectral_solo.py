@@ -58,6 +58,8 @@ CASES = {
     "deg34": (lattice, (470, 17), "standard"),
     # one long row per wave: some groups find no room for slots
     "hubs": (lambda: lattice(4096, 1, hubs=range(5, 4096, 64), hub_degree=60), (), "standard"),
+    # a row too long for slots, between groups that have them
+    "hub": (lambda: lattice(3000, 1, hubs=(700, 2100), hub_degree=900), (), "big"),
     # weights beyond a 4-byte slot, at its edge, and beyond an 8-byte one
     "wide": (lambda: lattice(300, 3, weight=lambda a, b: 2**20 - 1 + (a + b) % 2), (), "standard"),
     "wide_big": (lambda: lattice(300, 3, weight=lambda a, b: 2**40 + a), (), "big"),
