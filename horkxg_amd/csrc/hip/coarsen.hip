@@ -1153,7 +1153,7 @@ __global__ void map_and_weights_kernel(std::int64_t n, const std::int32_t* clust
 template <typename O, typename W, int G>
 __global__ void record_bound_kernel(std::int64_t count, const std::int32_t* list, const O* offsets,
                                     const std::int32_t* neighbors, const W* weights,
-                                    unsigned long long* row_bounds, unsigned long long* meta) {
+                                    unsigned long long* row_bounds, unsigned long long* unsorted_rows) {
     const std::int64_t group = (static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / G;
     const int sub = threadIdx.x & (G - 1);
     if (group >= count) return;
@@ -1174,7 +1174,7 @@ __global__ void record_bound_kernel(std::int64_t count, const std::int32_t* list
     unsorted = group_any<G>(unsorted);
     if (sub == 0) {
         row_bounds[v] = degree;
-        if (unsorted) atomicOr(meta + 1, 1ULL);  // rare: only unsorted inputs write it
+        if (unsorted) atomicOr(unsorted_rows, 1ULL);  // rare: only unsorted inputs write it
     }
 }
 
@@ -1436,8 +1436,8 @@ void record_bounds_impl(gpart_ctx* ctx, const gpart_csr_view* g, std::uint64_t* 
                         std::uint64_t* maximum, int* unsorted) {
     unsigned long long h[2] = {0, 0};  // unsorted, maximum
     if (g->n > 0) {
-        Scratch<unsigned long long> found(ctx, 1);
-        fill_bytes(ctx, found.get(), 0, 8);
+        Scratch<unsigned long long> unsorted_rows(ctx, 1);
+        fill_bytes(ctx, unsorted_rows.get(), 0, 8);
         Scratch<std::int32_t> low(ctx, g->n), medium(ctx, g->n), high(ctx, g->n);
         gpart_degree_classes c{low.get(), medium.get(), high.get(), 0, 0, 0, 0, 0, 0};
         build_classes<O, W>(ctx, g, &c);
@@ -1446,15 +1446,15 @@ void record_bounds_impl(gpart_ctx* ctx, const gpart_csr_view* g, std::uint64_t* 
         auto* rb = reinterpret_cast<unsigned long long*>(row_bounds);
         if (c.low_count)
             hipLaunchKernelGGL((record_bound_kernel<O, W, 8>), dim3(grid_for(c.low_count * 8)), dim3(kBlock), 0,
-                               ctx->stream, c.low_count, c.low, off, g->neighbors, w, rb, found.get());
+                               ctx->stream, c.low_count, c.low, off, g->neighbors, w, rb, unsorted_rows.get());
         if (c.medium_count)
             hipLaunchKernelGGL((record_bound_kernel<O, W, 64>), dim3(grid_for(c.medium_count * 64)), dim3(kBlock), 0,
-                               ctx->stream, c.medium_count, c.medium, off, g->neighbors, w, rb, found.get());
+                               ctx->stream, c.medium_count, c.medium, off, g->neighbors, w, rb, unsorted_rows.get());
         if (c.high_count)
             hipLaunchKernelGGL((record_bound_kernel<O, W, 64>), dim3(grid_for(c.high_count * 64)), dim3(kBlock), 0,
-                               ctx->stream, c.high_count, c.high, off, g->neighbors, w, rb, found.get());
+                               ctx->stream, c.high_count, c.high, off, g->neighbors, w, rb, unsorted_rows.get());
         GPART_LAUNCH_CHECK();
-        reduce_read<MaxU64>(ctx, U64Load{rb}, g->n, h, found.get(), 1);
+        reduce_read<MaxU64>(ctx, U64Load{rb}, g->n, h, unsorted_rows.get(), 1);
     }
     *maximum = h[1];
     *unsorted = h[0] != 0;
