@@ -2190,15 +2190,16 @@ struct Ops {
                                                               lds <= kRowsPairLds ? 2 * kRowsGroups : kRowsGroups));
     }
 
-    // Before the first round of a level.
+    // Before a round; the round that completes leaves the handle ready.
     static void prepare_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
                              gpart_refine_rows* r, const std::int32_t* labels, int k, C* cache) {
         if constexpr (sizeof(C) == 4) {
-            if (r->ready) return;
-            hipLaunchKernelGGL(rows_prepare_kernel, dim3(std::min<unsigned>(grid_for(g->n), kRoundBlocks)), dim3(256), 0,
-                               ctx->stream, row_lists(c, r), g->n, labels, r->states.get(), k, cache);
-            GPART_LAUNCH_CHECK();
-            r->ready = true;
+            if (!r->ready) {
+                hipLaunchKernelGGL(rows_prepare_kernel, dim3(std::min<unsigned>(grid_for(g->n), kRoundBlocks)),
+                                   dim3(256), 0, ctx->stream, row_lists(c, r), g->n, labels, r->states.get(), k, cache);
+                GPART_LAUNCH_CHECK();
+            }
+            r->ready = false;
         }
     }
 
@@ -2828,6 +2829,11 @@ int gpart_refine_rows_create(gpart_ctx* ctx, const gpart_csr_view* g, const gpar
         *rows = nullptr;
         if (cache_bytes != 4 || g->n <= 0 || g->m < kRowsMinDegree * g->n || g->n > kRowsMaxVertices) return;
         auto made = std::make_unique<gpart_refine_rows>();
+        made->n = g->n;
+        made->m = g->m;
+        made->high_count = classes->high_count;
+        made->width = g->width;
+        made->k = k;
         made->form = g->n <= kStateBytes ? kByteState
                      : k <= 8 && g->n <= 2 * kStateBytes ? kNibbleState
                                                          : kMemoryState;
@@ -2847,20 +2853,27 @@ int gpart_refine_rows_create(gpart_ctx* ctx, const gpart_csr_view* g, const gpar
 
 void gpart_refine_rows_destroy(gpart_refine_rows* rows) { delete rows; }
 
+int gpart_refine_rows_reset(gpart_refine_rows* rows) {
+    return guarded([&] {
+        if (!rows) throw Error(GPART_ERR_INVALID_ARGUMENT, "null rows");
+        rows->ready = false;
+    });
+}
+
 int gpart_refine_lp_round_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes,
                                gpart_refine_rows* rows, uint32_t* cache, int32_t* labels, int k, double filter,
                                int32_t* locks, int32_t* targets, int64_t* gains, int32_t* flags,
                                uint64_t* part_weights, gpart_refine_status* status) {
     return guarded([&] {
         if (!rows) throw Error(GPART_ERR_INVALID_ARGUMENT, "null rows");
-        if (k < 1 || k > 32) throw Error(GPART_ERR_INVALID_ARGUMENT, "part count must be in [1, 32]");
-        if (g->n <= 0) throw Error(GPART_ERR_INVALID_ARGUMENT, "refinement round needs vertices");
+        rows->check(g, classes, k);
         GPART_ROWS_DISPATCH(g->width, {
             OpsT::prepare_rows(ctx, g, classes, rows, labels, k, cache);
             OpsT::lp_round(ctx, g, classes, cache, labels, k, filter, locks, targets,
                            reinterpret_cast<long long*>(gains), flags,
                            reinterpret_cast<unsigned long long*>(part_weights), rows, status);
         });
+        rows->ready = true;
     });
 }
 
@@ -2870,14 +2883,14 @@ int gpart_refine_rebalance_round_rows(gpart_ctx* ctx, const gpart_csr_view* g, c
                                       gpart_refine_status* status) {
     return guarded([&] {
         if (!rows) throw Error(GPART_ERR_INVALID_ARGUMENT, "null rows");
-        if (k < 1 || k > 32) throw Error(GPART_ERR_INVALID_ARGUMENT, "part count must be in [1, 32]");
-        if (g->n <= 0) throw Error(GPART_ERR_INVALID_ARGUMENT, "refinement round needs vertices");
+        rows->check(g, classes, k);
         GPART_ROWS_DISPATCH(g->width, {
             OpsT::prepare_rows(ctx, g, classes, rows, labels, k, cache);
             OpsT::rebalance_round(ctx, g, classes, cache, labels, k,
                                   reinterpret_cast<unsigned long long*>(part_weights), capacity, targets, flags,
                                   rows, status);
         });
+        rows->ready = true;
     });
 }
 

@@ -336,11 +336,22 @@ __device__ __forceinline__ long long mover_gain(std::int32_t v, std::int32_t sou
 }  // namespace
 }  // namespace gpart_hip
 
-// A level in this form: the chunk map of its hub rows and the states of its vertices.
+// A level in this form: its sizes, the chunk map of its hub rows and the states of its
+// vertices.
 struct gpart_refine_rows {
+    std::int64_t n, m, high_count;
+    int width, k;
     gpart_hip::HubChunks chunks;
     gpart_hip::Scratch<unsigned char> states;  // n, rounded up to 16
     bool hubs = false;
     int form = gpart_hip::kByteState;
-    bool ready = false;  // states and hub rows are as a round expects them
+    // States and hub rows are as a round expects them: not before the first round, not
+    // after a round that failed, nor once the caller has changed labels.
+    bool ready = false;
+
+    // The arrays' sizes depend on these, so a round of another level is refused.
+    void check(const gpart_csr_view* g, const gpart_degree_classes* c, int parts) const {
+        if (g->n != n || g->m != m || g->width != width || c->high_count != high_count || parts != k)
+            throw gpart_hip::Error(GPART_ERR_INVALID_ARGUMENT, "the rows belong to another level or part count");
+    }
 };

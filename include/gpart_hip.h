@@ -479,11 +479,16 @@ int gpart_refine_rebalance_round(gpart_ctx* ctx, const gpart_csr_view* g,
  * is better served by the cached rounds above (a sparse or very large level, or 8-byte
  * entries); destroy it before its context. cache (n x k 4-byte entries, device) is the rounds'
  * scratch and needs no gpart_refine_build_cache; it stays with one handle. Same
- * labels, part weights and status as the cached rounds; rebuilt is 0. */
+ * labels, part weights and status as the cached rounds; rebuilt is 0. The handle follows
+ * the labels from round to round: a caller that changes them between rounds, or gives
+ * other arrays, calls gpart_refine_rows_reset before the next one (where the cached rounds
+ * need gpart_refine_build_cache again). Rounds of another level's sizes or another k than
+ * the handle's are refused. */
 typedef struct gpart_refine_rows gpart_refine_rows;
 int gpart_refine_rows_create(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes, int k,
                              int cache_bytes, gpart_refine_rows** rows);
 void gpart_refine_rows_destroy(gpart_refine_rows* rows);
+int gpart_refine_rows_reset(gpart_refine_rows* rows);
 int gpart_refine_lp_round_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes,
                                gpart_refine_rows* rows, uint32_t* cache, int32_t* labels, int k, double filter,
                                int32_t* locks, int32_t* targets, int64_t* gains, int32_t* flags,
