@@ -2193,14 +2193,33 @@ struct Ops {
     // Before a round; the round that completes leaves the handle ready.
     static void prepare_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
                              gpart_refine_rows* r, const std::int32_t* labels, int k, C* cache) {
+        if (!r->ready) launch_prepare(ctx, g, c, r, labels, r->states.get(), k, cache);
+        r->ready = false;
+    }
+    static void launch_prepare(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
+                               const gpart_refine_rows* r, const std::int32_t* labels, unsigned char* states, int k,
+                               C* cache) {
         if constexpr (sizeof(C) == 4) {
-            if (!r->ready) {
-                hipLaunchKernelGGL(rows_prepare_kernel, dim3(std::min<unsigned>(grid_for(g->n), kRoundBlocks)),
-                                   dim3(256), 0, ctx->stream, row_lists(c, r), g->n, labels, r->states.get(), k, cache);
-                GPART_LAUNCH_CHECK();
-            }
-            r->ready = false;
+            hipLaunchKernelGGL(rows_prepare_kernel, dim3(std::min<unsigned>(grid_for(g->n), kRoundBlocks)), dim3(256), 0,
+                               ctx->stream, row_lists(c, r), g->n, labels, states, k, cache);
+            GPART_LAUNCH_CHECK();
         }
+    }
+
+    // The entries in which the rows that the next round will sum, from the states and over
+    // the hub rows as the last one left them, differ from the expected ones.
+    static std::int64_t check_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
+                                   const gpart_refine_rows* r, const std::int32_t* labels, int k, C* cache,
+                                   const unsigned long long* part_weights, std::uint64_t capacity,
+                                   const unsigned* expected) {
+        unsigned long long differing = 0;
+        if constexpr (sizeof(C) == 4) {
+            rows(ctx, g, c, r, k, cache, part_weights, capacity);
+            reduce_read<SumU64>(ctx, RowsDiffer{cache, expected, labels, part_weights, capacity, k}, g->n * k,
+                                &differing);
+            launch_prepare(ctx, g, c, r, labels, nullptr, k, cache);
+        }
+        return static_cast<std::int64_t>(differing);
     }
 
     // The rows of every vertex, or (part_weights) of the parts above capacity.
@@ -2857,6 +2876,22 @@ int gpart_refine_rows_reset(gpart_refine_rows* rows) {
     return guarded([&] {
         if (!rows) throw Error(GPART_ERR_INVALID_ARGUMENT, "null rows");
         rows->ready = false;
+    });
+}
+
+int gpart_refine_rows_check(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes,
+                            gpart_refine_rows* rows, uint32_t* cache, const int32_t* labels, int k,
+                            const uint64_t* part_weights, uint64_t capacity, const uint32_t* expected,
+                            int64_t* differing) {
+    return guarded([&] {
+        if (!rows) throw Error(GPART_ERR_INVALID_ARGUMENT, "null rows");
+        rows->check(g, classes, k);
+        GPART_ROWS_DISPATCH(g->width, {
+            OpsT::prepare_rows(ctx, g, classes, rows, labels, k, cache);
+            *differing = OpsT::check_rows(ctx, g, classes, rows, labels, k, cache,
+                                          reinterpret_cast<const unsigned long long*>(part_weights), capacity, expected);
+        });
+        rows->ready = true;
     });
 }
 

@@ -283,13 +283,14 @@ __global__ void __launch_bounds__(kRowsThreads) rows_kernel(RowLists lists, cons
     });
 }
 
-// Before a level's first round: the states from the labels, every hub row of the cache
-// to zero (as each round leaves them).
+// Before a level's first round: the states (where given) from the labels, every hub row
+// of the cache to zero (as each round leaves them).
 __global__ void __launch_bounds__(256) rows_prepare_kernel(RowLists lists, std::int64_t n, const std::int32_t* labels,
                                                            unsigned char* states, int k, unsigned* cache) {
     const std::int64_t threads = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
-    for (std::int64_t v = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; v < n; v += threads)
-        states[v] = static_cast<unsigned char>(labels[v]);
+    if (states)
+        for (std::int64_t v = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; v < n; v += threads)
+            states[v] = static_cast<unsigned char>(labels[v]);
     if (!lists.chunk_total) return;
     for (std::int64_t c = blockIdx.x; c < *lists.chunk_total; c += gridDim.x) {
         const std::int32_t i = lists.chunk_hub[c];
@@ -298,6 +299,20 @@ __global__ void __launch_bounds__(256) rows_prepare_kernel(RowLists lists, std::
             cache[static_cast<std::int64_t>(lists.high[i]) * k + threadIdx.x] = 0;
     }
 }
+
+// Whether entry i of the rows that rows_kernel sums differs from the expected one.
+struct RowsDiffer {
+    const unsigned* cache;
+    const unsigned* expected;
+    const std::int32_t* labels;
+    const unsigned long long* part_weights;  // null: every row
+    std::uint64_t capacity;
+    int k;
+    __device__ __forceinline__ unsigned long long operator()(std::int64_t i) const {
+        if (part_weights && part_weights[labels[i / k]] <= capacity) return 0;
+        return cache[i] != expected[i];
+    }
+};
 
 // The cut change of a mover's entries [begin, end) with stride G (the lanes' shares), as
 // update_cache_movers counts it: a neighbour that moves too counts once, at the lower

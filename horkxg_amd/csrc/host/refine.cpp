@@ -173,7 +173,7 @@ RefineStats run_refinement(Level<Types>& level, const RefineOptions& options, in
         level.host_part_weights.assign(status.part_weights, status.part_weights + k);
         if (options.strict_verify) {
             if (level.cut() != current_cut) throw std::runtime_error("incremental cut differs from CSR scan");
-            if (rows) return;  // no cache is kept
+            if (rows) return;  // no cache is kept: check_rows
             DeviceVector<std::uint8_t> check(cache.size());
             GPART_CHECK(gpart_refine_build_cache(ctx, &view, &classes, level.partition.data(), k, check.data(),
                                                  cache_bytes));
@@ -181,10 +181,23 @@ RefineStats run_refinement(Level<Types>& level, const RefineOptions& options, in
                 throw std::runtime_error("incremental affinity cache differs from CSR rebuild");
         }
     };
+    // Strict: before a round that sums its rows, those rows against a build from the labels;
+    // of the parts above capacity for a rebalance iteration, which reads no others.
+    auto check_rows = [&](const std::uint64_t* part_weights) {
+        if (!rows || !options.strict_verify) return;
+        DeviceVector<std::uint8_t> check(cache.size());
+        GPART_CHECK(gpart_refine_build_cache(ctx, &view, &classes, level.partition.data(), k, check.data(), cache_bytes));
+        std::int64_t differing = 0;
+        GPART_CHECK(gpart_refine_rows_check(ctx, &view, &classes, rows.get(), row_cache, level.partition.data(), k,
+                                            part_weights, level.capacity,
+                                            reinterpret_cast<const std::uint32_t*>(check.data()), &differing));
+        if (differing) throw std::runtime_error("affinity rows differ from CSR rebuild");
+    };
     auto rebalance = [&]() {
         for (int iteration = 0; iteration < 2 * k + 4 && level.maximum() > level.capacity; ++iteration) {
             ++stats.admission_iterations;
             gpart_refine_status status{};
+            check_rows(level.part_weights.data());
             if (rows)
                 GPART_CHECK(gpart_refine_rebalance_round_rows(ctx, &view, &classes, rows.get(), row_cache,
                                                               level.partition.data(), k, level.part_weights.data(),
@@ -203,6 +216,7 @@ RefineStats run_refinement(Level<Types>& level, const RefineOptions& options, in
     for (int phase = 0; phase < rounds && stale < options.stale_rounds; ++phase) {
         stats.rounds = phase + 1;
         gpart_refine_status status{};
+        check_rows(nullptr);
         if (rows)
             GPART_CHECK(gpart_refine_lp_round_rows(ctx, &view, &classes, rows.get(), row_cache,
                                                    level.partition.data(), k, filter, locks.data(), targets.data(),

@@ -497,6 +497,14 @@ int gpart_refine_rebalance_round_rows(gpart_ctx* ctx, const gpart_csr_view* g, c
                                       gpart_refine_rows* rows, uint32_t* cache, int32_t* labels, int k,
                                       uint64_t* part_weights, uint64_t capacity, int32_t* targets, int32_t* flags,
                                       gpart_refine_status* status);
+/* Strict verification (src/refine_incremental.cuh:280-301 compares the cache): sums the
+ * rows that the next LP round (part_weights NULL) or rebalance iteration will read, from
+ * what the last round left, into cache and counts the entries that differ from expected
+ * (device, gpart_refine_build_cache of the labels, 4-byte entries). host out: *differing. */
+int gpart_refine_rows_check(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* classes,
+                            gpart_refine_rows* rows, uint32_t* cache, const int32_t* labels, int k,
+                            const uint64_t* part_weights, uint64_t capacity, const uint32_t* expected,
+                            int64_t* differing);
 /* Round graphs (no reference counterpart: the reference launches every kernel of a
  * round from the host). gpart_refine_lp_round and gpart_refine_rebalance_round
  * record the launches of a round the first time they see its level, arrays and

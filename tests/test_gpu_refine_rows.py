@@ -74,6 +74,6 @@ def test_dense_refinement_matches_oracle(hx, oracle, name, k, width, weighted):
     assert rep["rounds"] == st.rounds and rep["admission_iterations"] == st.admission_iterations
     assert rep["final_cut"] == st.final_cut
     assert np.array_equal(labels, expect)
-    # the strict checks recount the cut after every round
+    # the strict checks recount the cut and compare the rows of every round
     strict, _ = g.refine(start, k, 1.03, 6, 3, verify=True)
     assert np.array_equal(strict, expect)

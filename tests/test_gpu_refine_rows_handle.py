@@ -42,6 +42,7 @@ class Level:
             "gpart_refine_rows_create": [vp, vp, vp, i32, i32, vp],
             "gpart_refine_rows_destroy": [vp],
             "gpart_refine_rows_reset": [vp],
+            "gpart_refine_rows_check": [vp, vp, vp, vp, vp, vp, i32, vp, u64, vp, vp],
             "gpart_refine_lp_round_rows": [vp, vp, vp, vp, vp, vp, i32, C.c_double, vp, vp, vp, vp, vp, vp],
             "gpart_refine_rebalance_round_rows": [vp, vp, vp, vp, vp, vp, i32, vp, u64, vp, vp, vp],
         }
@@ -98,6 +99,17 @@ class Level:
             return self.L.gpart_refine_rebalance_round_rows(*head, self.rows, self.cache.ptr, *tail), st
         return self.L.gpart_refine_rebalance_round(*head, self.cache.ptr, 4, *tail), st
 
+    def differing(self, capacity=None):
+        """Entries of the rows the next round sums that differ from a build from the labels."""
+        D, out = self.D, C.c_int64(-1)
+        expected = D.DeviceArray(dtype=np.uint32, count=self.g.n * self.k)
+        head = (D._ctx(), self.view(), self.classes())
+        D._check(self.L.gpart_refine_build_cache(*head, self.labels.ptr, self.k, expected.ptr, 4))
+        D._check(self.L.gpart_refine_rows_check(*head, self.rows, self.cache.ptr, self.labels.ptr, self.k,
+                                                None if capacity is None else self.weights.ptr, capacity or 0,
+                                                expected.ptr, C.byref(out)))
+        return out.value
+
 
 @pytest.fixture(scope="module", autouse=True)
 def need_gpu(hx):
@@ -144,3 +156,46 @@ def test_rounds_of_another_level_are_refused(hx):
     assert np.array_equal(level.labels.get(), before)
     rc, st = level.lp()  # a refused round leaves the handle as it was
     assert rc == 0 and st.movers > 0
+
+
+@pytest.mark.parametrize("name,k", [("hubs", 8), ("hubs", 31), ("random", 5)])
+def test_check_finds_rows_of_other_labels(hx, name, k):
+    """What the strict checks compare: nothing differs before and after rounds, and rows
+    summed from other labels than the ones given are found."""
+    print(f"case rows check graph={name} k={k}", flush=True)
+    csr = hub_graph(hx, 12_001, 24) if name == "hubs" else random_graph(hx, 20_001, 26)
+    n = len(csr[0]) - 1
+    level = Level(hx, csr, k, True)
+    level.set_labels(shuffled(n, k, 1))
+    for step in range(4):
+        assert level.differing() == 0 and level.differing(n // k) == 0, step
+        rc, st = level.lp() if step % 2 == 0 else level.rebalance(n // k)
+        assert rc == 0 and st.movers > 0
+    assert level.differing() == 0
+    other = level.labels.get()
+    v = int(csr[1][csr[0][n // 2]])  # of some row: its neighbours' rows change
+    other[v] = (other[v] + 1) % k
+    level.D._check(level.L.gpart_memcpy_htod(level.D._ctx(), C.c_void_p(level.labels.ptr), other.ctypes.data, 4 * n))
+    assert level.differing() == 2 * (csr[0][v + 1] - csr[0][v])  # each neighbour: an entry less, an entry more
+    level.L.gpart_refine_rows_reset(level.rows)
+    assert level.differing() == 0
+
+
+def test_strict_verification_checks_the_rows(hx):
+    """verify=True builds a cache and sums the rows once more for every round."""
+    print("case rows strict", flush=True)
+    indptr, indices = random_graph(hx, 20_001, 26)
+    g = hx.Graph(indptr, indices)
+    start = shuffled(20_001, 8, 1)
+    launches = []
+    for verify in (False, True):
+        hx.profile_reset()
+        hx.profile_enable("refine_cache", True)
+        try:
+            labels, rep = g.refine(start, 8, 1.03, 6, 3, verify=verify)
+            launches.append(hx.profile_read("refine_cache")["launches"])
+        finally:
+            hx.profile_enable("refine_cache", False)
+    rounds = rep["rounds"] + rep["admission_iterations"]
+    assert rep["admission_iterations"] > 0
+    assert launches == [rounds, 3 * rounds]
