@@ -677,7 +677,7 @@ __global__ void __launch_bounds__(kRowsThreads) gain_commit_kernel(
     std::int64_t n, const O* offsets, const std::int32_t* neighbors, const W* weights, const W* vertex_weights,
     std::int32_t* labels, const std::int32_t* targets, const std::int32_t* flags, std::int32_t* locks, int k,
     unsigned* cache, unsigned long long* part_weights, unsigned long long* status, unsigned long long* counter) {
-    extern __shared__ unsigned lds[];
+    extern __shared__ __align__(16) unsigned lds[];  // the states, stored 16 bytes at once
     __shared__ long long wave_gain[kRowsWaves];
     __shared__ PartMoves moves;
     __shared__ int last;

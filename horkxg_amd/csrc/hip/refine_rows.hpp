@@ -39,6 +39,7 @@ constexpr std::size_t kRowsPairLds = 74 * 1024;  // two where their LDS allows i
 constexpr int kRowsWaveWords = 8 * 32 + kWave;
 constexpr std::size_t kRowsWaveBytes = static_cast<std::size_t>(kRowsWaves) * kRowsWaveWords * 4;
 constexpr std::int64_t kStateBytes = 128 * 1024;
+static_assert(kRowsWaveBytes % 16 == 0, "the states behind the waves' words are aligned to 16 bytes");
 static_assert(kRowsWaveBytes + kStateBytes + 9 * 1024 <= 160 * 1024, "with the row list they fit a CU's 160 KB");
 // Dense: from this many entries per vertex. R-MAT levels have 29 and more (refinement of
 // R-MAT 18, k = 8: 36 -> 20 ms); the mesh levels' 17 and less stay with the cache, whose
@@ -231,7 +232,7 @@ __global__ void __launch_bounds__(kRowsThreads) rows_kernel(RowLists lists, cons
                                                             const std::int32_t* neighbors, const W* weights, int k,
                                                             unsigned* cache, const unsigned long long* part_weights,
                                                             std::uint64_t capacity) {
-    extern __shared__ unsigned lds[];
+    extern __shared__ __align__(16) unsigned lds[];  // stage_states stores 16 bytes at once
     __shared__ RowQueue queue;
     const int lane = lane_id(), wave_in = threadIdx.x / kWave;
     unsigned* sums = lds + wave_in * kRowsWaveWords;
