@@ -1471,6 +1471,7 @@ int gpart_degree_classes_build(gpart_ctx* ctx, const gpart_csr_view* g, gpart_de
     return guarded([&] {
         if (g->width == GPART_WIDTH_STANDARD) build_classes<std::int32_t, std::uint32_t>(ctx, g, classes);
         else build_classes<std::int64_t, std::uint64_t>(ctx, g, classes);
+        complete_outputs(ctx);
     });
 }
 

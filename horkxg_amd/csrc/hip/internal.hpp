@@ -49,6 +49,9 @@ struct gpart_ctx {
     // word and publish its value (so a captured launch needs no new argument per
     // call); the host counts the same publications in status_seq.
     std::uint64_t status_seq = 0;
+    // The caller reads device outputs through this context's stream only
+    // (gpart_ctx_set_stream_ordered).
+    bool stream_ordered = false;
     // Device words: that counter, and the workgroups of the reduction under way that
     // have finished (its last one leaves 0; one stream, so one reduction at a time).
     unsigned long long* status_counter = nullptr;
@@ -193,6 +196,10 @@ struct Publication {
 };
 Publication publication(gpart_ctx* ctx);
 void read_published(gpart_ctx* ctx, void* host, std::size_t bytes);
+// At the end of an entry point whose last kernel publishes host values and writes device
+// outputs as well: the kernel may still be writing them when the host has the values.
+// Waits for it unless the caller's reads are ordered behind it anyway.
+void complete_outputs(gpart_ctx* ctx);
 constexpr int kStatusWords = 512;  // 4 KiB of status memory per context
 
 template <typename T>

@@ -2837,6 +2837,7 @@ int gpart_refine_lp_round(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_d
                              OpsT::lp_round(ctx, g, classes, static_cast<CacheT*>(cache), labels, k, filter, locks,
                                             targets, reinterpret_cast<long long*>(gains), flags,
                                             reinterpret_cast<unsigned long long*>(part_weights), nullptr, status));
+        complete_outputs(ctx);
     });
 }
 
@@ -2909,6 +2910,7 @@ int gpart_refine_lp_round_rows(gpart_ctx* ctx, const gpart_csr_view* g, const gp
                            reinterpret_cast<unsigned long long*>(part_weights), rows, status);
         });
         rows->ready = true;
+        complete_outputs(ctx);
     });
 }
 
@@ -2926,6 +2928,7 @@ int gpart_refine_rebalance_round_rows(gpart_ctx* ctx, const gpart_csr_view* g, c
                                   rows, status);
         });
         rows->ready = true;
+        complete_outputs(ctx);
     });
 }
 
@@ -2965,6 +2968,7 @@ int gpart_refine_rebalance_round(gpart_ctx* ctx, const gpart_csr_view* g, const 
                              OpsT::rebalance_round(ctx, g, classes, static_cast<CacheT*>(cache), labels, k,
                                                    reinterpret_cast<unsigned long long*>(part_weights), capacity,
                                                    targets, flags, nullptr, status));
+        complete_outputs(ctx);
     });
 }
 

@@ -156,6 +156,10 @@ void read_published(gpart_ctx* ctx, void* host, std::size_t bytes) {
     std::memcpy(host, ctx->status_host + 1, bytes);
 }
 
+void complete_outputs(gpart_ctx* ctx) {
+    if (!ctx->stream_ordered) GPART_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+}
+
 // Small read-backs: a one-wave kernel copies the bytes into the fine-grained
 // status words and stores the sequence number after them; the host polls for it
 // (no copy engine, no blocking wait).
@@ -390,6 +394,14 @@ int gpart_ctx_synchronize(gpart_ctx* ctx) {
 }
 
 void* gpart_ctx_stream(gpart_ctx* ctx) { return ctx->stream; }
+
+int gpart_ctx_set_stream_ordered(gpart_ctx* ctx, int enabled, int* previous) {
+    return guarded([&] {
+        if (!ctx) throw Error(GPART_ERR_INVALID_ARGUMENT, "null context");
+        if (previous) *previous = ctx->stream_ordered ? 1 : 0;
+        ctx->stream_ordered = enabled != 0;
+    });
+}
 
 int gpart_device_alloc(gpart_ctx* ctx, size_t bytes, void** out) {
     return guarded([&] { *out = bytes ? ctx_alloc(ctx, bytes) : nullptr; });

@@ -46,6 +46,7 @@ struct SclpWorkspace<Types>::Impl {
             high.resize_discard(static_cast<std::size_t>(std::max<std::int64_t>(n, 1)));
             classes = gpart_degree_classes{low.data(), medium.data(), high.data(), 0, 0, 0, 0, 0, 0};
             const auto view = g.view();
+            const detail::StreamOrdered ordered(detail::context());
             GPART_CHECK(gpart_degree_classes_build(detail::context(), &view, &classes));
             classes_for = g.offsets.data();
             classes_n = n;

@@ -80,6 +80,7 @@ RefineStats run_refinement(Level<Types>& level, const RefineOptions& options, in
                            const std::uint64_t* known_cut = nullptr) {
     const auto start = clock_type::now();
     auto* ctx = detail::context();
+    const detail::StreamOrdered ordered(ctx);
     validate_gain_range(level.graph);
     const auto n = level.graph.vertices();
     const int k = options.parts;

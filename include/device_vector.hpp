@@ -25,6 +25,20 @@ gpart_ctx* context();
 void bind_context(gpart_ctx* ctx);
 // Synchronise and return all cached device blocks (ScratchPoolSession::finish).
 void release_context_cache();
+// For its scope, the host code here reads device outputs through the context's stream only.
+class StreamOrdered {
+public:
+    explicit StreamOrdered(gpart_ctx* ctx) : ctx_(ctx) {
+        GPART_CHECK(gpart_ctx_set_stream_ordered(ctx_, 1, &previous_));
+    }
+    ~StreamOrdered() { gpart_ctx_set_stream_ordered(ctx_, previous_, nullptr); }
+    StreamOrdered(const StreamOrdered&) = delete;
+    StreamOrdered& operator=(const StreamOrdered&) = delete;
+
+private:
+    gpart_ctx* ctx_;
+    int previous_ = 0;
+};
 }  // namespace detail
 
 template <typename T>

@@ -50,6 +50,12 @@ int gpart_ctx_create(int device, gpart_ctx** out);
 int gpart_ctx_destroy(gpart_ctx* ctx);
 int gpart_ctx_synchronize(gpart_ctx* ctx);
 void* gpart_ctx_stream(gpart_ctx* ctx);
+/* enabled: the caller reads what the context's kernels write through its stream only, so
+ * gpart_degree_classes_build and the refinement rounds return as soon as their host
+ * values are known, while the kernel that sends them may still be writing the arrays
+ * (a wait of its own per round costs as much as a small round's kernels). Default 0: they
+ * synchronise the stream. previous (may be NULL): the setting before. */
+int gpart_ctx_set_stream_ordered(gpart_ctx* ctx, int enabled, int* previous);
 /* Stream-ordered caching allocator; replaces ScratchAllocator/ScratchPoolSession
  * (include/detail/scratch_pool.hpp:15-106). Blocks are cut best-fit from device
  * segments the context keeps; a freed block serves later allocations on the same
