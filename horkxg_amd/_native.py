@@ -140,6 +140,8 @@ def hip_lib():
         H.gpart_refine_set_graphs.argtypes = [C.c_void_p, C.c_int]
         H.gpart_refine_set_balance_blocks.argtypes = [C.c_void_p, C.c_int64]
         H.gpart_contract_set_stash.argtypes = [C.c_void_p, C.c_int64]
+        H.gpart_refine_set_few_leaving.argtypes = [C.c_void_p, C.c_int64]
+        H.gpart_refine_selection_stats.argtypes = [C.c_void_p] + 3 * [C.POINTER(C.c_int64)]
         H.gpart_refine_graph_stats.argtypes = [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_int64),
                                                C.POINTER(C.c_int64)]
         H.gpart_spectral_queue_set_tuning.argtypes = [C.c_int32, C.c_int32]
@@ -335,6 +337,19 @@ def set_refine_graphs(enabled: bool = True) -> None:
 def set_refine_balance_blocks(blocks: int) -> None:
     """The calling thread's cap on the rebalance proposals grid (result-neutral)."""
     _check(hip_lib().gpart_refine_set_balance_blocks(_ctx(), int(blocks)))
+
+
+def set_refine_few_leaving(vertices: int = 16384) -> None:
+    """Leaving vertices up to which the calling thread's large rebalance iterations select
+    the destinations in one workgroup; -1: in no iteration (result-neutral)."""
+    _check(hip_lib().gpart_refine_set_few_leaving(_ctx(), int(vertices)))
+
+
+def refine_selection_stats() -> dict:
+    """The calling thread's large rebalance iterations so far: by form, and run again."""
+    out = [C.c_int64() for _ in range(3)]
+    _check(hip_lib().gpart_refine_selection_stats(_ctx(), *(C.byref(x) for x in out)))
+    return dict(zip(("single", "slices", "refused"), (x.value for x in out)))
 
 
 def set_contract_stash(min_vertices: int) -> None:

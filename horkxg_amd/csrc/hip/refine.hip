@@ -48,6 +48,7 @@ struct RoundState {
     long long edges;       // CSR entries of all movers (light + heavy)
     unsigned long long cut_directed;  // rebuild rounds: directed cut weight after the round
     unsigned long long arrivals;  // workgroups of the round's last launch that have finished
+    unsigned long long refused;   // rebalance: more vertices leave than one workgroup selects among
     unsigned long long pw[32];
 };
 
@@ -1470,10 +1471,13 @@ __global__ void __launch_bounds__(kSelectThreads) balance_select_kernel(
 // hundreds to thousands where the candidates are 10^4 to 10^6), so the destinations'
 // histogram, scan, ranks and mover lists take one workgroup 12 us; as launches over
 // the candidates they were four (six above 256 workgroups) of 4.4-6.2 us each. Where
-// the part weights of the last round say that more than kFewLeaving vertices leave, the
+// the part weights of the last round say that more than ctx->few_leaving vertices leave, the
 // destinations too are selected by passes over the slices (R-MAT levels move up to a
 // tenth of their vertices at once: 4.2 M vertices, 1.5 against 4.3 ms an iteration).
-constexpr std::int64_t kFewLeaving = 16384;
+// That guess counts vertices of average weight, and the last round may have been another
+// level's. So the workgroup that finds more than kRefusedShare times as many refuses: the
+// iteration moves nothing and runs again with the passes.
+constexpr std::int64_t kRefusedShare = 4;
 
 // balance_scan_buckets (:188-202): the boundary bucket of every overloaded part
 // (sources) or of every part (destinations) and the weight before it, from the
@@ -1726,8 +1730,8 @@ template <typename O, typename W>
 __global__ void __launch_bounds__(kSelectThreads) balance_destinations_kernel(
     RoundState* st, int slices, const std::int32_t* left_vertex, const std::int32_t* left_code,
     const std::int32_t* left_count, const std::int32_t* labels, const W* vertex_weights, const O* offsets, int k,
-    const unsigned long long* part_weights, std::uint64_t capacity, std::int32_t* light, std::int32_t* heavy,
-    std::int32_t* flags, unsigned char* state) {
+    const unsigned long long* part_weights, std::uint64_t capacity, std::int64_t most, std::int32_t* light,
+    std::int32_t* heavy, std::int32_t* flags, unsigned char* state) {
     __shared__ DestinationShared sh;
     const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
     const long long candidates = st->candidates, per = (candidates + slices - 1) / slices;
@@ -1744,6 +1748,10 @@ __global__ void __launch_bounds__(kSelectThreads) balance_destinations_kernel(
     for (int w = 0; w < kSelectWaves; ++w) {
         if (w == wave) below = count;
         count += sh.waves[w];
+    }
+    if (count > most) {  // uniform
+        if (t == 0) st->refused = 1;
+        return;
     }
     if (t < kSliceBlocks) sh.first[t] = below + inclusive - mine;
     unsigned long long total = 0;
@@ -2344,7 +2352,8 @@ struct Ops {
 
     // The host's wait for the status that apply's last launch publishes, and its
     // reading.
-    static void finish(gpart_ctx* ctx, RoundRun& run, const gpart_csr_view* g, int k, bool rows_form,
+    // False: a rebalance iteration refused (kRefusedShare) and left everything as it was.
+    static bool finish(gpart_ctx* ctx, RoundRun& run, const gpart_csr_view* g, int k, bool rows_form,
                        gpart_refine_status* out) {
         run.end();
         const std::uint64_t seq = ++ctx->status_seq;
@@ -2379,6 +2388,7 @@ struct Ops {
             out->cut_after = h.cut_directed / 2;
             out->cut_delta = 0;
         }
+        return h.refused == 0;
     }
 
     // One LP round: proposals, priority filter, movers, apply; one synchronisation.
@@ -2543,9 +2553,16 @@ struct Ops {
         if (g->n <= kSelectVertices)
             rebalance_round_small(ctx, g, c, cache, labels, k, part_weights, capacity, targets, flags, powers, r,
                                   out);
-        else
-            rebalance_round_large(ctx, g, c, cache, labels, k, part_weights, capacity, targets, flags, powers, r,
-                                  out);
+        else {
+            const bool few = expected_leaving(ctx, g->n, k, capacity) <= ctx->few_leaving;
+            ++(few ? ctx->single_selections : ctx->slice_selections);
+            if (!rebalance_round_large(ctx, g, c, cache, labels, k, part_weights, capacity, targets, flags, powers,
+                                       r, few, out)) {
+                ++ctx->refused_selections;
+                rebalance_round_large(ctx, g, c, cache, labels, k, part_weights, capacity, targets, flags, powers, r,
+                                      false, out);
+            }
+        }
         // per candidate: id, label, weight, cache row, target and bucket writes
         profile_add_bytes(ctx, GPART_PROFILE_REBALANCE,
                           static_cast<double>(out->candidates) * (16.0 + sizeof(W) + sizeof(C) * k));
@@ -2553,10 +2570,11 @@ struct Ops {
         profile_add_units(ctx, GPART_PROFILE_REBALANCE, static_cast<double>(out->candidates));
     }
 
-    static void rebalance_round_large(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
+    // few: one workgroup selects the destinations, or refuses (returns false).
+    static bool rebalance_round_large(gpart_ctx* ctx, const gpart_csr_view* g, const gpart_degree_classes* c,
                                       C* cache, std::int32_t* labels, int k, unsigned long long* part_weights,
                                       std::uint64_t capacity, std::int32_t* targets, std::int32_t* flags,
-                                      const PowerTable& powers, const gpart_refine_rows* r,
+                                      const PowerTable& powers, const gpart_refine_rows* r, bool few,
                                       gpart_refine_status* out) {
         const std::int64_t n = g->n;
         const auto* off = static_cast<const O*>(g->offsets);
@@ -2576,9 +2594,10 @@ struct Ops {
         }
         if (!ctx->rebalance_counters_zero) fill_bytes(ctx, ctx->rebalance_counters, 0, ctx->rebalance_counter_bytes);
         ctx->rebalance_counters_zero = false;  // until this round completes
-        const bool few = expected_leaving(ctx, n, k, capacity) <= kFewLeaving;
+        const std::int64_t most = kRefusedShare * ctx->few_leaving;
         RoundRun run(ctx, round_plan(ctx, n, round_key(ctx, g, c, cache, labels, k, targets, flags, part_weights, r,
-                                                       {1, capacity, few, key_of(ctx->rebalance_counters)})));
+                                                       {1, capacity, few, static_cast<std::uint64_t>(most),
+                                                        key_of(ctx->rebalance_counters)})));
         Scratch<RoundState> st(ctx, 1);
         auto* st_ptr = st.get();
         auto* replicas = static_cast<unsigned long long*>(ctx->rebalance_counters);
@@ -2641,7 +2660,7 @@ struct Ops {
                 ranks(balance_source_ranks_kernel<W, false>);
                 hipLaunchKernelGGL((balance_destinations_kernel<O, W>), dim3(1), dim3(kSelectThreads), 0, ctx->stream,
                                    st_ptr, slices, left_vertex.get(), left_code.get(), left_count.get(), labels, vw, off,
-                                   k, part_weights, capacity, light.get(), heavy.get(), flags, state);
+                                   k, part_weights, capacity, most, light.get(), heavy.get(), flags, state);
             } else {
                 ranks(balance_source_ranks_kernel<W, true>);
                 hipLaunchKernelGGL(bucket_boundaries_kernel<true>, dim3(k), dim3(kBucketScanThreads), 0, ctx->stream,
@@ -2663,8 +2682,9 @@ struct Ops {
         else
             apply(ctx, run, g, c, st_ptr, light.get(), heavy.get(), labels, targets, flags, k, cache, part_weights,
                   nullptr);
-        finish(ctx, run, g, k, r != nullptr, out);
+        const bool done = finish(ctx, run, g, k, r != nullptr, out);
         ctx->rebalance_counters_zero = true;
+        return done;
     }
 };
 
@@ -2936,6 +2956,23 @@ int gpart_refine_set_balance_blocks(gpart_ctx* ctx, int64_t blocks) {
     return guarded([&] {
         if (blocks < 1 || blocks > (int64_t{1} << 20)) throw Error(GPART_ERR_INVALID_ARGUMENT, "block count out of range");
         ctx->balance_blocks = blocks;
+    });
+}
+
+int gpart_refine_set_few_leaving(gpart_ctx* ctx, int64_t vertices) {
+    return guarded([&] {
+        if (!ctx || vertices < -1 || vertices > (int64_t{1} << 28))
+            throw Error(GPART_ERR_INVALID_ARGUMENT, "leaving vertices out of range");
+        ctx->few_leaving = vertices;
+    });
+}
+
+int gpart_refine_selection_stats(gpart_ctx* ctx, int64_t* single, int64_t* slices, int64_t* refused) {
+    return guarded([&] {
+        if (!ctx) throw Error(GPART_ERR_INVALID_ARGUMENT, "null context");
+        if (single) *single = ctx->single_selections;
+        if (slices) *slices = ctx->slice_selections;
+        if (refused) *refused = ctx->refused_selections;
     });
 }
 

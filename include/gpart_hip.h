@@ -525,6 +525,13 @@ int gpart_refine_set_graphs(gpart_ctx* ctx, int enabled);
 /* Workgroups of the rebalance proposals launch at most (default from the tuning
  * header); results do not depend on it. */
 int gpart_refine_set_balance_blocks(gpart_ctx* ctx, int64_t blocks);
+/* Levels above 16,384 vertices: rebalance iterations that are expected to move at most
+ * this many vertices (default 16,384; -1: none) select the destinations in one workgroup,
+ * others in passes over all candidates; one that turns out to move more than four times as
+ * many runs again with the passes. Results do not depend on it. The stats count the
+ * iterations started in either form, and those that ran again, since the context was made. */
+int gpart_refine_set_few_leaving(gpart_ctx* ctx, int64_t vertices);
+int gpart_refine_selection_stats(gpart_ctx* ctx, int64_t* single, int64_t* slices, int64_t* refused);
 int gpart_refine_graphs_enabled(gpart_ctx* ctx);
 int gpart_refine_graph_stats(gpart_ctx* ctx, int64_t* plans, int64_t* captures, int64_t* replays);
 /* Outcome of gpart_refine_level. */
