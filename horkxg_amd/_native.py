@@ -339,7 +339,7 @@ def set_refine_balance_blocks(blocks: int) -> None:
     _check(hip_lib().gpart_refine_set_balance_blocks(_ctx(), int(blocks)))
 
 
-def set_refine_few_leaving(vertices: int = 16384) -> None:
+def set_refine_few_leaving(vertices: int = 4096) -> None:
     """Leaving vertices up to which the calling thread's large rebalance iterations select
     the destinations in one workgroup; -1: in no iteration (result-neutral)."""
     _check(hip_lib().gpart_refine_set_few_leaving(_ctx(), int(vertices)))

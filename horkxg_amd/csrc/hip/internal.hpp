@@ -83,7 +83,7 @@ struct gpart_ctx {
     std::int64_t balance_blocks = gpart_tuned::kBalanceBlocks;
     // Vertices that may leave in a large level's rebalance iteration for one workgroup to
     // select their destinations (gpart_refine_set_few_leaving); the iterations by form.
-    std::int64_t few_leaving = 16384;
+    std::int64_t few_leaving = 4096;
     std::int64_t single_selections = 0, slice_selections = 0, refused_selections = 0;
     // contraction: levels of at least this many fine vertices stash every entry's
     // coarse neighbour in the count pass (gpart_contract_set_stash)

@@ -1473,11 +1473,15 @@ __global__ void __launch_bounds__(kSelectThreads) balance_select_kernel(
 // the candidates they were four (six above 256 workgroups) of 4.4-6.2 us each. Where
 // the part weights of the last round say that more than ctx->few_leaving vertices leave, the
 // destinations too are selected by passes over the slices (R-MAT levels move up to a
-// tenth of their vertices at once: 4.2 M vertices, 1.5 against 4.3 ms an iteration).
+// tenth of their vertices at once). An iteration by one workgroup and by passes, in us,
+// on grids of 250,000 vertices, k = 8: 60 and 68 for 172 leaving vertices, 68 and 72 for
+// 2,226, 79 and 77 for 3,951, 92 and 82 for 6,618, 124 and 89 for 13,943; of 4 M: 108 and
+// 120 for 386, 128 and 127 for 5,336, 273 and 155 for 26,998. The line is 4,096.
 // That guess counts vertices of average weight, and the last round may have been another
 // level's. So the workgroup that finds more than kRefusedShare times as many refuses: the
-// iteration moves nothing and runs again with the passes.
-constexpr std::int64_t kRefusedShare = 4;
+// iteration moves nothing and runs again with the passes. Its launches up to there are
+// spent, 60 to 110 us of the above, which is what one workgroup takes longer for 30,000.
+constexpr std::int64_t kRefusedShare = 8;
 
 // balance_scan_buckets (:188-202): the boundary bucket of every overloaded part
 // (sources) or of every part (destinations) and the weight before it, from the

@@ -526,8 +526,8 @@ int gpart_refine_set_graphs(gpart_ctx* ctx, int enabled);
  * header); results do not depend on it. */
 int gpart_refine_set_balance_blocks(gpart_ctx* ctx, int64_t blocks);
 /* Levels above 16,384 vertices: rebalance iterations that are expected to move at most
- * this many vertices (default 16,384; -1: none) select the destinations in one workgroup,
- * others in passes over all candidates; one that turns out to move more than four times as
+ * this many vertices (default 4,096; -1: none) select the destinations in one workgroup,
+ * others in passes over all candidates; one that turns out to move more than eight times as
  * many runs again with the passes. Results do not depend on it. The stats count the
  * iterations started in either form, and those that ran again, since the context was made. */
 int gpart_refine_set_few_leaving(gpart_ctx* ctx, int64_t vertices);

@@ -115,7 +115,7 @@ def test_more_leave_than_expected(hx, oracle, few_leaving, dense, width):
     vw = np.ones(n, np.uint64)
     start = shuffled(n, k)
     heavy = np.arange(5 * k) * 7
-    vw[heavy], start[heavy] = 100_000, np.arange(5 * k) % k
-    few_leaving(20)
-    counts = compare(hx, oracle, indptr, indices, vw, k, width, 1.001, start)
+    vw[heavy], start[heavy] = 1_000_000, np.arange(5 * k) % k
+    few_leaving(4)
+    counts = compare(hx, oracle, indptr, indices, vw, k, width, 1.0001, start)
     assert counts["refused"] > 0
