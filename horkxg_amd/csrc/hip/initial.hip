@@ -303,17 +303,25 @@ __global__ void __launch_bounds__(kBatchThreads) depth_finish_kernel(DepthTasks 
 // below the root: 3.29 -> 2.33 ms.
 constexpr int kSoloThreads = 1024;
 constexpr int kSoloGroups = kMaxBatchedTask / kWave;  // groups of 64 rows, one width each
-// Entries of a task, estimated by its share of the graph's vertices, up to which the
-// solo form is taken. Weighted 3D meshes, FP64, a depth of tasks of 3,700 vertices and
-// 21,000 entries: 500 us, the launch form 500; of 1,860 and 10,500: 300 and 500; of 930
-// and 5,300: 190 and 490; of 460 and 2,600: 145 and 490.
+// Where every task of a depth is small and sparse enough the form is tried: up to this
+// many entries by the task's share of the graph's vertices. Weighted 3D meshes, FP64, a
+// depth of tasks of 3,700 vertices and 21,000 entries: 500 us, the launch form 500; of
+// 1,860 and 10,500: 300 and 500; of 930 and 5,300: 190 and 490; of 460 and 2,600: 145 and
+// 490.
 constexpr double kSoloEntries = 16384;
-
-constexpr int kSoloWidth = 256;  // longest row of a group with slots
+// The share says nothing of how a skewed graph's entries lie, so the depth is measured
+// first and left to the launch form where a task has more slots, or a longer row, than
+// these: slots are padded to the longest row of each 64, and a wave has its groups to
+// itself while the launch form spreads rows over all CUs. Bisections of one task, the
+// launch form and the solo one in us: mesh, 216 rows of slots, 463 and 367; 344, 543 and
+// 490; 424, 557 and 563; random, 16 entries a vertex, 488, 392 and 352; 664, 459 and 502;
+// 936, 465 and 599; R-MAT 8, 248 and a row of 94, 384 and 371; 384 and a row of 119, 403
+// and 449; R-MAT 9, 584 and 141, 434 and 506.
+constexpr int kSoloRows = 416;  // slots of a task, in rows of 64
+constexpr int kSoloWidth = 96;  // longest row, padded
 
 struct SoloTasks {
     int count;
-    long long first_slot[kMaxDepthTasks + 1];  // of each task's slots, in rows of 64
     gpart_bisect_task task[kMaxDepthTasks];
 };
 
@@ -375,17 +383,63 @@ struct SoloShared {
     T y[kMaxBatchedTask];   // a step's result
     Moments partials[kMaxBatchedTask / 8];
     int width[kSoloGroups];  // of a group of 64 rows: its longest
-    long long slots[kSoloGroups];  // its first slot, in rows of 64; -1: it has none
-    int slot_bytes[kSoloGroups];   // 0: its entries are read from the CSR
+    int slots[kSoloGroups];  // its first slot, in rows of 64
+    int slot_bytes[kSoloGroups];
 };
+
+// Whether a task is one for the solo form, by its rows: refused[task] is 1 where one is
+// longer than kSoloWidth, where the padded groups together need more than kSoloRows, or
+// where a weight does not fit a slot. Also clears the depth's counters (two words).
+template <typename O, typename W>
+__global__ void __launch_bounds__(kSoloThreads) depth_measure_kernel(SoloTasks st, const int* order, const O* offsets,
+                                                                     const W* weights, int* refused,
+                                                                     unsigned long long* counters) {
+    __shared__ int wave_rows[kSoloThreads / kWave];
+    const gpart_bisect_task task = st.task[blockIdx.x];
+    const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
+    if (blockIdx.x == 0 && t < 2) counters[t] = 0;
+    int rows = 0;
+    bool unfit = false;
+    for (int first = wave * kWave; first < task.count; first += kSoloThreads) {
+        int width = 0;
+        if (first + lane < task.count) {
+            const int v = order[task.begin + first + lane];
+            const auto begin = static_cast<std::int64_t>(offsets[v]), end = static_cast<std::int64_t>(offsets[v + 1]);
+            width = static_cast<int>(end - begin < kSoloWidth + 1 ? end - begin : kSoloWidth + 1);
+            if constexpr (sizeof(W) == 8) {
+                std::uint64_t bits = 0;
+                for (int e = 0; e < width; ++e) bits |= weights[begin + e];
+                unfit = unfit || bits >> (64 - kSlotShift) != 0;
+            }
+        }
+#pragma unroll
+        for (int m = kWave / 2; m > 0; m /= 2) width = max(width, __shfl_xor(width, m, kWave));
+        width = padded_width(width);
+        unfit = unfit || width > kSoloWidth;
+        rows += width;
+    }
+    if (lane == 0) wave_rows[wave] = rows;
+    unfit = __syncthreads_or(unfit);
+    if (t == 0) {
+        int total = 0;
+        for (int w = 0; w < kSoloThreads / kWave; ++w) total += wave_rows[w];
+        refused[blockIdx.x] = unfit || total > kSoloRows;
+    }
+}
+
+constexpr int kSoloRefused = -1;  // status of a depth with a refused task: nothing was done
 
 template <typename O, typename W, typename T>
 __global__ void __launch_bounds__(kSoloThreads) depth_solo_kernel(
-    SoloTasks st, int* labels, int* order, const O* offsets, const int* neighbors, const W* weights,
-    const std::uint64_t* vertex_weights, unsigned seed, std::uint64_t capacity, double* coords, int* position,
-    std::uint64_t* slot, gpart_bisect_task* next, int* next_count, int* status,
+    SoloTasks st, const int* refused, int* labels, int* order, const O* offsets, const int* neighbors,
+    const W* weights, const std::uint64_t* vertex_weights, unsigned seed, std::uint64_t capacity, double* coords,
+    int* position, std::uint64_t* slot, gpart_bisect_task* next, int* next_count, int* status,
     unsigned long long* entries) {
     __shared__ SoloShared<T> sh;
+    if (__syncthreads_or(static_cast<int>(threadIdx.x) < st.count && refused[threadIdx.x])) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *status = kSoloRefused;
+        return;
+    }
     const gpart_bisect_task task = st.task[blockIdx.x];
     const int count = task.count, group = task.first_part, blocks = (count + 7) / 8;
     const int rounds = (count + kSoloThreads - 1) / kSoloThreads;
@@ -411,11 +465,8 @@ __global__ void __launch_bounds__(kSoloThreads) depth_solo_kernel(
     if (entries && lane == 0 && scanned) atomicAdd(entries, scanned);
     __syncthreads();  // widths and positions
     if (wave == 0) {
-        const int padded = padded_width(sh.width[lane]);
-        const int width = padded <= kSoloWidth ? padded : 0;  // a long row's group does without
-        const long long inclusive = wave_scan(static_cast<long long>(width));
-        const long long first = st.first_slot[blockIdx.x] + inclusive - width;
-        sh.slots[lane] = width > 0 && first + width <= st.first_slot[blockIdx.x + 1] ? first : -1;
+        const int width = padded_width(sh.width[lane]);
+        sh.slots[lane] = static_cast<int>(blockIdx.x) * kSoloRows + wave_scan(width) - width;
     }
     __syncthreads();
     static_assert(kSoloGroups == kWave, "one wave places the groups");
@@ -476,29 +527,8 @@ __global__ void __launch_bounds__(kSoloThreads) depth_solo_kernel(
             });
         };
         const int bytes = __builtin_amdgcn_readfirstlane(sh.slot_bytes[g]);
-        const std::uint64_t* at = slot + sh.slots[g] * kWave;
-        if (bytes == 4) return stored(reinterpret_cast<const std::uint32_t*>(at) + lane);
-        if (bytes == 8) return stored(at + lane);
-        // without slots a half-wave takes a row, as in the launch form
-        A result = A(0);
-#pragma unroll 1
-        for (int first = 0; first < (width > 0 ? kWave : 0); first += 2) {
-            const int row = g * kWave + first + lane / kHalf;
-            A acc = A(0);
-            if (row < count) {
-                const int v = ids[row];
-                const auto end = static_cast<std::int64_t>(offsets[v + 1]);
-                for (std::int64_t e = static_cast<std::int64_t>(offsets[v]) + lane % kHalf; e < end; e += kHalf) {
-                    const int u = neighbors[e];
-                    if (labels[u] == group) acc = term(weights[e], position[u], acc);
-                }
-            }
-            acc = tree32(acc);
-            const A even = __shfl(acc, 0, kWave), odd = __shfl(acc, kHalf, kWave);
-            if (lane == first) result = even;
-            if (lane == first + 1) result = odd;
-        }
-        return result;
+        const std::uint64_t* at = slot + static_cast<std::int64_t>(sh.slots[g]) * kWave;
+        return bytes == 4 ? stored(reinterpret_cast<const std::uint32_t*>(at) + lane) : stored(at + lane);
     };
     // a row's moments into its block of eight rows
     auto absorb = [&](int r, double mass, double a) {
@@ -518,17 +548,11 @@ __global__ void __launch_bounds__(kSoloThreads) depth_solo_kernel(
 #pragma unroll 1
     for (int r = t; r < rounds * kSoloThreads; r += kSoloThreads) {
         const int g = r / kWave;
-        std::uint64_t* slots = sh.slots[g] >= 0 ? slot + sh.slots[g] * kWave : nullptr;
-        int bytes = 0;
-        if (slots) {
-            const std::uint64_t bits = fill(r, reinterpret_cast<std::uint32_t*>(slots));
-            bytes = 4;
-            if (__any(bits >> (32 - kSlotShift) != 0)) {
-                fill(r, slots);
-                bytes = __any(bits >> (64 - kSlotShift) != 0) ? 0 : 8;
-            }
-        }
-        if (lane == 0) sh.slot_bytes[g] = bytes;
+        std::uint64_t* slots = slot + static_cast<std::int64_t>(sh.slots[g]) * kWave;
+        const std::uint64_t bits = fill(r, reinterpret_cast<std::uint32_t*>(slots));
+        const bool wide = __any(bits >> (32 - kSlotShift) != 0);
+        if (wide) fill(r, slots);
+        if (lane == 0) sh.slot_bytes[g] = wide ? 8 : 4;
         const double d = over_row(r, 0.0, [](auto w, int, double acc) { return acc + static_cast<double>(w); });
         T x = 0;
         if (r < count) {
@@ -719,12 +743,10 @@ int gpart_spectral_depth(gpart_ctx* ctx, const gpart_csr_view* g, int32_t* label
         Scratch<Moments> pa(ctx, blocks), pb(ctx, blocks);
         // next_count and status (two ints), then the scanned CSR entries
         Scratch<unsigned long long> counters(ctx, 2);
-        fill_bytes(ctx, counters.get(), 0, 16);
         int* next_and_status = reinterpret_cast<int*>(counters.get());
         unsigned long long* entries = ctx->profile[GPART_PROFILE_SPECTRAL].enabled ? counters.get() + 1 : nullptr;
         int vertices = 0;
         for (int t = 0; t < task_count; ++t) vertices += tasks[t].count;
-        profile_begin(ctx, GPART_PROFILE_SPECTRAL);
         auto launch = [&](auto o_tag, auto w_tag, auto t_tag) {
             using O = decltype(o_tag);
             using W = decltype(w_tag);
@@ -756,38 +778,41 @@ int gpart_spectral_depth(gpart_ctx* ctx, const gpart_csr_view* g, int32_t* label
             const double share = static_cast<double>(g->m) * tasks[t].count / static_cast<double>(n);
             alone = alone && share <= kSoloEntries;
             solo.task[t] = tasks[t];
-            // twice the estimate in whole rows of 64, and as much again for uneven widths
-            solo.first_slot[t + 1] =
-                solo.first_slot[t] + static_cast<long long>(4.0 * share / kWave) + kSoloGroups * 8;
         }
-        const std::int64_t slots = alone ? solo.first_slot[task_count] * kWave : 0;
-        Scratch<int> position(ctx, alone ? n : 0);
-        Scratch<std::uint64_t> slot(ctx, slots);
+        Scratch<int> position(ctx, alone ? n : 0), refused(ctx, alone ? task_count : 0);
+        Scratch<std::uint64_t> slot(ctx, alone ? std::int64_t{task_count} * kSoloRows * kWave : 0);
         auto launch_solo = [&](auto o_tag, auto w_tag, auto t_tag) {
             using O = decltype(o_tag);
             using W = decltype(w_tag);
             using T = decltype(t_tag);
+            const auto* off = static_cast<const O*>(g->offsets);
+            const auto* w = static_cast<const W*>(g->edge_weights);
+            hipLaunchKernelGGL((depth_measure_kernel<O, W>), dim3(task_count), dim3(kSoloThreads), 0, ctx->stream, solo,
+                               order, off, w, refused.get(), counters.get());
             hipLaunchKernelGGL((depth_solo_kernel<O, W, T>), dim3(task_count), dim3(kSoloThreads), 0, ctx->stream, solo,
-                               labels, order, static_cast<const O*>(g->offsets), g->neighbors,
-                               static_cast<const W*>(g->edge_weights), vertex_weights, seed, capacity, coords,
-                               position.get(), slot.get(), next,
-                               next_and_status, next_and_status + 1, entries);
+                               refused.get(), labels, order, off, g->neighbors, w, vertex_weights, seed, capacity,
+                               coords, position.get(), slot.get(), next, next_and_status, next_and_status + 1, entries);
             GPART_LAUNCH_CHECK();
         };
         const bool fp32 = precision == GPART_SPECTRAL_FP32;
-        auto run = [&](auto o_tag, auto w_tag) {
-            if (alone && fp32) launch_solo(o_tag, w_tag, float{});
-            else if (alone) launch_solo(o_tag, w_tag, double{});
-            else if (fp32) launch(o_tag, w_tag, float{});
-            else launch(o_tag, w_tag, double{});
-        };
-        if (g->width == GPART_WIDTH_STANDARD) run(std::int32_t{}, std::uint32_t{});
-        else run(std::int64_t{}, std::uint64_t{});
-        profile_end(ctx, GPART_PROFILE_SPECTRAL, 0.0);
         unsigned long long h[2];
-        read_back(ctx, h, counters.get(), sizeof(h));
         int ns[2];
-        std::memcpy(ns, h, sizeof(ns));
+        auto run = [&](auto&& form) {
+            profile_begin(ctx, GPART_PROFILE_SPECTRAL);
+            const bool standard = g->width == GPART_WIDTH_STANDARD;
+            if (standard && fp32) form(std::int32_t{}, std::uint32_t{}, float{});
+            else if (standard) form(std::int32_t{}, std::uint32_t{}, double{});
+            else if (fp32) form(std::int64_t{}, std::uint64_t{}, float{});
+            else form(std::int64_t{}, std::uint64_t{}, double{});
+            profile_end(ctx, GPART_PROFILE_SPECTRAL, 0.0);
+            read_back(ctx, h, counters.get(), sizeof(h));
+            std::memcpy(ns, h, sizeof(ns));
+        };
+        if (alone) run(launch_solo);
+        if (!alone || ns[1] == kSoloRefused) {
+            fill_bytes(ctx, counters.get(), 0, 16);
+            run(launch);
+        }
         *next_count = ns[0];
         *status = ns[1];
         const std::size_t o_size = g->width == GPART_WIDTH_STANDARD ? 4 : 8;

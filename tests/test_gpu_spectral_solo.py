@@ -1,6 +1,8 @@
 """A depth of small sparse bisection tasks in one launch (hip/initial.hip, depth_solo_kernel).
 
-A workgroup does a task's start, 64 steps and split. FP64 labels and coordinates must be
+A workgroup does a task's start, 64 steps and split, where every task of the depth has at
+most 416 rows of 64 slots, rows of at most 96 and weights below 2^52; else the depth takes
+its 66 launches. FP64 labels and coordinates must be
 bit-identical to the oracle's recursive bisection (src/initial_partition_gpu.cu:170-276),
 FP32 ones to the task queue's, which sums the same terms in the same order.
 """
@@ -56,13 +58,15 @@ CASES = {
     "deg22": (lattice, (700, 11), "standard"),
     "deg30": (lattice, (540, 15), "big"),
     "deg34": (lattice, (470, 17), "standard"),
-    # one long row per wave: some groups find no room for slots
+    "deg34_solo": (lattice, (200, 17), "standard"),
+    # one long row per wave: more slots than the form takes
     "hubs": (lambda: lattice(4096, 1, hubs=range(5, 4096, 64), hub_degree=60), (), "standard"),
-    # a row too long for slots, between groups that have them
+    # a row too long for the form
     "hub": (lambda: lattice(3000, 1, hubs=(700, 2100), hub_degree=900), (), "big"),
-    # weights beyond a 4-byte slot, at its edge, and beyond an 8-byte one
+    # weights beyond a 4-byte slot, at its edge, at an 8-byte one's and beyond it
     "wide": (lambda: lattice(300, 3, weight=lambda a, b: 2**20 - 1 + (a + b) % 2), (), "standard"),
     "wide_big": (lambda: lattice(300, 3, weight=lambda a, b: 2**40 + a), (), "big"),
+    "wide_edge": (lambda: lattice(300, 2, weight=lambda a, b: 2**52 - 1 - (a + b) % 2), (), "big"),
     "widest": (lambda: lattice(300, 2, weight=lambda a, b: 2**52 + a * 2**20), (), "big"),
 }
 
@@ -92,3 +96,46 @@ def test_solo_depths(hx, oracle, no_queue, name):
         ql, qc = g.initial_partition(k, 1.2, 3, "batched_fp32", with_coords=True)
         assert np.array_equal(labels, ql), k
         assert np.array_equal(coords.view(np.uint64), qc.view(np.uint64)), k
+
+
+# a row of 27 to 32 entries in each of 13 groups: 416 rows of slots, and 4 more for one more
+# vertex; rows of 96 and of 98; weights of 52 and 53 bits
+HUBS = dict(hubs=range(5, 832, 64), hub_degree=26)
+
+
+@pytest.mark.parametrize("name,make,width,solo", [
+    ("rows", lambda: lattice(832, 1, **HUBS), "standard", True),
+    ("more rows", lambda: lattice(833, 1, **HUBS), "standard", False),
+    ("width", lambda: lattice(160, 48), "big", True), ("wider", lambda: lattice(160, 49), "big", False),
+    ("weights", lambda: lattice(300, 2, lambda a, b: 2**52 - 1), "big", True),
+    ("heavier", lambda: lattice(300, 2, lambda a, b: 2**52), "big", False)])
+def test_form_of_a_depth(hx, oracle, no_queue, name, make, width, solo):
+    """A refused depth is launched in both forms; the results are the oracle's either way."""
+    off, adj, ew, vw = make()
+    print(f"case solo form {name} n={len(off) - 1} m={len(adj)}", flush=True)
+    g = hx.Graph(off, adj, width=width, edge_weights=ew, vertex_weights=vw)
+    ol, oc, _ = oracle.initial_partition(oracle.Graph(off, adj, ew, vw), 2, 1.2, 3, with_coords=True)
+    hx.set_spectral_queue(False)
+    hx.profile_reset()
+    hx.profile_enable("spectral", True)
+    try:
+        labels, coords = g.initial_partition(2, 1.2, 3, "batched_fp64", with_coords=True)
+        launches = hx.profile_read("spectral")["launches"]
+    finally:
+        hx.profile_enable("spectral", False)
+    assert np.array_equal(labels, ol)
+    assert np.array_equal(coords.view(np.uint64), oc.view(np.uint64))
+    assert launches == (1 if solo else 2)
+
+
+def test_skewed_graphs(hx, oracle, no_queue):
+    """Coarse graphs with long rows, at whose depths some tasks suit the form and others do not."""
+    for scale, factor in ((9, 4), (11, 8), (12, 8)):
+        indptr, indices = hx.generate_rmat(scale, factor)
+        print(f"case solo rmat scale={scale} m={len(indices)}", flush=True)
+        g, og = hx.Graph(indptr, indices), oracle.Graph(indptr, indices.astype(np.int32))
+        hx.set_spectral_queue(False)
+        labels, coords = g.initial_partition(16, 1.2, 3, "batched_fp64", with_coords=True)
+        ol, oc, _ = oracle.initial_partition(og, 16, 1.2, 3, with_coords=True)
+        assert np.array_equal(labels, ol), scale
+        assert np.array_equal(coords.view(np.uint64), oc.view(np.uint64)), scale
