@@ -1213,11 +1213,6 @@ __global__ void contract_bounds_kernel(std::int64_t n, const std::int32_t* map, 
     }
 }
 
-__global__ void identity_list_kernel(std::int64_t n, std::int32_t* list) {
-    const std::int64_t v = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (v < n) list[v] = static_cast<std::int32_t>(v);
-}
-
 inline unsigned grid_for(std::int64_t threads) { return static_cast<unsigned>((threads + kBlock - 1) / kBlock); }
 
 // Sort the valid-proposal list `order` (p entries, vertex ids ascending) into
@@ -1619,7 +1614,6 @@ int gpart_sclp_two_hop(gpart_ctx* ctx, int64_t n, const int32_t* proposals, cons
         auto* cw = reinterpret_cast<unsigned long long*>(cluster_weights);
         const auto* gn = reinterpret_cast<const unsigned long long*>(gains);
         Scratch<std::int32_t> favorites(ctx, n), order(ctx, n), order_alt(ctx, n);
-        Scratch<std::int64_t> d_count(ctx, 1);
         hipLaunchKernelGGL(favorite_kernel, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, n, vertex_weights, cw,
                            clusters, proposals, favorites.get());
         GPART_LAUNCH_CHECK();

@@ -90,11 +90,6 @@ __device__ __forceinline__ unsigned lane_xor(unsigned v, int mask, int width) {
     return __shfl_xor(v, mask, width);
 }
 
-template <typename T>
-__device__ __forceinline__ T shfl(T v, int src, int width) {
-    return __shfl(v, src, width);
-}
-
 __device__ __forceinline__ unsigned long long shfl_u64(unsigned long long v, int src, int width) {
     const unsigned lo = __shfl(static_cast<unsigned>(v), src, width);
     const unsigned hi = __shfl(static_cast<unsigned>(v >> 32), src, width);
@@ -107,20 +102,10 @@ __device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v,
     return (static_cast<unsigned long long>(hi) << 32) | lo;
 }
 
-__device__ __forceinline__ unsigned long long shfl_down_u64(unsigned long long v, int delta, int width) {
-    const unsigned lo = __shfl_down(static_cast<unsigned>(v), delta, width);
-    const unsigned hi = __shfl_down(static_cast<unsigned>(v >> 32), delta, width);
-    return (static_cast<unsigned long long>(hi) << 32) | lo;
-}
-
 __device__ __forceinline__ unsigned long long shfl_up_u64(unsigned long long v, int delta, int width) {
     const unsigned lo = __shfl_up(static_cast<unsigned>(v), delta, width);
     const unsigned hi = __shfl_up(static_cast<unsigned>(v >> 32), delta, width);
     return (static_cast<unsigned long long>(hi) << 32) | lo;
-}
-
-__device__ __forceinline__ long long shfl_xor_i64(long long v, int mask, int width) {
-    return static_cast<long long>(shfl_xor_u64(static_cast<unsigned long long>(v), mask, width));
 }
 
 template <int G>
@@ -167,10 +152,6 @@ struct WidthTypes<1> {
     using O = std::int64_t;
     using W = std::uint64_t;
 };
-
-__device__ __forceinline__ void atomic_add_u64(unsigned long long* p, unsigned long long v) {
-    atomicAdd(p, v);
-}
 
 inline int ceil_div_int(std::int64_t a, std::int64_t b) { return static_cast<int>((a + b - 1) / b); }
 

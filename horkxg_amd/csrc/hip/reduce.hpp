@@ -15,7 +15,7 @@
 namespace gpart_hip {
 
 constexpr int kReduceThreads = 256;
-constexpr int kReduceMaxBlocks = 1024;
+constexpr int kReduceMaxBlocks = 2048;
 constexpr int kReduceLoads = 4;  // of a thread, under way together
 
 // Op: T identity(); T operator()(T, T).
@@ -178,7 +178,7 @@ void reduce_read(gpart_ctx* ctx, Load load, std::int64_t n, unsigned long long* 
                  const unsigned long long* known = nullptr, int known_count = 0) {
     constexpr std::int64_t kTile = kReduceThreads * kReduceLoads;
     const auto blocks =
-        static_cast<int>(std::min<std::int64_t>(std::max<std::int64_t>((n + kTile - 1) / kTile, 1), 2 * kReduceMaxBlocks));
+        static_cast<int>(std::min<std::int64_t>(std::max<std::int64_t>((n + kTile - 1) / kTile, 1), kReduceMaxBlocks));
     Scratch<unsigned long long> partials(ctx, blocks > 1 ? blocks * static_cast<std::int64_t>(sizeof...(Ops)) : 0);
     hipLaunchKernelGGL((reduce_publish_kernel<Load, Ops...>), dim3(blocks), dim3(kReduceThreads), 0, ctx->stream, load,
                        n, partials.get(), known, known_count, publication(ctx));

@@ -64,6 +64,8 @@ constexpr int kCacheBlocks = 4096;  // cap of the cache build launches (grid-str
 
 // ---------------------------------------------------------------- cut / weights
 
+constexpr int kCutBlocks = 1024;  // of a cut's pass over the edge tiles at most, a partial each
+
 // Directed cut weight over edge tiles (grid-stride over tiles); one partial per
 // workgroup in directed[blockIdx.x]. A lane loads its run's neighbours and
 // weights up front, then gathers their labels, so 16 loads are in flight per lane.
@@ -2072,12 +2074,12 @@ struct Ops {
     static void cut(gpart_ctx* ctx, const gpart_csr_view* g, const std::int32_t* labels, std::uint64_t* out) {
         const std::int64_t tiles = g->n > 0 && g->m > 0 ? tile_count(g->m) : 0;
         Scratch<std::int32_t> tile_row(ctx, tiles);
-        Scratch<unsigned long long> partials(ctx, std::min<std::int64_t>(tiles, kReduceMaxBlocks));
+        Scratch<unsigned long long> partials(ctx, std::min<std::int64_t>(tiles, kCutBlocks));
         cut_with(ctx, g, labels, tile_row.get(), partials.get(), out);
     }
 
     // The cut over caller-provided device scratch: tile_row (tile_count(m) entries) and
-    // partials (min(tiles, kReduceMaxBlocks) words, folded by one workgroup).
+    // partials (min(tiles, kCutBlocks) words, folded by one workgroup).
     static void cut_with(gpart_ctx* ctx, const gpart_csr_view* g, const std::int32_t* labels,
                          std::int32_t* tile_row, unsigned long long* partials, std::uint64_t* out) {
         unsigned long long directed = 0;
@@ -2088,11 +2090,11 @@ struct Ops {
             const std::int64_t tiles = tile_count(g->m);
             hipLaunchKernelGGL(tile_rows_kernel<O>, dim3(grid_for(g->n)), dim3(kBlock), 0, ctx->stream, g->n, off,
                                tile_row);
-            const int blocks = static_cast<int>(std::min<std::int64_t>(tiles, kReduceMaxBlocks));
+            const int blocks = static_cast<int>(std::min<std::int64_t>(tiles, kCutBlocks));
             hipLaunchKernelGGL((cut_kernel<O, W>), dim3(blocks), dim3(kTileLanes), 0, ctx->stream, g->n, g->m, tiles,
                                off, tile_row, g->neighbors, w, labels, partials);
             GPART_LAUNCH_CHECK();
-            static_assert(kReduceMaxBlocks <= kReduceThreads * kReduceLoads, "one workgroup: no scratch");
+            static_assert(kCutBlocks <= kReduceThreads * kReduceLoads, "one workgroup: no scratch");
             reduce_read<SumU64>(ctx, WidenLoad<unsigned long long>{partials}, blocks, &directed);
         }
         if (directed & 1ULL) throw Error(GPART_ERR_RUNTIME, "refinement cut is not symmetric");
@@ -2703,7 +2705,7 @@ namespace gpart_hip {
 namespace {
 constexpr std::int64_t kCutScratchTiles = std::int64_t{1} << 20;  // CSRs up to 2^20 * 4096 entries
 constexpr std::size_t kCutScratchPartialsOffset = 0;
-constexpr std::size_t kCutScratchTilesOffset = kCutScratchPartialsOffset + 8 * kReduceMaxBlocks;
+constexpr std::size_t kCutScratchTilesOffset = kCutScratchPartialsOffset + 8 * kCutBlocks;
 constexpr std::size_t kCutScratchBytes = kCutScratchTilesOffset + 4 * kCutScratchTiles;  // 4 MiB + 8 KiB
 constexpr int kCutScratchDevices = 64;
 
