@@ -3,7 +3,8 @@ when a round reads them, against the oracle.
 
 The graphs cover what the form distinguishes: rows of every degree class, hub rows of
 several chunks, vertex states of a byte and of half a byte (k <= 8 on levels above
-131,072 vertices), both widths, unit and larger entry weights, and the neighbours of a
+131,072 vertices) in LDS and of a byte in memory (above, from k = 9 on, or above 262,144
+vertices), both widths, unit and larger entry weights, and the neighbours of a
 mover that move too. Labels, cuts and round counts are whole numbers and must be equal.
 """
 from __future__ import annotations
@@ -43,7 +44,9 @@ GRAPHS = {
     "hubs12001": lambda hx: hub_graph(hx, 12_001, 24),
     "hubs20011": lambda hx: hub_graph(hx, 20_011, 20),
     "byte131072": lambda hx: random_graph(hx, 131_072, 26),
-    "nibble131073": lambda hx: random_graph(hx, 131_073, 26),
+    "random131073": lambda hx: random_graph(hx, 131_073, 26),
+    "memory262145": lambda hx: random_graph(hx, 262_145, 26),
+    "hubs140001": lambda hx: hub_graph(hx, 140_001, 16),
 }
 
 
@@ -51,7 +54,9 @@ GRAPHS = {
     ("rmat10", 2, "standard", False), ("rmat10", 32, "big", True), ("rmat13", 8, "standard", True),
     ("rmat13", 31, "standard", False), ("hubs12001", 8, "standard", True), ("hubs12001", 32, "big", False),
     ("hubs20011", 5, "big", True), ("hubs20011", 32, "standard", False), ("byte131072", 9, "standard", False),
-    ("nibble131073", 8, "standard", True), ("nibble131073", 7, "big", False),
+    ("random131073", 8, "standard", True), ("random131073", 7, "big", False),
+    ("random131073", 9, "standard", True), ("random131073", 32, "big", False), ("memory262145", 8, "big", True),
+    ("hubs140001", 9, "big", False), ("hubs140001", 32, "standard", True),
 ])
 def test_dense_refinement_matches_oracle(hx, oracle, name, k, width, weighted):
     if hx.device_count() < 1:
