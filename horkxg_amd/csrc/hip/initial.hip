@@ -224,9 +224,18 @@ __global__ void __launch_bounds__(256) depth_step_kernel(DepthTasks dt, const in
     T sum = 0;
     if (i < task.count) {
         const int v = ids[i];
-        for (std::int64_t e = static_cast<std::int64_t>(offsets[v]) + lane; e < offsets[v + 1]; e += 32) {
-            const int u = neighbors[e];
+        const auto end = static_cast<std::int64_t>(offsets[v + 1]);
+        std::int64_t e = static_cast<std::int64_t>(offsets[v]) + lane;
+        // the next neighbour under way while this one's label and value are: a long row is a
+        // chain of such loads, which normalising on read lengthens (a row of 4,096 entries
+        // took 12% longer than with the normalisation in a launch of its own)
+        int u = e < end ? neighbors[e] : -1;
+        while (u >= 0) {
+            const std::int64_t next = e + 32;
+            const int then = next < end ? neighbors[next] : -1;
             if (labels[u] == group) sum = VecTraits<T>::fmadd(static_cast<T>(weights[e]), normalized(x, u, norm), sum);
+            e = next;
+            u = then;
         }
     }
     const double sd = static_cast<double>(tree32(sum));
@@ -598,10 +607,14 @@ __global__ void __launch_bounds__(kSoloThreads) depth_solo_kernel(
 }
 
 // Single tasks of at most this size take their steps through the depth's fused launches:
-// one per step, of 5.5 us at 7,429 vertices, where step, moments and normalisation were
-// three, of 9.7 us. Each workgroup reads all partials, 3 bytes a vertex, so the form's
-// cost grows with the square of the size: the line is where a step's reads reach 25 MB
-// of L2 traffic.
+// one per step where step, moments and normalisation are three. Each workgroup reads all
+// partials, 3 bytes a vertex, so the form's cost grows with the square of the size.
+// Bisections of one task in us, three launches a step and one: 2D grids of 4,096 vertices
+// 810 and 561, 8,281 940 and 784, 12,100 989 and 887, 13,924 1018 and 986, 15,876 1033 and
+// 1061, 24,025 1235 and 1550; 3D meshes and random graphs of 16 and 64 entries a vertex
+// cross at the same sizes, 14,000 to 16,000. With rows of half the vertices, whose chain of
+// loads normalising on read lengthens, they are level from 6,000 (3305 and 3280) to 8,192
+// (4228 and 4395) and one launch is behind above: the line lies there.
 constexpr int kMaxFusedTask = 8192;
 
 template <typename O, typename W>
