@@ -605,7 +605,8 @@ __device__ __forceinline__ void block_add_i64(long long v, long long* block_sum,
 // part weights and the cut decrease -- was written by device-scope atomics, which
 // have left the workgroup when it arrives (s_waitcnt before its barrier) and are
 // performed past the XCDs' caches; it reads them with device-scope atomic loads. No
-// cache write-back is needed: the labels are read by later launches only.
+// cache write-back is needed: the labels are read by later launches, or after the entry
+// point's wait for this one's end (complete_outputs).
 template <typename O, typename W, typename C>
 __global__ void __launch_bounds__(kBlock) update_cache_kernel(
     RoundState* st, const std::int32_t* light, const std::int32_t* heavy, unsigned light_blocks,
